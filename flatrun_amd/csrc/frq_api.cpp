@@ -304,23 +304,89 @@ bool mb_takes(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_
 // Q6_K 4096 x 14336: 13.3 against 70; Q8_0 4096 x 4096: 5.4 against 20.7).
 constexpr int64_t kRowsBeforeGemm = 3;
 
+// Formats without a small-M kernel and gemm_f32 (Q5_K, Q1_0): one GEMV per row
+// below this many rows, the pair GEMM from there on (us, rows 2 / 4 / 8: Q5_K
+// 4096 x 4096 17.8 / 35.5 / 71 by rows, 18.6 from 4 by the pair GEMM; Q1_0
+// 2048 x 2048 6.5 / 12.9 / 28 and 15).
+constexpr int64_t kPairRowsMin = 4;
+
+// Where gemm_f32 is the faster one of the two: its two launches against the
+// pair GEMM's three decide on small matrices. Measured (us, gemm_f32 / pair):
+// Q4_K 4096 x 4096 rows 12 / 64 / 128 / 192: 17.8 / 25.5 / 33.7 / 45.9 and
+// 18.5 / 28.7 / 34.5 / 39.4; 18944 x 3584 rows 12 / 64: 51 / 79 and 30 / 43;
+// Q6_K 1024 x 4096 rows 40 / 128 / 512: 16.7 / 20.6 / 30.8 and 20 / 24 / 36;
+// 4096 x 14336 rows 12 / 64 / 512: 64 / 69 / 265 and 39 / 46 / 192.
+// Q8_0 always (4096 x 4096 rows 16 / 512: 18 / 70 and 29 / 79).
+bool f32_before_pair(int qtype, int64_t batch, int64_t n, int64_t k) {
+    if (qtype == FRQ_Q5_K || qtype == FRQ_Q1_0) return false;
+    if (qtype == FRQ_Q8_0) return true;
+    return (double)n * (double)k < 2.4e7 && (batch <= 64 || qtype == FRQ_Q6_K);
+}
+
+// Scratch a pair launch may hold per stream; shapes beyond it take the kernels
+// that need less (gemm_f32, one GEMV per row).
+constexpr size_t kPairScratchMax = (size_t)1 << 30;
+
+// The pair GEMM's plan for up to kPairRows rows of x, false where it does not
+// take the shape, the alignment or the scratch.
+bool pair_plan(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_t n, int64_t k, size_t cap,
+               frq::PairPlan* p) {
+    const uintptr_t wa = reinterpret_cast<uintptr_t>(w);
+    if ((reinterpret_cast<uintptr_t>(x) & 15) || (qtype == FRQ_Q4_K || qtype == FRQ_Q5_K ? (wa & 15) : (wa & 1)))
+        return false;
+    return frq::plan_gemm_pair(qtype, batch < frq::kPairRows ? batch : frq::kPairRows, n, k, cap, p);
+}
+
 // Which kernels a batch of x rows takes: the small-M kernel for two to
 // mr_rows_before_gemm rows, else one GEMV per row up to kRowsBeforeGemm
-// rows, else the GEMM where batched_gemm allows, else one GEMV per row.
-enum class BatchRoute { SmallM, Gemm, Rows };
-BatchRoute batch_route(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_t n, int64_t k) {
+// rows, else a GEMM where there is one (the pair GEMM, or gemm_f32 where its
+// scratch does not fit), else one GEMV per row.
+enum class BatchRoute { SmallM, Pair, Gemm, Rows };
+BatchRoute batch_route(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_t n, int64_t k,
+                       size_t pair_cap) {
     if (mb_takes(qtype, w, x, batch, n, k) ||
         (batch >= 2 && batch <= mr_rows_before_gemm(qtype) && frq::gemv_mr_ok(qtype, w, x, k)))
         return BatchRoute::SmallM;
+    const bool own = qtype == FRQ_Q5_K || qtype == FRQ_Q1_0;
+    frq::PairPlan p;
+    if (batch >= (own ? kPairRowsMin : kRowsBeforeGemm + 1) &&
+        !(f32_before_pair(qtype, batch, n, k) && batched_gemm(qtype, w, x, batch, n, k)) && pair_plan(qtype, w, x, batch, n, k, pair_cap, &p))
+        return BatchRoute::Pair;
     if (batch > kRowsBeforeGemm && batched_gemm(qtype, w, x, batch, n, k)) return BatchRoute::Gemm;
     return BatchRoute::Rows;
+}
+size_t pair_cap(const frq::FixedScratch* fixed) { return fixed ? fixed->part_bytes : kPairScratchMax; }
+
+// Scratch for a pair launch of `bytes` on stream `s`; the caller holds g_sk_mu.
+// Null where it cannot be had (a stream under capture that has less, or no
+// memory): the call then takes the kernels that need less.
+uint8_t* pair_scratch_locked(hipStream_t s, size_t bytes) {
+    float* part = nullptr;
+    uint32_t* cnt = nullptr;
+    if (sk_scratch_locked(s, bytes, 0, &part, &cnt) == FRQ_OK) return reinterpret_cast<uint8_t*>(part);
+    (void)hipGetLastError();
+    g_err.clear();
+    return nullptr;
+}
+
+// The pair GEMM over all rows, kPairRows at a time. x_ready: the scratch holds
+// the pairs of these rows (one chunk) already.
+int pair_rows(int qtype, const uint8_t* w, const float* x, float* y, int64_t n, int64_t k, int64_t batch, int64_t ldy,
+              hipStream_t s, uint8_t* scratch, size_t cap, bool x_ready) {
+    for (int64_t b = 0; b < batch; b += frq::kPairRows) {
+        frq::PairPlan p;
+        const int64_t m = batch - b < frq::kPairRows ? batch - b : frq::kPairRows;
+        if (!frq::plan_gemm_pair(qtype, m, n, k, cap, &p)) return fail(FRQ_ERR_UNSUPPORTED, "gemm: no plan");
+        FRQ_HIP(frq::launch_gemm_pair(qtype, w, x + b * k, y + b * ldy, ldy, p, s, scratch, x_ready));
+    }
+    return FRQ_OK;
 }
 
 // y[b * ldy + i] = (W x_b)[i] for b < batch, by batch_route. Scratch as
 // gemv_device (the small-M kernel uses none).
 int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t n, int64_t k, int64_t batch,
                  int64_t ldy, hipStream_t s, const frq::FixedScratch* fixed = nullptr) {
-    const BatchRoute route = batch_route(qtype, w, x, batch, n, k);
+    BatchRoute route = batch_route(qtype, w, x, batch, n, k, pair_cap(fixed));
     if (route == BatchRoute::SmallM && mb_takes(qtype, w, x, batch, n, k)) {
         frq::MbPlan p;
         frq::plan_gemv_mb(n, k, (int)batch, &p);
@@ -334,6 +400,17 @@ int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t 
             b += m;
         }
         return FRQ_OK;
+    }
+    if (route == BatchRoute::Pair) {
+        if (fixed)
+            return pair_rows(qtype, w, x, y, n, k, batch, ldy, s, reinterpret_cast<uint8_t*>(fixed->part),
+                             fixed->part_bytes, false);
+        frq::PairPlan p;
+        pair_plan(qtype, w, x, batch, n, k, kPairScratchMax, &p);
+        std::lock_guard<std::mutex> lk(g_sk_mu);
+        if (uint8_t* scratch = pair_scratch_locked(s, p.bytes))
+            return pair_rows(qtype, w, x, y, n, k, batch, ldy, s, scratch, p.bytes, false);
+        route = batched_gemm(qtype, w, x, batch, n, k) ? BatchRoute::Gemm : BatchRoute::Rows;
     }
     if (route == BatchRoute::Gemm) {
         if (fixed) {   // as many K-splits as the fixed partial region holds
@@ -350,6 +427,42 @@ int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t 
     }
     for (int64_t b = 0; b < batch; ++b)
         if (int rc = gemv_device(qtype, w, x + b * k, y + b * ldy, n, k, s, fixed)) return rc;
+    return FRQ_OK;
+}
+
+// gemv_batched for matrices that share x: those that take the pair GEMM run
+// first, one after the other under one lock, so that x is split once per order
+// of its elements. Same bits as separate calls.
+int gemv_batched_group(int count, const int* qtypes, const uint8_t* const* w, const float* x, float* const* y,
+                       const int64_t* n, int64_t k, int64_t batch, const int64_t* ldy, hipStream_t s) {
+    bool done[frq::kGemvGroupMax] = {};
+    frq::PairPlan p[frq::kGemvGroupMax];
+    size_t need = 0;
+    for (int i = 0; i < count; ++i) {
+        done[i] = n[i] == 0;
+        if (!done[i] && batch <= frq::kPairRows &&
+            batch_route(qtypes[i], w[i], x, batch, n[i], k, kPairScratchMax) == BatchRoute::Pair &&
+            pair_plan(qtypes[i], w[i], x, batch, n[i], k, kPairScratchMax, &p[i]) && p[i].bytes > need)
+            need = p[i].bytes;
+    }
+    if (need) {
+        std::lock_guard<std::mutex> lk(g_sk_mu);
+        if (uint8_t* scratch = pair_scratch_locked(s, need))
+            for (int i = 0; i < count; ++i) {
+                if (done[i] || !p[i].bytes) continue;
+                bool ready = false;
+                for (int j = i; j < count; ++j)          // every matrix of this element order
+                    if (!done[j] && p[j].bytes && p[j].layout == p[i].layout && p[j].bm == p[i].bm) {
+                        if (int rc = pair_rows(qtypes[j], w[j], x, y[j], n[j], k, batch, ldy[j], s, scratch, p[j].bytes,
+                                               ready))
+                            return rc;
+                        ready = done[j] = true;
+                    }
+            }
+    }
+    for (int i = 0; i < count; ++i)
+        if (!done[i])
+            if (int rc = gemv_batched(qtypes[i], w[i], x, y[i], n[i], k, batch, ldy[i], s)) return rc;
     return FRQ_OK;
 }
 
@@ -599,7 +712,8 @@ static int dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, fl
         size_t sb = 0, pb = 0;
         // the small-M kernel needs no scratch and the batched GEMM splits K
         // within what is there; rows that run one GEMV each need theirs
-        if (batch_route(qtype, wp, x, batch, n, k) == BatchRoute::Rows) gemv_scratch_need(qtype, wp, x, n, k, &sb, &pb);
+        if (batch_route(qtype, wp, x, batch, n, k, pair_cap(fixed)) == BatchRoute::Rows)
+            gemv_scratch_need(qtype, wp, x, n, k, &sb, &pb);
         if (sb > fixed->slot_bytes || pb > fixed->part_bytes)
             return fail(FRQ_ERR_UNSUPPORTED,
                         "%s gemv n=%lld k=%lld needs %zu slot + %zu partial bytes of scratch; the fixed scratch "
@@ -638,11 +752,9 @@ int frq_dev_gemv_group(int count, const int* qtypes, const void* const* w, const
     for (int i = 0; i < count; ++i) wp[i] = static_cast<const uint8_t*>(w[i]);
     const bool fused = k > 0 && frq::gemv_group_fusable(count, qtypes, wp, k);
     if (k > 0 && batch >= 2) {   // prefill-shaped: each matrix once, its rows of x together
-        for (int i = 0; i < count; ++i)
-            if (n[i])
-                if (int rc = gemv_batched(qtypes[i], wp[i], x, y[i], n[i], k, batch, y_stride ? y_stride : n[i], s))
-                    return rc;
-        return FRQ_OK;
+        int64_t ldy[frq::kGemvGroupMax];
+        for (int i = 0; i < count; ++i) ldy[i] = y_stride ? y_stride : n[i];
+        return gemv_batched_group(count, qtypes, wp, x, y, n, k, batch, ldy, s);
     }
     for (int64_t b = 0; b < batch; ++b) {
         for (int i = 0; i < count; ++i) yb[i] = y[i] + b * (y_stride ? y_stride : n[i]);

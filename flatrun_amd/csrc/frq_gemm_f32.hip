@@ -1,4 +1,5 @@
-// Batched matvec with the fp32 contract on the gfx950 matrix cores:
+// Batched matvec with the fp32 contract on the gfx950 matrix cores, for Q8_0, for
+// small matrices and where the pair GEMM's scratch (frq_gemm_pair.hip) cannot be had:
 //   Y[M, N] (fp32) = X[M, K] (fp32) . W[N, K]^T, W = raw Q4_K, Q6_K or Q8_0 blocks.
 //
 // The reference's batched entry points (matmul_<q>_batched, _C.cpp:154-283)
@@ -46,6 +47,7 @@
 // D register r of lane l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "frq_common.h"
 #include "frq_kernels.h"
+#include "frq_weight_at.h"
 
 #include <atomic>
 
@@ -209,31 +211,6 @@ struct CFmt<kTypeQ6K> {
         }
     }
 };
-
-// Element j of a W row as the dequantizer gives it (fp32, gguf.py op order):
-// Q4_K fl(d sc q) - fl(dmin m), Q6_K d sc (q - 32), Q8_0 d q.
-template <int QT>
-__device__ float weight_at(const uint8_t* __restrict__ wrow, int j) {
-    if constexpr (QT == kTypeQ4K) {
-        const uint8_t* bp = wrow + (int64_t)(j >> 8) * kQ4KBytes;
-        const int e = j & 255, sb = e >> 5, l = e & 31;
-        const uint4 h = *reinterpret_cast<const uint4*>(bp);
-        uint32_t sc, mn;
-        k4_scale_min(h.y, h.z, h.w, sb, sc, mn);
-        const uint32_t q = (bp[16 + 32 * (sb >> 1) + l] >> (4 * (sb & 1))) & 15u;
-        return f16_bits_to_f32(h.x) * (float)sc * (float)q - f16_bits_to_f32(h.x >> 16) * (float)mn;
-    } else if constexpr (QT == kTypeQ6K) {
-        const uint8_t* bp = wrow + (int64_t)(j >> 8) * kQ6KBytes;
-        const int e = j & 255, hh = e >> 7, ks = (e >> 5) & 3, l = e & 31;
-        const uint32_t ql = (bp[64 * hh + 32 * (ks & 1) + l] >> (ks >= 2 ? 4 : 0)) & 15u;
-        const uint32_t qh = (bp[128 + 32 * hh + l] >> (2 * ks)) & 3u;
-        const float sc = (float)(int)(int8_t)bp[192 + 8 * hh + (l >> 4) + 2 * ks];
-        return f16_bits_to_f32(ld_u16(bp + 208)) * sc * (float)((int)(ql | (qh << 4)) - 32);
-    } else {
-        const uint8_t* bp = wrow + (int64_t)(j >> 5) * kQ80Bytes;
-        return f16_bits_to_f32(ld_u16(bp)) * (float)(int)(int8_t)bp[2 + (j & 31)];
-    }
-}
 
 // sum_j w[j] x[j] in fp64 (products of fp32 values exact), rounded to fp32 once.
 template <int QT>

@@ -1,0 +1,1056 @@
+// Batched matvec with the fp32 contract, x as pairs of fp16 values:
+//   Y[M, N] (fp32) = X[M, K] (fp32) . W[N, K]^T, W = raw Q4_K, Q5_K, Q6_K or
+//   Q1_0 blocks.
+//
+// The reference's batched entry points (matmul_<q>_batched, _C.cpp:154-283)
+// run one fp32 matvec per row of X. Here the products run on
+// v_mfma_f32_32x32x16_f16, two per product:
+//   * x enters as hi + lo, hi = f16(x 2^e), lo = f16(x 2^e - hi), with 2^e a
+//     power of two per row that puts the row's largest |x| in [2^14, 2^15).
+//     The pair carries every element down to 2^-16 of the row's largest to
+//     within 2^-23 of itself, smaller ones to within 2^-40 of the largest.
+//   * W enters as integers that f16 holds exactly (times 2^-14): Q4_K / Q5_K
+//     sc q - R with R the integer nearest dmin m / d, Q6_K q - 32, Q1_0 +-1.
+//     A nibble masked in place is the f16 subnormal
+//     q 2^-24 (or 16 q 2^-24), so one v_pk_fma_f16 turns two of them into
+//     codes, scale and centre included.
+//   * the matrix cores sum 64 elements (Q6_K 16, one sub-block) in fp32, then
+//     acc += scale * sum in fp32 (the scale of a Q4_K / Q5_K block alone, since
+//     sc is in the code). With up to 64 rows a wave, acc is added to the result's
+//     accumulator every 256 elements, so that the sums round less often at
+//     full size. Q4_K / Q5_K add -(dmin m - d R) sum(x) per 32-element sub-block
+//     on the matrix cores as well: three bf16 pieces of each factor, the six
+//     products down to 2^-24 of their product.
+//   With R the nearest integer, |d (sc q - R)| + |dmin m - d R| <= 3 |w|, so a
+//   large x on a weight that is exactly zero leaves the others their bits.
+//
+// split_kernel writes the pairs once per call in the order the matrix cores
+// take them, with the scale per row. It also measures, per row, the error
+// of the split beyond 2^-23 of each element, against 2^-24 of sum |x| with
+// elements capped at 2^-10 of the largest: a row beyond that (an outlier some
+// 2^17 above the rest), one whose largest |x| is outside [2^-100, 2^100], and
+// one with an inf or NaN are computed weight by weight in fp64 instead
+// (finish_kernel), as gemm_f32's are.
+//
+// Tiling: BM x BN of Y per workgroup; a wave owns 32 MT x 32 NT. W goes from
+// memory to registers to the matrix cores (lane = one row of W; both halves
+// of the wave read consecutive 16-byte parts), decoded once per workgroup
+// where WM = 1; x goes through LDS, 32 KB per barrier, double-buffered, as
+// every wave reads all of it. K is split over S workgroups where the tiles
+// do not fill the GPU; finish_kernel adds the partial planes in split order.
+// Measured (kernel us, gemm_f32 / here): 333 rows, Q4_K 18944 x 3584 261 / 125
+// (837 TFLOP/s of matrix work on rows padded to 384, about 1300 in a large
+// library product), Q6_K 3584 x 18944 351 / 173 (its scale per 16 elements:
+// eight times the vector work); whole calls, 97 rows of Q5_K 14336 x 4096 1391
+// (a GEMV per row) / 53, 16 rows of Q4_K 4096 x 14336 35.5 / 30.3. 128-row tiles
+// are bound by the matrix cores' issue and power, few rows by the chain of
+// decode and products per wave (2.9 us per 256 of k) and the three launches.
+// MFMA operand layouts (32x32x16, 8 values per lane): A lane l holds row l%32,
+// k = 8*(l/32) .. +7; B lane l column l%32, same k; D register r of lane l is
+// row 8*(r/4) + 4*(l/32) + r%4, column l%32. The order of k is free as long as
+// A and B agree: it is chosen so that masked fields of a dword land in place.
+#include "frq_common.h"
+#include "frq_kernels.h"
+#include "frq_weight_at.h"
+
+namespace frq {
+namespace {
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+// dword-aligned parts of rows, and the 2-byte aligned dwords of Q1_0 blocks
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x3 u32x3_a4 __attribute__((aligned(4)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+
+constexpr int kUnit = 256;               // K per unit (4 stages of 64)
+constexpr int kStageBytes = 8192;        // 32 rows x 64 k x 2 pieces x 2 bytes
+
+template <int QT>
+constexpr bool kK4 = QT == kTypeQ4K || QT == kTypeQ5K;
+
+__device__ __forceinline__ f16x2 as_f16x2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ uint32_t as_u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ uint32_t fma2(uint32_t a, f16x2 b, f16x2 c) {
+    return as_u32(__builtin_elementwise_fma(as_f16x2(a), b, c));
+}
+__device__ __forceinline__ f16x2 pair_of(float v) {   // v exact in f16
+    return __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(v, v));
+}
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
+template <int S>
+__device__ __forceinline__ uint32_t shl(uint32_t v) {   // left by S, right by -S
+    if constexpr (S >= 0) return v << S;
+    else return v >> -S;
+}
+
+// A pointer in scalar registers, from here on opaque to the optimiser: loads
+// through it take the lane's part of the address as a 32-bit offset, instead of
+// a 64-bit address per lane and load that is advanced every unit.
+typedef const __attribute__((address_space(1))) uint8_t* gptr;
+__device__ __forceinline__ gptr scalar_base(const uint8_t* p) {
+    gptr g = (gptr)p;
+    asm("" : "+s"(g));
+    return g;
+}
+template <typename V>
+__device__ __forceinline__ auto ld(gptr base, uint32_t off) {
+    asm("" : "+v"(off));     // its extension to 64 bits stays beside the load, which folds it
+    return *(const __attribute__((address_space(1))) V*)(base + off);
+}
+
+// 16 bytes per lane from memory straight to LDS, lane l's to dst + 16 l.
+__device__ __forceinline__ void lds_copy(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off, uint8_t* dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, (int)lane_off, (int)off,
+                                             0, 0);
+}
+
+// The 2-byte aligned fields of Q6_K blocks are read by dword-aligned loads and
+// shifted when they are used: wide loads off dword boundaries run at a fraction
+// of the rate (4096 x 14336, 16 rows: 54 us against 39). A window starts at
+// the dword that holds the field's first byte and ends at the one that holds
+// its last, or inside the block.
+struct Window {
+    gptr base;
+    uint32_t off;           // of the dword that holds the byte at base + off
+    __device__ __forceinline__ Window(gptr p, uint32_t o) {
+        const uint64_t a = (uint64_t)p;
+        base = (gptr)(a & ~(uint64_t)3);
+        off = (o + ((uint32_t)a & 3u)) & ~3u;
+    }
+};
+__device__ __forceinline__ uint32_t misaligned(gptr p, uint32_t o) {   // 16 where p + o is 2 past a dword, else 0
+    return (((uint32_t)(uint64_t)p + o) & 2u) * 8u;
+}
+__device__ __forceinline__ uint32_t shifted(uint32_t lo, uint32_t hi, uint32_t sh) {
+    return __builtin_amdgcn_alignbit(hi, lo, sh);
+}
+
+// One row's fields of one 256-element unit, as the lane (half h of its row)
+// needs them: Head<QT> those used all through the unit, Body<QT> the codes,
+// load<T> those of stage T (`unit` = the unit in the first of the
+// workgroup's rows, `row` the lane's row from there, `left` = blocks of Q8_0 /
+// Q1_0 from the unit on). frag<T, I>: the eight codes of slice
+// I of stage T; scale<T, I>: what the sum of the group that ends with that
+// slice is multiplied by. Stage / slice / element orders are those of
+// Order<QT> below.
+template <int QT>
+struct Head;
+template <int QT>
+struct Body;
+
+// Q4_K: stage t = qs bytes 32t .. 32t+31 (sub-blocks 2t low, 2t+1 high
+// nibbles; gguf.py:209-219), half h the 16 bytes 32t + 16h; slice i = dword i.
+template <>
+struct Head<kTypeQ4K> {
+    u32x4 hd;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int) { hd = ld<u32x4>(unit, row); }
+};
+template <>
+struct Body<kTypeQ4K> {
+    static constexpr int kLoads = 1, kHeadLoads = 1;   // vector loads of every load<T> / of the head, at least
+    u32x4 q[4];
+    template <int T>
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int h, int) {
+        q[T] = ld<u32x4>(unit + 16 + 32 * T, row + 16 * h);
+    }
+    template <int T, int I>
+    __device__ __forceinline__ u32x4 fields(const Head<kTypeQ4K>&) const {   // (low b0 b2, high b0 b2, low b1 b3, high b1 b3)
+        const uint32_t v = q[T][I], v8 = v >> 8;
+        return u32x4{v & 0x000F000Fu, v & 0x00F000F0u, v8 & 0x000F000Fu, v8 & 0x00F000F0u};
+    }
+};
+
+// Q5_K: as Q4_K, bit 2t (2t + 1) of qh byte l is the fifth bit of element l of
+// sub-block 2t (2t + 1) (gguf.py:258-275).
+template <>
+struct Head<kTypeQ5K> {
+    u32x4 hd, qh;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int h) {
+        hd = ld<u32x4>(unit, row);
+        qh = ld<u32x4>(unit + 16, row + 16 * h);
+    }
+};
+template <>
+struct Body<kTypeQ5K> {
+    static constexpr int kLoads = 1, kHeadLoads = 2;   // vector loads of every load<T> / of the head, at least
+    u32x4 q[4];
+    template <int T>
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int h, int) {
+        q[T] = ld<u32x4>(unit + 48 + 32 * T, row + 16 * h);
+    }
+    template <int T, int I>
+    __device__ __forceinline__ u32x4 fields(const Head<kTypeQ5K>& hh) const {
+        const uint32_t v = q[T][I], v8 = v >> 8, b = hh.qh[I];
+        return u32x4{(v & 0x000F000Fu) | (shl<4 - 2 * T>(b) & 0x00100010u),
+                     (v & 0x00F000F0u) | (shl<7 - 2 * T>(b) & 0x01000100u),
+                     (v8 & 0x000F000Fu) | (shl<-4 - 2 * T>(b) & 0x00100010u),
+                     (v8 & 0x00F000F0u) | (shl<-1 - 2 * T>(b) & 0x01000100u)};
+    }
+};
+
+// Q6_K: stage (h', p) = 2h' + p: ql bytes 64h' + 32p + l; slices (nibble c,
+// l / 16 = u) = 2c + u are the 16-element groups of ks = p + 2c, half h their
+// bytes 8h .. 8h+7 (gguf.py:401-419).
+template <>
+struct Head<kTypeQ6K> {
+    uint32_t d, sh;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int) {
+        d = ld<uint16_t>(unit + 208, row);
+        sh = misaligned(unit, row);
+    }
+};
+template <>
+struct Body<kTypeQ6K> {
+    static constexpr int kLoads = 2, kHeadLoads = 1;   // vector loads of every load<T> / of the head, at least
+    u32x3 ql[4][2], qh[2][2], sc[2];                    // windows of eight bytes
+    template <int T>
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int h, int) {
+        const Window f(unit, row + 8 * h), f0(unit, row);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            ql[T][g] = ld<u32x3_a4>(f.base + 32 * T + 16 * g, f.off);
+            if constexpr (T % 2 == 0) qh[T / 2][g] = ld<u32x3_a4>(f.base + 128 + 16 * T + 16 * g, f.off);
+        }
+        if constexpr (T % 2 == 0) sc[T / 2] = ld<u32x3_a4>(f0.base + 192 + 4 * T, f0.off);
+    }
+    template <int T, int I>
+    __device__ __forceinline__ u32x4 frag(const Head<kTypeQ6K>& hh) const {
+        constexpr int p = T & 1, c = I >> 1, g = I & 1;
+        u32x4 r;
+        const f16x2 m = c ? pair_of(64.0f) : pair_of(1024.0f), o = pair_of(-32.0f / 16384.0f);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t v = shifted(ql[T][g][e], ql[T][g][e + 1], hh.sh), v8 = v >> 8;
+            const uint32_t b = shifted(qh[T >> 1][g][e], qh[T >> 1][g][e + 1], hh.sh);
+            const uint32_t b0 = shl<4 - 2 * p>(b), b1 = shl<-4 - 2 * p>(b);
+            const uint32_t f0 = c ? (v & 0x00F000F0u) | (b0 & 0x03000300u) : (v & 0x000F000Fu) | (b0 & 0x00300030u);
+            const uint32_t f1 = c ? (v8 & 0x00F000F0u) | (b1 & 0x03000300u) : (v8 & 0x000F000Fu) | (b1 & 0x00300030u);
+            r[2 * e] = fma2(f0, m, o);
+            r[2 * e + 1] = fma2(f1, m, o);
+        }
+        return r;
+    }
+    // d * sc[8h' + u + 2 (p + 2c)]
+    template <int T, int I>
+    __device__ __forceinline__ float scale(const Head<kTypeQ6K>& hh) const {
+        constexpr int j = (I & 1) + 2 * ((T & 1) + 2 * (I >> 1)), e = j >> 2;
+        const uint32_t v = shifted(sc[T >> 1][e], sc[T >> 1][e + 1], hh.sh);
+        return f16_bits_to_f32(hh.d) * 16384.0f * (float)(int)(int8_t)(v >> (8 * (j & 3)));
+    }
+};
+
+// Q1_0: stage t = bytes 8 (t & 1) .. of block t / 2, half h a dword of them;
+// slice i register r = the signs of bits 4i + r and 16 + 4i + r (1 = +).
+// The codes are negated (bit 1 -> -1), the scale with them.
+template <>
+struct Head<kTypeQ10> {
+    __device__ __forceinline__ void load(gptr, uint32_t, int) {}
+};
+template <>
+struct Body<kTypeQ10> {
+    static constexpr int kLoads = 1, kHeadLoads = 0;   // vector loads of every load<T> / of the head, at least
+    uint32_t q[4];
+    uint32_t d[2];                       // of the two blocks
+    template <int T>
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int h, int left) {
+        const gptr bp = unit + (T / 2 < left ? T / 2 : left - 1) * kQ10Bytes;
+        if constexpr (T % 2 == 0) {
+            const uint32_t dv = ld<uint16_t>(bp, row);
+            d[T / 2] = T / 2 < left ? dv : 0u;
+        }
+        q[T] = ld<u32_a2>(bp + 2 + 8 * (T % 2), row + 4 * h);
+    }
+    template <int T, int I>
+    __device__ __forceinline__ u32x4 frag(const Head<kTypeQ10>&) const {
+        u32x4 r;
+        static_for<0, 4>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            r[j] = ((q[T] << (15 - 4 * I - j)) & 0x80008000u) | 0x3C003C00u;
+        });
+        return r;
+    }
+    template <int T, int I>
+    __device__ __forceinline__ float scale(const Head<kTypeQ10>&) const {
+        return -f16_bits_to_f32(d[T >> 1]);
+    }
+};
+
+// Where the eight x of (stage st, slice i, half h) are in the row: two runs
+// of four from a and b, and the order they take in the fragment.
+template <int QT>
+struct Order {
+    __device__ __forceinline__ static void runs(int st, int i, int h, int& a, int& b) {
+        if constexpr (kK4<QT>) {
+            a = 64 * st + 16 * h + 4 * i;
+            b = a + 32;
+        } else if constexpr (QT == kTypeQ6K) {
+            a = 128 * (st >> 1) + 32 * ((st & 1) + (i & 2)) + 16 * (i & 1) + 8 * h;
+            b = a + 4;
+        } else {
+            a = 64 * st + 32 * h + 4 * i;
+            b = a + 16;
+        }
+    }
+    __device__ __forceinline__ static void order(const f32x4 a, const f32x4 b, float (&v)[8]) {
+        if constexpr (kK4<QT>) {
+            v[0] = a[0], v[1] = a[2], v[2] = b[0], v[3] = b[2], v[4] = a[1], v[5] = a[3], v[6] = b[1], v[7] = b[3];
+        } else if constexpr (QT == kTypeQ10) {
+            v[0] = a[0], v[1] = b[0], v[2] = a[1], v[3] = b[1], v[4] = a[2], v[5] = b[2], v[6] = a[3], v[7] = b[3];
+        } else {
+            v[0] = a[0], v[1] = a[2], v[2] = a[1], v[3] = a[3], v[4] = b[0], v[5] = b[2], v[6] = b[1], v[7] = b[3];
+        }
+    }
+};
+
+// Workgroup-wide sum / max over the TPR threads of a row (LDS, fixed order).
+template <int TPR, typename T, typename Op>
+__device__ __forceinline__ T row_reduce(T v, T* lds, int tr, Op op) {
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) v = op(v, __shfl_xor(v, s, 64));
+    if constexpr (TPR == 64) return v;
+    __syncthreads();
+    if ((tr & 63) == 0) lds[tr >> 6] = v;
+    __syncthreads();
+    T t = lds[0];
+#pragma unroll
+    for (int i = 1; i < TPR / 64; ++i) t = op(t, lds[i]);
+    return t;
+}
+
+// The pairs of every row of x, the sub-block sums' pieces (Q4_K / Q5_K) and
+// the factor that undoes the row's scale (0 = row computed weight by weight).
+// RW rows per workgroup, TPR threads each, NC pieces of eight elements per
+// thread: x is read once, into registers (NC = 0: rows too long for that are
+// read twice). Eight neighbouring rows, whose 16-byte parts share lines of
+// the output, go to workgroups of one XCD, where their writes meet in L2.
+template <int QT, int RW, int TPR, int NC>
+__global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict__ x, int M, int K, int units,
+                                                         uint8_t* __restrict__ xf, uint8_t* __restrict__ xsum,
+                                                         float* __restrict__ inv) {
+    __shared__ float red[RW][TPR / 64];
+    static_assert(RW <= 8, "rows of a workgroup share an XCD's eight");
+    constexpr int WR = 8 / RW;                         // workgroups of eight rows
+    const int rr = threadIdx.x / TPR, tr = threadIdx.x % TPR, slot = (int)blockIdx.x >> 3;
+    const int m = 64 * (slot / WR) + 8 * ((int)blockIdx.x & 7) + RW * (slot % WR) + rr;
+    if (m - rr >= M) return;                           // none of this workgroup's rows
+    const bool live = m < M;
+    const float* xr = x + (int64_t)(live ? m : M - 1) * K;
+    const int chunks = units * 32;                     // (stage, slice, half) triples
+    auto load = [&](int c, f32x4& a, f32x4& b) __attribute__((always_inline)) {
+        int ra, rb;
+        Order<QT>::runs(c >> 3, (c >> 1) & 3, c & 1, ra, rb);
+        const bool in = c < chunks;
+        a = in && ra < K ? *reinterpret_cast<const f32x4*>(xr + ra) : f32x4{};
+        b = in && rb < K ? *reinterpret_cast<const f32x4*>(xr + rb) : f32x4{};
+    };
+    auto largest = [](uint32_t big, const f32x4 v) __attribute__((always_inline)) {   // |x| as bits, NaN above inf
+#pragma unroll
+        for (int e = 0; e < 4; ++e) big = max(big, __float_as_uint(v[e]) & 0x7FFFFFFFu);
+        return big;
+    };
+    f32x4 xa[NC ? NC : 1], xb[NC ? NC : 1];
+    uint32_t big = 0;
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) load(tr + j * TPR, xa[j], xb[j]);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) big = largest(largest(big, xa[j]), xb[j]);
+    } else {
+        for (int c = tr; c < K / 4; c += TPR) big = largest(big, *reinterpret_cast<const f32x4*>(xr + 4 * c));
+    }
+    big = row_reduce<TPR>(big, reinterpret_cast<uint32_t*>(red[rr]), tr,
+                          [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+    // exponent fields 27 .. 227: 2^-100 <= max |x| < 2^101
+    const int ef = (int)(big >> 23);
+    bool ok = big == 0 || (ef >= 27 && ef <= 227);
+    const int e = big == 0 || !ok ? 0 : 127 + 14 - ef;   // max |x| 2^e in [2^14, 2^15)
+    const float scale = ok ? ldexpf(1.0f, e) : 0.0f;
+    const float cap = 16.0f;                             // 2^-10 of the largest
+    float err = 0.0f, body = 0.0f;
+    const int64_t mt = m >> 5;
+    const int nst = units * 4;
+    auto split = [&](int c, f32x4 a, f32x4 b) __attribute__((always_inline)) {
+        const int st = c >> 3, i = (c >> 1) & 3, h = c & 1;
+        if (!ok) a = b = f32x4{};                        // inf * 0 would be NaN
+        a *= scale;
+        b *= scale;
+        float v[8];
+        Order<QT>::order(a, b, v);
+        u32x4 hi, lo;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const f16x2 hv = {(_Float16)v[2 * p], (_Float16)v[2 * p + 1]};
+            const float r0 = v[2 * p] - (float)hv[0], r1 = v[2 * p + 1] - (float)hv[1];
+            const f16x2 lv = {(_Float16)r0, (_Float16)r1};
+            hi[p] = as_u32(hv);
+            lo[p] = as_u32(lv);
+            // error beyond 2^-23 of the element (only elements below 2^-16 of the largest have any)
+            err += fmaxf(fabsf(r0 - (float)lv[0]) - 0x1p-23f * fabsf(v[2 * p]), 0.0f) +
+                   fmaxf(fabsf(r1 - (float)lv[1]) - 0x1p-23f * fabsf(v[2 * p + 1]), 0.0f);
+            body += fminf(fabsf(v[2 * p]), cap) + fminf(fabsf(v[2 * p + 1]), cap);
+        }
+        const bool out = live && c < chunks;
+        if (out) {
+            uint8_t* fp = xf + ((mt * nst + st) * 8 + 2 * i) * 1024 + ((m & 31) + 32 * h) * 16;
+            *reinterpret_cast<u32x4*>(fp) = hi;
+            *reinterpret_cast<u32x4*>(fp + 1024) = lo;
+        }
+        if constexpr (kK4<QT>) {                         // a, b: four elements of each sub-block, eight lanes
+            float s0 = (a[0] + a[1]) + (a[2] + a[3]), s1 = (b[0] + b[1]) + (b[2] + b[3]);
+            s0 += dpp_mov<0xB1>(s0);
+            s1 += dpp_mov<0xB1>(s1);
+            s0 += dpp_mov<0x4E>(s0);
+            s1 += dpp_mov<0x4E>(s1);
+            s0 += dpp_mov<0x141>(s0);
+            s1 += dpp_mov<0x141>(s1);
+            if ((c & 7) == 0 && out) {
+                const uint32_t p1 = bf16_pair(s0, s1);
+                const float r0 = s0 - bf16_lo(p1), r1 = s1 - bf16_hi(p1);
+                const uint32_t p2 = bf16_pair(r0, r1), p3 = bf16_pair(r0 - bf16_lo(p2), r1 - bf16_hi(p2));
+                uint8_t* sp = xsum + (mt * nst + st) * 1024 + (m & 31) * 16;
+                *reinterpret_cast<u32x4*>(sp) = u32x4{p1, p2, p1, p2};
+                *reinterpret_cast<u32x4*>(sp + 512) = u32x4{p3, p1, 0u, 0u};
+            }
+        }
+    };
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) split(tr + j * TPR, xa[j], xb[j]);
+    } else {
+        for (int c = tr; c < chunks; c += TPR) {
+            f32x4 a, b;
+            load(c, a, b);
+            split(c, a, b);
+        }
+    }
+    const auto add = [](float a, float b) { return a + b; };
+    err = row_reduce<TPR>(err, red[rr], tr, add);
+    body = row_reduce<TPR>(body, red[rr], tr, add);
+    ok = ok && err <= 0x1p-24f * body;
+    if (tr == 0 && live) inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
+}
+
+template <int QT>
+__device__ __forceinline__ u32x4 head_words(const Head<QT>& h) {   // d, dmin and the scales
+    if constexpr (kK4<QT>) return h.hd;
+    else return u32x4{};
+}
+
+// What Q4_K / Q5_K add to a stage: its two sub-blocks' code constants and the
+// B fragment of (R - dmin m / d) 2^-14, to be multiplied by sum(x) (the pieces
+// of split_kernel's fragment: w1 x1, w1 x2, w2 x1, w2 x2 | w1 x3, w3 x1).
+struct K4Stage {
+    f16x2 mul[2], off[2];
+    u32x4 uf;
+    template <int QT, int T>
+    __device__ __forceinline__ void set(const u32x4 hd, int h) {
+        const float d = f16_bits_to_f32(hd[0]), dm = f16_bits_to_f32(hd[0] >> 16);
+        // d = 0: the codes are 0 and the whole weight, -dmin m, is the second term
+        const bool z = d == 0.0f;
+        const float rd = z ? 1.0f : __builtin_amdgcn_rcpf(d);
+        float u[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t sc, mn;
+            k4_scale_min(hd[1], hd[2], hd[3], 2 * T + j, sc, mn);
+            const float s = z ? 0.0f : (float)sc, tm = dm * (float)mn;      // exact
+            // d non-finite: fmaxf drops a NaN, so R lands in range anyway
+            const float R = fminf(fmaxf(__builtin_rintf(tm * rd), 0.0f), (QT == kTypeQ4K ? 15.0f : 31.0f) * s);
+            u[j] = __builtin_fmaf(d, R, -tm) * (rd * 0x1p-14f);             // d R - tm in one rounding
+            mul[j] = pair_of(s * (j ? 64.0f : 1024.0f));
+            off[j] = pair_of(R * -0x1p-14f);
+        }
+        const uint32_t p1 = bf16_pair(u[0], u[1]);
+        const float r0 = u[0] - bf16_lo(p1), r1 = u[1] - bf16_hi(p1);
+        const uint32_t p2 = bf16_pair(r0, r1), p3 = bf16_pair(r0 - bf16_lo(p2), r1 - bf16_hi(p2));
+        uf = u32x4{p1, h ? p3 : p1, h ? 0u : p2, h ? 0u : p2};
+    }
+    __device__ static __forceinline__ float scale(const u32x4 hd) {
+        const float d = f16_bits_to_f32(hd[0]);
+        return d == 0.0f ? 16384.0f : d * 16384.0f;
+    }
+};
+
+// Scheduling of one chain: after each of its N matrix instructions, V of the
+// vector instructions that run beside it and an LDS read.
+template <int N, int V>
+__device__ __forceinline__ void interleave() {
+    static_for<0, N>([&](auto) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, V, 0);   // VALU
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+    });
+}
+
+// WM x WN = 8 waves of 32 MT x 32 NT; LS stages of x per barrier (32 KB),
+// three buffers: period p + 2 is written while p is computed, so the first
+// fragments of p + 1 are read before the barrier. A wave's work is a sequence
+// of chains of matrix instructions, one tile and scale group each: the small
+// lo products before the hi ones (their sums round at their own size), into
+// one of two register sets, while the other one is scaled into its tile's
+// accumulator and the codes to come are made.
+// DEPTH > 1: as many register sets of W, each loaded DEPTH units ahead (few
+// rows of x: the kernel waits for W); else one, whose stages are loaded again,
+// for the next unit, two stages ahead (128 rows: registers).
+template <int QT, int WM, int WN, int MT, int NT, int DEPTH>
+__global__ void __launch_bounds__(512) gemm_pair_kernel(
+    const uint8_t* __restrict__ w, const uint8_t* __restrict__ xf, const uint8_t* __restrict__ xsum,
+    const float* __restrict__ inv, float* __restrict__ y, int M, int N, int K, int units, int64_t ldy, int S,
+    float* __restrict__ part) {
+    static_assert(WM * WN == 8, "eight waves");
+    constexpr bool DB = DEPTH > 1;
+    constexpr int BT = WM * MT, BM = 32 * BT, BN = 32 * WN * NT;
+    constexpr int LS = 4 / BT;                         // stages per barrier
+    static_assert(BT == 1 || BT == 2 || BT == 4, "32 KB of x per barrier");
+    // slices summed before the scale
+    constexpr int GS = QT == kTypeQ6K ? 1 : 4;
+    // vector memory instructions of one period's copies; at least, of W's
+    // loads per stage and per unit
+    constexpr int kCopies = kK4<QT> ? 5 : 4, kStageLoads = NT * Body<QT>::kLoads;
+    constexpr int kUnitLoads = NT * Body<QT>::kHeadLoads + 4 * kStageLoads;
+    constexpr int kTileBytes = LS * kStageBytes, kSumOff = 32768, kBuf = kSumOff + (kK4<QT> ? 4096 : 0);
+    __shared__ __attribute__((aligned(16))) uint8_t xs[4 * kBuf];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % WM, wn = wave / WM, h = lane >> 5;
+    // consecutive tiles on one XCD (workgroups go round the eight XCDs):
+    // its L2 then serves a range of W to all tiles of x, and one split's x
+    const int G = (int)gridDim.x, xcd = (int)blockIdx.x & 7, gq = G >> 3, gr = G & 7;
+    const int id = (xcd < gr ? xcd * (gq + 1) : gr * (gq + 1) + (xcd - gr) * gq) + ((int)blockIdx.x >> 3);
+    const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
+    const int mt0 = (id % mtiles) * BT, rest = id / mtiles, n0 = (rest % ntiles) * BN, split = rest / ntiles;
+    const int u0 = (int)((int64_t)split * units / S), u1 = (int)((int64_t)(split + 1) * units / S);
+
+    constexpr int kUnitBytes = (int)weight_row_bytes<QT>(kUnit), kUnitBlocks = 2;   // Q1_0 blocks
+    const uint8_t* wtile = w + (int64_t)n0 * weight_row_bytes<QT>(K);
+    uint32_t wrow[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int n = 32 * (NT * wn + nt) + (lane & 31);
+        wrow[nt] = (uint32_t)(n0 + n < N ? n : N - 1 - n0) * (uint32_t)weight_row_bytes<QT>(K);
+    }
+    // LDS order of x: [32-row tile][stage][slice][piece][lane], then
+    // [tile][stage][lane] of the sums; a thread moves 16 bytes of each of the
+    // period's four 8 KB parts and 8 of the sums
+    const int tile_units = units * (4 * kStageBytes);  // from one 32-row tile to the next
+    const auto xrs = buffer_rsrc(xf + (int64_t)mt0 * tile_units, (uint32_t)(BT * tile_units));
+    const auto srs = buffer_rsrc(xsum + (int64_t)mt0 * units * 4096, (uint32_t)(BT * units * 4096));
+    const uint32_t sl = 16 * (tid & 255), soff = sl / (LS * 1024) * (uint32_t)units * 4096u + sl % (LS * 1024);
+    const int periods = (u1 - u0) * (4 / LS);          // barriers
+    auto copy_x = [&](int p, int buf) __attribute__((always_inline)) {
+        const int pp = (p < periods ? p : periods - 1) + u0 * (4 / LS);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            lds_copy(xrs, 16 * tid, (uint32_t)(pp * kTileBytes + (j / LS) * tile_units + (j % LS) * kStageBytes),
+                     &xs[buf + kStageBytes * j + 1024 * wave]);
+        if constexpr (kK4<QT>) lds_copy(srs, soff, (uint32_t)(pp * (LS * 1024)), &xs[buf + kSumOff + 1024 * (wave & 3)]);
+    };
+    // fragments of (stage `st` of its period) in the buffer at `buf`
+    auto afrag = [&](int buf, int st, int mt, int i, int pc) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f16x8*>(
+            &xs[buf + (MT * wm + mt) * kTileBytes + st * kStageBytes + (2 * i + pc) * 1024 + lane * 16]);
+    };
+    auto sfrag = [&](int buf, int st, int mt) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8*>(&xs[buf + kSumOff + (MT * wm + mt) * (LS * 1024) + st * 1024 + lane * 16]);
+    };
+
+    constexpr bool kTwo = MT * NT <= 2;                // room for a second level
+    f32x16 acc[MT][NT], tot[kTwo ? MT : 1][NT], t[2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[mt][nt][r] = 0.0f;
+                if (kTwo) tot[kTwo ? mt : 0][nt][r] = 0.0f;
+            }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[1][r] = 0.0f;
+    float tsc = 0.0f;                                  // the scale of the set not yet in acc
+
+    // one set of heads is enough where the last stage's codes are made before
+    // its second chain and the scale is kept apart (K4)
+    constexpr int HS = DB ? DEPTH : kK4<QT> ? 1 : 2, UR = DB ? DEPTH : 2;   // sets, units per round of the loop
+    Head<QT> hd[HS][NT];
+    Body<QT> bd[DEPTH][NT];
+    float d14[NT] = {};
+    auto load_head = [&](Head<QT> (&hh)[NT], int u) __attribute__((always_inline)) {
+        const gptr up = scalar_base(wtile + (int64_t)(u < u1 ? u : u1 - 1) * kUnitBytes);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) hh[nt].load(up, wrow[nt], h);
+    };
+    auto load_body = [&](auto pc, Body<QT> (&bb)[NT], int u) __attribute__((always_inline)) {
+        const int uu = u < u1 ? u : u1 - 1;
+        const gptr up = scalar_base(wtile + (int64_t)uu * kUnitBytes);
+        const int left = K / kQ10Elems - uu * kUnitBlocks;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) bb[nt].template load<decltype(pc)::value>(up, wrow[nt], h, left);
+    };
+
+    // a stage's codes of one 32-row tile of W
+    struct Codes {
+        f16x8 s[GS];
+        bf16x8 u;
+    };
+    // the codes of stage T's slices from group `gc` of GS on
+    auto decode = [&](auto tc, auto gc, const Head<QT>& hh, const Body<QT>& bb) __attribute__((always_inline)) {
+        constexpr int T = decltype(tc)::value, I0 = decltype(gc)::value * GS;
+        Codes c;
+        K4Stage ks;
+        if constexpr (kK4<QT>) {
+            ks.template set<QT, T>(head_words(hh), h);
+            c.u = __builtin_bit_cast(bf16x8, ks.uf);
+        }
+        static_for<0, GS>([&](auto ic) {
+            constexpr int I = I0 + decltype(ic)::value;
+            u32x4 f;
+            if constexpr (kK4<QT>) {
+                f = bb.template fields<T, I>(hh);
+                f[0] = fma2(f[0], ks.mul[0], ks.off[0]);
+                f[1] = fma2(f[1], ks.mul[1], ks.off[1]);
+                f[2] = fma2(f[2], ks.mul[0], ks.off[0]);
+                f[3] = fma2(f[3], ks.mul[1], ks.off[1]);
+            } else {
+                f = bb.template frag<T, I>(hh);
+            }
+            c.s[I - I0] = __builtin_bit_cast(f16x8, f);
+        });
+        return c;
+    };
+
+    // carried from chain to chain: a group's x fragments of one 32-row tile,
+    // its codes and scales
+    f16x8 a[GS][2];
+    float gsc[NT] = {};
+    bf16x8 sx;
+    Codes b[NT];
+    int cur = 0, nxt = kBuf, nx2 = 2 * kBuf, wr3 = 3 * kBuf;   // buffers of periods p .. p + 3
+
+    // one unit: four stages of 64 k; (hn, bn) = the next unit's fields (none in
+    // the tail, whose loads of them are dropped)
+    auto unit = [&](auto tail, Head<QT> (&hh)[NT], Body<QT> (&bb)[NT], Head<QT> (&hn)[NT], Body<QT> (&bn)[NT], int u)
+        __attribute__((always_inline)) {
+        static_for<0, 4>([&](auto tc) {
+            constexpr int T = decltype(tc)::value, TN = (T + 1) & 3;
+            constexpr bool turn = T % LS == LS - 1;    // last stage of its period
+            if constexpr (T % LS == 0) {
+                const int p = (u - u0) * (4 / LS) + T / LS;
+                copy_x(p + 3, wr3);
+                asm volatile("" ::: "memory");         // loads of W stay behind the copies
+            }
+            if constexpr (kK4<QT> && T == 0) {
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) d14[nt] = K4Stage::scale(head_words(hh[nt]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (GS == 4) {
+                static_for<0, MT * NT>([&](auto pc) {
+                    constexpr int PH = decltype(pc)::value, mt = PH / NT, nt = PH % NT;
+                    constexpr bool lastnt = nt == NT - 1, last = PH == MT * NT - 1;
+                    if constexpr (NT == 2 && PH == 0) b[1] = decode(tc, Int<0>{}, hh[1], bb[1]);
+                    Codes b0;
+                    if constexpr (last) {
+                        if constexpr (T < 3) b0 = decode(Int<TN>{}, Int<0>{}, hh[0], bb[0]);
+                        else b0 = decode(Int<0>{}, Int<0>{}, hn[0], bn[0]);
+                    }
+                    // next x fragments: the next tile's, or the next stage's first
+                    f16x8 an[4][2];
+                    bf16x8 sn = sx;
+                    if constexpr (lastnt) {
+                        constexpr int mn = last ? 0 : mt + 1, sn_ = last ? (turn ? 0 : T % LS + 1) : T % LS;
+                        const int buf = last && turn ? nxt : cur;
+                        if constexpr (kK4<QT>) sn = sfrag(buf, sn_, mn);
+#pragma unroll
+                        for (int q = 1; q >= 0; --q)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) an[i][q] = afrag(buf, sn_, mn, i, q);
+                    }
+                    constexpr int C = (T * MT * NT + PH) & 1;          // this chain's set
+                    const f32x16 zero = {};
+                    if constexpr (kK4<QT>) t[C] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sx, b[nt].u, zero, 0, 0, 0);
+#pragma unroll
+                    for (int q = 1; q >= 0; --q)                        // lo, then hi
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            t[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                a[i][q], b[nt].s[i], !kK4<QT> && q == 1 && i == 0 ? zero : t[C], 0, 0, 0);
+                    constexpr int PP = (PH + MT * NT - 1) % (MT * NT);  // the chain before this one
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        acc[PP / NT][PP % NT][r] = __builtin_fmaf(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
+                    if constexpr (kK4<QT>) tsc = d14[nt];
+                    else tsc = bb[nt].template scale<T, 3>(hh[nt]);
+                    if constexpr (last) b[0] = b0;
+                    if constexpr (lastnt) {
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) a[i][q] = an[i][q];
+                        sx = sn;
+                    }
+                    interleave<8 + (kK4<QT> ? 1 : 0), 2 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0)>();
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (!DB && PH == (QT == kTypeQ5K && MT * NT > 2 ? 1 : 0)) {
+                        if constexpr (T == (HS == 1 ? 3 : 2)) load_head(hn, u + 1);
+                        load_body(Int<(T + 2) & 3>{}, bb, T < 2 ? u : u + 1);
+                    }
+                });
+            } else {
+                static_for<0, 4 / GS * MT>([&](auto pc) {
+                    constexpr int G_ = decltype(pc)::value / MT, mt = decltype(pc)::value % MT;
+                    constexpr bool lastmt = mt == MT - 1, last = lastmt && G_ == 4 / GS - 1;
+                    // next x fragments: the next tile's, or the next group's first
+                    constexpr int mn = lastmt ? 0 : mt + 1, gn = (G_ + lastmt) % (4 / GS);
+                    constexpr int sn_ = last ? (turn ? 0 : T % LS + 1) : T % LS;
+                    const int buf = last && turn ? nxt : cur;
+                    f16x8 an[GS][2];
+#pragma unroll
+                    for (int q = 1; q >= 0; --q)
+#pragma unroll
+                        for (int i = 0; i < GS; ++i) an[i][q] = afrag(buf, sn_, mn, gn * GS + i, q);
+                    Codes bx[NT];
+                    if constexpr (lastmt) {
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt) {
+                            if constexpr (!last) bx[nt] = decode(tc, Int<gn>{}, hh[nt], bb[nt]);
+                            else if constexpr (T < 3) bx[nt] = decode(Int<TN>{}, Int<0>{}, hh[nt], bb[nt]);
+                            else bx[nt] = decode(Int<0>{}, Int<0>{}, hn[nt], bn[nt]);
+                        }
+                    }
+                    static_for<0, NT>([&](auto nc) {
+                        constexpr int nt = decltype(nc)::value;
+                        constexpr int C = (((T * (4 / GS) + G_) * MT + mt) * NT + nt) & 1;
+                        const f32x16 zero = {};
+#pragma unroll
+                        for (int q = 1; q >= 0; --q)
+#pragma unroll
+                            for (int i = 0; i < GS; ++i)
+                                t[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i][q], b[nt].s[i],
+                                                                              q == 1 && i == 0 ? zero : t[C], 0, 0, 0);
+                        constexpr int PP = (mt * NT + nt + MT * NT - 1) % (MT * NT);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            acc[PP / NT][PP % NT][r] = __builtin_fmaf(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
+                        if constexpr (mt == 0) gsc[nt] = bb[nt].template scale<T, G_ * GS>(hh[nt]);
+                        tsc = gsc[nt];
+                    });
+                    if constexpr (lastmt) {
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt) b[nt] = bx[nt];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int i = 0; i < GS; ++i) a[i][q] = an[i][q];
+                    interleave<2 * GS * NT, (GS == 1 ? 9 : 5) + (lastmt ? (GS == 1 ? 9 : 7) : 0)>();
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (!DB && G_ == 0 && mt == 0) {
+                        if constexpr (T == 2) load_head(hn, u + 1);
+                        load_body(Int<(T + 2) & 3>{}, bb, T < 2 ? u : u + 1);
+                    }
+                });
+            }
+            if constexpr (turn) {
+                // Vector memory instructions finish in order: the copies of two
+                // periods ahead are done when all but this period's copies and
+                // the loads of W issued after the former are. Every wave has
+                // then used its fragments of this period.
+                constexpr int loads = decltype(tail)::value ? 0 : !DB ? LS * kStageLoads : T < LS ? kUnitLoads : 0;
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCopies + loads) : "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                const int tmp = cur;
+                cur = nxt;
+                nxt = nx2;
+                nx2 = wr3;
+                wr3 = tmp;
+            }
+        });
+    };
+
+    auto load_unit = [&](Head<QT> (&hh)[NT], Body<QT> (&bb)[NT], int u) __attribute__((always_inline)) {
+        load_head(hh, u);
+        static_for<0, 4>([&](auto tc) { load_body(tc, bb, u); });
+    };
+
+    copy_x(0, 0);
+    copy_x(1, kBuf);
+    copy_x(2, 2 * kBuf);
+    asm volatile("" ::: "memory");
+    if constexpr (DB) {
+        static_for<0, DEPTH>([&](auto jc) {
+            constexpr int J = decltype(jc)::value;
+            load_unit(hd[J], bd[J], u0 + J);
+        });
+    } else {
+        load_head(hd[0], u0);
+        load_body(Int<0>{}, bd[0], u0);
+        load_body(Int<1>{}, bd[0], u0);
+    }
+    // the first two periods' copies, as above
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kCopies + (DB ? DEPTH * kUnitLoads : NT * Body<QT>::kHeadLoads + 2 * kStageLoads))
+                 : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int i = 0; i < GS; ++i) a[i][q] = afrag(0, 0, 0, i, q);
+    if constexpr (kK4<QT>) sx = sfrag(0, 0, 0);
+#pragma unroll
+    for (int nt = 0; nt < (GS == 4 ? 1 : NT); ++nt) b[nt] = decode(Int<0>{}, Int<0>{}, hd[0][nt], bd[0][nt]);
+    // a unit's sums into the result's (the one still in t joins the next unit's)
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (kTwo) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    tot[mt][nt] += acc[mt][nt];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+                }
+        }
+    };
+    int u = u0;
+    for (; u + UR <= u1; u += UR) {
+        static_for<0, UR>([&](auto jc) {
+            constexpr int J = decltype(jc)::value, JN = (J + 1) % UR;
+            unit(Int<0>{}, hd[J % HS], bd[J % DEPTH], hd[JN % HS], bd[JN % DEPTH], u + J);
+            flush();
+            if constexpr (DB) {
+                load_unit(hd[J], bd[J], u + J + DEPTH);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+    }
+    static_for<0, UR - 1>([&](auto jc) {               // the last, incomplete round
+        constexpr int J = decltype(jc)::value, JN = (J + 1) % UR;
+        if (u + J < u1) {
+            unit(Int<1>{}, hd[J % HS], bd[J % DEPTH], hd[JN % HS], bd[JN % DEPTH], u + J);
+            flush();
+        }
+    });
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[MT - 1][NT - 1][r] = __builtin_fmaf(tsc, t[1][r], acc[MT - 1][NT - 1][r]);
+    if constexpr (kTwo) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] += tot[mt][nt];
+    }
+
+    float* out = S == 1 ? y : part + (int64_t)split * M * N;
+    const int64_t ld = S == 1 ? ldy : N;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = 32 * (mt0 + MT * wm + mt) + 8 * i + 4 * h;
+            f32x4 f = {1.0f, 1.0f, 1.0f, 1.0f};
+            if (S == 1) f = *reinterpret_cast<const f32x4*>(inv + m);   // inv is padded to whole tiles
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int n = n0 + 32 * (NT * wn + nt) + (lane & 31);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (m + r < M && n < N) out[(int64_t)(m + r) * ld + n] = acc[mt][nt][4 * i + r] * f[r];
+            }
+        }
+}
+
+// S > 1: y = inv * (the planes added in split order, in fp64: free here, and
+// one rounding instead of S). Then, S = 1 too, the rows
+// that the pairs do not carry (inv = 0), weight by weight in fp64, a wave per
+// output over the whole grid.
+template <int QT>
+__global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ part, float* __restrict__ y, int S,
+                                                     int M, int N, int64_t ldy, const float* __restrict__ inv,
+                                                     const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                     int K) {
+    const int64_t plane = (int64_t)M * N;
+    if (S > 1) {
+        if (((N | ldy) & 3) == 0 && !(reinterpret_cast<uintptr_t>(y) & 15)) {
+            const int nq = N >> 2;
+            const int64_t total = (int64_t)M * nq, step = (int64_t)gridDim.x * 256;
+            for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += step) {
+                const int m = (int)(e / nq), n = 4 * (int)(e - (int64_t)m * nq);
+                const float* p = part + (int64_t)m * N + n;
+                f64x4 v = {};
+                for (int q0 = 0; q0 < S; q0 += 8) {      // eight loads in flight
+                    f32x4 t[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) t[q] = *reinterpret_cast<const f32x4*>(p + (q0 + q < S ? q0 + q : 0) * plane);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        if (q0 + q < S) v += __builtin_convertvector(t[q], f64x4);
+                }
+                const float f = inv[m];
+                if (f != 0.0f)
+                    *reinterpret_cast<f32x4*>(y + (int64_t)m * ldy + n) = __builtin_convertvector(v * (double)f, f32x4);
+            }
+        } else {
+            const int64_t step = (int64_t)gridDim.x * 256;
+            for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < plane; e += step) {
+                const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
+                const double v = sum_planes<double>([&](int q) { return (double)part[e + q * plane]; }, S);
+                const float f = inv[m];
+                if (f != 0.0f) y[(int64_t)m * ldy + n] = (float)(v * f);
+            }
+        }
+    }
+    const int lane = threadIdx.x & 63, wv = (int)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int)gridDim.x * 4;
+    for (int m0 = 0; m0 < M; m0 += 64) {                // every wave scans all rows of inv
+        uint64_t hit = __ballot(m0 + lane < M && inv[m0 + lane < M ? m0 + lane : 0] == 0.0f);
+        while (hit) {
+            const int m = m0 + __builtin_ctzll(hit);
+            hit &= hit - 1;
+            const float* xr = x + (int64_t)m * K;
+            for (int n = wv; n < N; n += waves) {
+                const uint8_t* wr = w + (int64_t)n * weight_row_bytes<QT>(K);
+                double s = 0.0;
+                for (int j = lane; j < K; j += 64) s = __builtin_fma((double)weight_at<QT>(wr, j), (double)xr[j], s);
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+                if (lane == 0) y[(int64_t)m * ldy + n] = (float)s;
+            }
+        }
+    }
+}
+
+template <int QT, int WM, int WN, int MT, int NT, int DEPTH>
+void pair_go(const PairPlan& p, const uint8_t* w, float* y, int64_t ldy, hipStream_t s, uint8_t* scratch) {
+    const int64_t ntiles = (p.n + 32 * WN * NT - 1) / (32 * WN * NT), mtiles = (p.m + 32 * WM * MT - 1) / (32 * WM * MT);
+    gemm_pair_kernel<QT, WM, WN, MT, NT, DEPTH><<<dim3((unsigned)(ntiles * mtiles * p.splits)), dim3(512), 0, s>>>(
+        w, scratch + p.x_off, scratch + p.sum_off, reinterpret_cast<const float*>(scratch), y, (int)p.m, (int)p.n,
+        (int)p.k, (int)p.units, ldy, p.splits, reinterpret_cast<float*>(scratch + p.part_off));
+}
+
+// Few rows: 1024 threads each, for latency; more: enough threads that every
+// one holds two to five pieces of the row in registers.
+template <int QT, int RW, int TPR, int NC>
+void split_launch(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv) {
+    const unsigned grid = (unsigned)((p.m + 63) / 64 * 64 / RW);
+    split_kernel<QT, RW, TPR, NC><<<dim3(grid), dim3(RW * TPR), 0, s>>>(x, (int)p.m, (int)p.k, (int)p.units, xf, xsum, inv);
+}
+template <int QT>
+void split_go(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv) {
+    const int64_t chunks = p.units * 32;
+    if (p.m <= 64 && chunks > 512) {
+        if (chunks <= 1024) return split_launch<QT, 1, 1024, 1>(p, x, s, xf, xsum, inv);
+        if (chunks <= 2048) return split_launch<QT, 1, 1024, 2>(p, x, s, xf, xsum, inv);
+        if (chunks <= 3072) return split_launch<QT, 1, 1024, 3>(p, x, s, xf, xsum, inv);
+    }
+    if (chunks <= 256) return split_launch<QT, 4, 128, 2>(p, x, s, xf, xsum, inv);
+    if (chunks <= 512) return split_launch<QT, 2, 256, 2>(p, x, s, xf, xsum, inv);
+    if (chunks <= 1024) return split_launch<QT, 2, 256, 4>(p, x, s, xf, xsum, inv);
+    if (chunks <= 2560) return split_launch<QT, 1, 512, 5>(p, x, s, xf, xsum, inv);
+    split_launch<QT, 1, 1024, 0>(p, x, s, xf, xsum, inv);
+}
+
+template <int QT>
+void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int64_t ldy, hipStream_t s,
+              uint8_t* scratch, bool x_ready) {
+    float* inv = reinterpret_cast<float*>(scratch);
+    if (!x_ready) split_go<QT>(p, x, s, scratch + p.x_off, scratch + p.sum_off, inv);
+    if (p.bm == 32)
+        pair_go<QT, 1, 8, 1, 1, 2>(p, w, y, ldy, s, scratch);
+    else if (p.bm == 64)
+        pair_go<QT, 1, 8, 2, 1, QT == kTypeQ10 ? 2 : 1>(p, w, y, ldy, s, scratch);
+    else if constexpr (QT == kTypeQ4K || QT == kTypeQ6K)
+        pair_go<QT, 2, 4, 2, 2, 1>(p, w, y, ldy, s, scratch);
+    const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
+    const unsigned fin = (unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work);
+    finish_kernel<QT><<<dim3(fin), dim3(256), 0, s>>>(reinterpret_cast<const float*>(scratch + p.part_off), y,
+                                                      p.splits, (int)p.m, (int)p.n, ldy, inv, w, x, (int)p.k);
+}
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+}  // namespace
+
+bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, PairPlan* p) {
+    const int64_t kq = qtype == kTypeQ10 ? kQ10Elems
+                       : (qtype == kTypeQ4K || qtype == kTypeQ5K || qtype == kTypeQ6K) ? kQKElems
+                                                                                      : 0;
+    if (kq == 0 || m <= 0 || n <= 0 || k <= 0 || k % kq || m > kPairRows || n > 0x3FFFFFFF || k > (1 << 22))
+        return false;
+    const bool k4 = qtype == kTypeQ4K || qtype == kTypeQ5K;
+    p->m = m;
+    p->n = n;
+    p->k = k;
+    p->units = (k + kUnit - 1) / kUnit;
+    p->bn = 256;
+    p->layout = k4 ? kTypeQ4K : qtype;
+    const int64_t ntiles = (n + p->bn - 1) / p->bn;
+    // The row tile and the split of k with the least estimated time: rounds of
+    // 256 workgroups (one per CU), each its share of units and a fixed start,
+    // and every plane written and read. Per unit, measured with k unsplit (us):
+    // 2.9 for 32 rows, 3.9 for 64, 7.0 for 128 (Q6_K 9.0).
+    const double plane_us = (double)m * (double)n * 8.0 / 2.5e6;
+    // Q5_K and Q1_0, whose rows otherwise run one GEMV each, keep to the tiles
+    // with two-level sums, which match a GEMV's error.
+    const bool wide = qtype == kTypeQ4K || qtype == kTypeQ6K;
+    const int bms[2] = {m <= 32 ? 32 : 64, m <= 32 ? 32 : m <= 64 || !wide ? 64 : 128};
+    double best = 0.0;
+    bool found = false;
+    for (int c = 0; c < 2; ++c) {
+        const int bm = bms[c];
+        const int64_t mtiles = (m + bm - 1) / bm, mpad = mtiles * bm;
+        const size_t sum_off = align256((size_t)mpad * 4), x_off = sum_off + (k4 ? (size_t)(mpad / 32 * p->units) * 4096 : 0);
+        const size_t part_off = x_off + (size_t)mpad * (size_t)p->units * kUnit * 4;
+        if (part_off > cap) continue;
+        const double unit_us = bm == 32 ? 2.9 : bm == 64 ? 3.9 : qtype == kTypeQ6K ? 9.0 : 7.0, start_us = 6.0;
+        for (int64_t s = 1; s <= 64 && s <= p->units; ++s) {
+            const size_t bytes = s > 1 ? (size_t)s * (size_t)m * (size_t)n * 4 : 0;
+            if (part_off + bytes > cap) break;
+            const double rounds = (double)((mtiles * ntiles * s + 255) / 256);
+            const double us = rounds * (start_us + (double)((p->units + s - 1) / s) * unit_us) + (s > 1 ? s * plane_us + 1.0 : 0.0);
+            if (!found || us < best) {
+                found = true;
+                best = us;
+                p->bm = bm;
+                p->splits = (int)s;
+                p->sum_off = sum_off;
+                p->x_off = x_off;
+                p->part_off = part_off;
+            }
+        }
+    }
+    if (!found) return false;
+    p->bytes = p->part_off + (p->splits > 1 ? (size_t)p->splits * (size_t)m * (size_t)n * 4 : 0);
+    return true;
+}
+
+hipError_t launch_gemm_pair(int qtype, const uint8_t* w, const float* x, float* y, int64_t ldy, const PairPlan& p,
+                            hipStream_t stream, uint8_t* scratch, bool x_ready) {
+    if (ldy < p.n || (reinterpret_cast<uintptr_t>(x) & 15) || !scratch) return hipErrorInvalidValue;
+    const uintptr_t wa = reinterpret_cast<uintptr_t>(w);
+    if (qtype == kTypeQ4K || qtype == kTypeQ5K ? (wa & 15) : (wa & 1)) return hipErrorInvalidValue;
+    switch (qtype) {
+        case kTypeQ4K: pair_run<kTypeQ4K>(p, w, x, y, ldy, stream, scratch, x_ready); break;
+        case kTypeQ5K: pair_run<kTypeQ5K>(p, w, x, y, ldy, stream, scratch, x_ready); break;
+        case kTypeQ6K: pair_run<kTypeQ6K>(p, w, x, y, ldy, stream, scratch, x_ready); break;
+        case kTypeQ10: pair_run<kTypeQ10>(p, w, x, y, ldy, stream, scratch, x_ready); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace frq

@@ -162,17 +162,23 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  * and of max |y| (normwise) -- including outliers x_j on weights that are
  * exactly zero while their scales are not (d*sc*q = dmin*m), where a sum
  * written as s * sum(q x) - t * sum(x) in fp32 would cancel.
- * batch >= 2 with Q4_K, Q6_K or Q8_0 (x 16-byte aligned, k a multiple of the
- * block) is one fp32-contract GEMM that reads W once per 32 or 64 rows of x:
- * bf16 matrix cores on exact integer codes (Q4_K q - c with c the code
- * nearest dmin*m / d*sc, so every term stays within 3 |w_j x_j|) and on x
- * split into three bf16 pieces (all 24 bits of every x in {0} U
- * [2^-100, 2^100]), fp32 sums per sub-block, then the sub-block scales in
- * fp32 -- the same error bound, other bits than one row at a time. A row of
- * x with any value outside that range (tiny, subnormal, huge, inf, NaN) is
- * computed again weight by weight in fp64 (one rounding; inf and NaN as
- * IEEE arithmetic has them) by a second kernel. A few
- * rows run a small-M matvec instead, W read once per launch: Q4_K with 4
+ * batch >= 2 (x 16-byte aligned, k a multiple of the block) reads W once per
+ * tile of x rows, with the same error bound and other bits than one row at a
+ * time, by one of two fp32-contract GEMMs:
+ *   Q4_K, Q5_K, Q6_K, Q1_0 (frq_gemm_pair.hip): fp16 matrix cores on exact
+ * integer codes (Q4_K / Q5_K sc q - R with R the integer nearest dmin*m / d,
+ * so every term stays within 3 |w_j x_j|) and on x as hi + lo, two fp16 values
+ * under a power of two per row of x: every element down to 2^-16 of the row's
+ * largest to within 2^-23 of itself, smaller ones to within 2^-40 of the
+ * largest. A row whose elements that loses more than 2^-24 of its sum |x|
+ * (outliers capped at 2^-10 of the largest), or with an inf, a NaN or a largest
+ * |x| outside [2^-100, 2^101), is computed weight by weight in fp64 (one
+ * rounding; inf and NaN as IEEE arithmetic has them).
+ *   Q8_0, small Q4_K and Q6_K matrices (n k < 24 M; Q4_K up to 64 rows), and
+ * Q4_K / Q6_K where the former's scratch cannot be had (frq_gemm_f32.hip): x as
+ * three bf16 pieces (all 24 bits of every x in {0} U [2^-100, 2^100]); rows
+ * with any other value weight by weight in fp64.
+ * A few rows run a small-M matvec instead, W read once per launch: Q4_K with 4
  * rows (k <= 24576), or 5 to 8 rows where k <= 8192, in one launch of the
  * fp32 matrix-core matvec (per-weight dequant, each product fused into an
  * fp32 sum by v_mfma_f32_4x4x1_16b_f32; a row's bits independent of the
@@ -182,8 +188,9 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  * the same in any batch this kernel takes; Q6_K and Q8_0 with the bits of a
  * batch-1 call); up to 3 rows that neither takes run one GEMV per row. Few output
  * tiles split k over workgroups whose fp32 partials a second kernel adds in
- * a fixed order (scratch of the stream). Q5_K and Q1_0 run one matvec per
- * row. */
+ * a fixed order. Scratch of the stream: the pairs (4 bytes per element of up to
+ * 1024 rows of x, padded to the tile) and the partials, at most 1 GiB; a
+ * stream under capture that has less runs the kernels that need less. */
 int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
                  int64_t batch, void* stream);
 
@@ -199,9 +206,10 @@ int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float
  * longer than one workgroup). A batch-1 shape that needs more is refused
  * with FRQ_ERR_UNSUPPORTED before anything is launched. A batch that takes
  * a small-M matvec (see frq_dev_gemv) needs no scratch; a batch that takes
- * the batched GEMM (more rows of Q4_K, Q6_K, Q8_0) keeps one flag word per row of x
- * in the 3 MiB and splits k only as far as its partials (splits x batch x n
- * x 4 bytes) fit beside them, so neither is refused (up to 786432 rows); where the GEMM splits less than
+ * a batched GEMM keeps its pairs of x in the 3 MiB where they fit (Q4_K and Q6_K
+ * else run the GEMM with one flag word per row of x, Q5_K and Q1_0 one GEMV per
+ * row) and splits k only as far as its partials (splits x batch x n
+ * x 4 bytes) fit beside them, so none is refused (up to 786432 rows); where the GEMM splits less than
  * frq_dev_gemv would, the bits differ from frq_dev_gemv's within the same
  * bound. Any other batch runs one GEMV per row and is refused as batch 1
  * would be (for example 2 or 3 rows of Q4_K with k > 24576). Every call on a GPU shares that GPU's array: calls that overlap

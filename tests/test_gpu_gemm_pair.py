@@ -1,0 +1,110 @@
+"""The batched matvec on pairs of fp16 values (frq_gemm_pair.hip) against the
+oracle, at the sizes where its tiles, units and splits end.
+
+Rows around the 32-, 64- and 128-row tiles, columns around the 256-column tile
+(one wave, one lane short of it), rows of W from one block to several units
+with a remainder in every split, each format, and rows of x that the pairs do
+not carry (outliers far above the rest, non-finite values), which are computed
+weight by weight. The bound is the matvec's: 1e-5 of sum |w_j x_j| per output
+and of max |y| per row (conftest.assert_matvec_close).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from conftest import assert_matvec_close, bits_equal
+from flatrun_amd import device, synth
+from oracle import gguf_np as G
+
+pytestmark = pytest.mark.gpu
+
+
+def run(q, raw, xs, n, k):
+    b = xs.shape[0]
+    w, xd = device.DeviceBuffer.from_host(raw), device.DeviceBuffer.from_host(xs)
+    yd = device.DeviceBuffer.from_host(np.full(b * n, np.nan, np.float32))
+    try:
+        device.gemv(q, w, xd, yd, n, k, batch=b)
+        device.synchronize()
+        return yd.to_host(np.float32).reshape(b, n)
+    finally:
+        for d in (w, xd, yd):
+            d.free()
+
+
+def check(q, raw, xs, n, k, y, what):
+    y64, a64 = G.matmul_f64(q, xs, raw, n, k), G.abs_matmul_f64(q, xs, raw, n, k)
+    for r in range(xs.shape[0]):
+        assert_matvec_close(y[r], y64[r], a64[r], what=f"{what} row {r}")
+
+
+@pytest.mark.parametrize("q,n,k,rows", [
+    ("Q5_K", 1, 256, 4), ("Q5_K", 255, 512, 31), ("Q5_K", 257, 1280, 32), ("Q5_K", 289, 768, 33),
+    ("Q5_K", 300, 4352, 64), ("Q5_K", 513, 256, 65), ("Q5_K", 256, 2304, 97), ("Q5_K", 33, 20992, 7),
+    ("Q1_0", 1, 128, 4), ("Q1_0", 31, 384, 5), ("Q1_0", 257, 640, 32), ("Q1_0", 300, 4224, 63),
+    ("Q1_0", 256, 2048, 130), ("Q1_0", 65, 18944, 33),
+    ("Q4_K", 255, 256, 65), ("Q4_K", 257, 1280, 129), ("Q4_K", 300, 2816, 100), ("Q4_K", 64, 1024, 1030),
+    ("Q4_K", 1500, 16384, 7), ("Q4_K", 1500, 16384, 40), ("Q6_K", 1500, 16384, 11), ("Q6_K", 1501, 16640, 33),
+    ("Q6_K", 1500, 16384, 70), ("Q6_K", 6001, 4096, 129),
+])
+def test_edges(frq, q, n, k, rows):
+    raw = synth.make_blocks(q, n, k, seed=n + k)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    y = run(q, raw, xs, n, k)
+    some = sorted({0, 1, 30, 31, 32, 63, 64, 95, 96, 127, 128, rows // 2, rows - 2, rows - 1} & set(range(rows)))
+    check(q, raw, xs[some], n, k, y[some], f"{q} {n}x{k} rows {rows}")
+
+
+@pytest.mark.parametrize("q,n,k,rows", [("Q5_K", 70, 4096, 9), ("Q1_0", 70, 4096, 40), ("Q4_K", 70, 2048, 66)])
+def test_rows_beyond_the_pairs(frq, q, n, k, rows):
+    """Outliers from 2^14 to 2^40 above the rest, all rows tiny or huge, one inf
+    and one NaN: every finite row meets the bound, the others are not finite,
+    and ordinary rows keep their bits."""
+    raw = synth.make_blocks(q, n, k, seed=5)
+    xs = synth.make_x(k, seed=6, batch=rows)
+    calm = xs.copy()
+    for r, e in ((0, 14), (1, 18), (2, 24), (3, 40)):
+        xs[r, 7 * r + 3] = 2.0**e
+    xs[4] *= np.float32(2.0**-120)
+    xs[5] *= np.float32(2.0**105)
+    xs[6, 11] = np.inf
+    xs[7, 12] = np.nan
+    y = run(q, raw, xs, n, k)
+    check(q, raw, xs[:4], n, k, y[:4], q)
+    W = G.DEQUANT[q](raw, (n, k), np.float32).astype(np.float64)
+    for r in (4, 5):
+        x64 = xs[r].astype(np.float64)
+        with np.errstate(over="ignore"):
+            ok = np.abs(W @ x64) < float(np.finfo(np.float32).max) / 2
+        err, bound = np.abs(y[r] - W @ x64), 1e-5 * (np.abs(W) @ np.abs(x64)) + k * 2.0**-150
+        assert np.all(err[ok] <= bound[ok]), r
+    assert not np.any(np.isfinite(y[6][W[:, 11] != 0])) and np.all(np.isnan(y[7]))
+    assert bits_equal(y[8:], run(q, raw, calm, n, k)[8:])
+
+
+def test_group_shares_the_pairs(frq):
+    """A group whose matrices take both element orders (Q5_K and Q6_K / Q1_0):
+    each has the bits it has alone."""
+    k, rows = 1024, 70
+    qs, ns = ("Q5_K", "Q1_0", "Q4_K", "Q5_K"), (300, 70, 256, 33)
+    raws = [synth.make_blocks(q, n, k, seed=n) for q, n in zip(qs, ns)]
+    xs = synth.make_x(k, seed=3, batch=rows)
+    ws = [device.DeviceBuffer.from_host(r) for r in raws]
+    xd, yd = device.DeviceBuffer.from_host(xs), device.DeviceBuffer(4 * rows * sum(ns))
+    try:
+        off, parts = 0, []
+        for q, n, w, r in zip(qs, ns, ws, raws):
+            parts.append((q, w, n, yd.ptr + 4 * off, r.nbytes))
+            off += n
+        device.gemv_group(parts, xd, k, batch=rows, y_stride=sum(ns))
+        device.synchronize()
+        y = yd.to_host(np.float32).reshape(rows, sum(ns))
+    finally:
+        for b in ws + [xd, yd]:
+            b.free()
+    off = 0
+    for q, n, r in zip(qs, ns, raws):
+        assert bits_equal(y[:, off:off + n], run(q, r, xs, n, k)), q
+        off += n
