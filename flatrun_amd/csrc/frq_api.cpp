@@ -306,7 +306,7 @@ constexpr int64_t kRowsBeforeGemm = 3;
 
 // Formats without a small-M kernel and gemm_f32 (Q5_K, Q1_0): one GEMV per row
 // below this many rows, the pair GEMM from there on (us, rows 2 / 4 / 8: Q5_K
-// 4096 x 4096 17.8 / 35.5 / 71 by rows, 18.6 from 4 by the pair GEMM; Q1_0
+// 4096 x 4096 10.6 / 21 / 42 by rows, 18.6 from 4 by the pair GEMM; Q1_0
 // 2048 x 2048 6.5 / 12.9 / 28 and 15).
 constexpr int64_t kPairRowsMin = 4;
 

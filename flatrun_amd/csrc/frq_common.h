@@ -342,9 +342,15 @@ struct PairDecode {
     }
 };
 
-template <int CPL>
-struct Q4KRow {
+// A lane's loads of one row of Q4_K or (Q5) Q5_K.
+template <int CPL, bool Q5 = false>
+struct KRow {
     uint4 hd;
+    uint4 q[CPL];
+};
+template <int CPL>
+struct KRow<CPL, true> {
+    uint4 hd, qh;
     uint4 q[CPL];
 };
 

@@ -97,14 +97,20 @@ __device__ __forceinline__ void finish_rows(int64_t row0, int64_t row_end, float
 // rows 0 .. H-1, to y) and the same rows of w2 (ring rows H .. 2H-1, to y2),
 // so a pair of matrices shares one x load and one unbroken load pipeline;
 // thread r then writes both rows r and keeps them in keep[r], keep[H + r].
-template <int CPL, int U, int R, bool PRIO = false, int H = 0>
+//
+// Q5: the same body for Q5_K (CPL 1): 16 more header bytes per lane, bit 2g
+// (2g + 1) of qh byte i the fifth bit of element i of sub-block 2g (2g + 1)
+// (gguf.py:252-262).
+template <int CPL, int U, int R, bool PRIO = false, int H = 0, bool Q5 = false>
 __device__ __forceinline__ void gemv_q4_k_body(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                float* __restrict__ y, int64_t n, int nb, int64_t wg,
                                                float* keep = nullptr, const uint8_t* __restrict__ w2 = nullptr,
                                                float* __restrict__ y2 = nullptr) {
     static_assert(H == 0 || R == 2 * H, "two matrices: R = 2H");
     static_assert(U <= R, "ring deeper than the row count");
+    static_assert(!Q5 || CPL == 1, "Q5_K: 16-byte units");
     __shared__ float red[R * 64];                           // [row][wave][DPP row]
+    constexpr int kBlk = Q5 ? kQ5KBytes : kQ4KBytes, kQs = kBlk - 128;
     constexpr int LPB = 8 / CPL;
     constexpr int NE = 16 * CPL;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
@@ -125,27 +131,31 @@ __device__ __forceinline__ void gemv_q4_k_body(const uint8_t* __restrict__ w, co
     // CPL = 1: codes enter as q * u, u = the value of the fp8 code 1 (a power
     // of two): a nibble below 16 in a byte converts exactly, two per
     // instruction; the scales carry 1 / u so that s' * (q u) = s q exactly.
-    const float u_inv = 1.0f / fp8_unit();
+    // (a five-bit code does not; it converts byte by byte)
+    const float u_inv = Q5 ? 1.0f : 1.0f / fp8_unit();
+    // rotations that take the fifth bits to bit 4 of their bytes
+    const uint32_t rot_lo = (uint32_t)(2 * g + 28) & 31u, rot_hi = (uint32_t)(2 * g + 29) & 31u;
     row_priority<PRIO, R, 0>();                             // x and the first rows load at the top priority
 
     constexpr int RM = H ? H : R;                           // rows per matrix
     const int64_t row0 = rb * RM;
     const int nrows = (int)(n - row0 < RM ? n - row0 : RM);
-    const int64_t row_bytes = (int64_t)nb * kQ4KBytes;
-    const uint32_t hoff = (uint32_t)gblk * kQ4KBytes;       // lane's block inside a row
-    const uint32_t qoff = hoff + 16 + 32 * g + 16 * hh;
+    const int64_t row_bytes = (int64_t)nb * kBlk;
+    const uint32_t hoff = (uint32_t)gblk * kBlk;            // lane's block inside a row
+    const uint32_t qoff = hoff + kQs + 32 * g + 16 * hh;
 
     // Loads are unconditional (no control flow around them): rows past the
     // end re-read the last row (cache hits; results not stored), and inactive
     // lanes read block 0 with x zeroed and their partial forced to 0. Each row
     // is one buffer descriptor (wave-uniform, scalar registers) read at the
     // lane's 32-bit offset: no VALU address math per row.
-    auto load1 = [&](Q4KRow<CPL>& t, int j) {
+    auto load1 = [&](KRow<CPL, Q5>& t, int j) {
         const uint8_t* base = (H && j >= H) ? w2 : w;
         const int jr = (H && j >= H) ? j - H : j;
         const uint8_t* rp = base + (row0 + (jr < nrows ? jr : nrows - 1)) * row_bytes;
         const auto rs = buffer_rsrc(rp, (uint32_t)row_bytes);
         t.hd = bload_b128(rs, hoff);
+        if constexpr (Q5) t.qh = bload_b128(rs, hoff + 16 + 16 * hh);
 #pragma unroll
         for (int c = 0; c < CPL; ++c) t.q[c] = bload_b128(rs, qoff + 16 * c);
     };
@@ -168,14 +178,14 @@ __device__ __forceinline__ void gemv_q4_k_body(const uint8_t* __restrict__ w, co
     // the scheduler from reordering the phases. Inactive lanes keep block 0's
     // x; their partial is discarded by a select below.
     __builtin_amdgcn_sched_barrier(0);
-    Q4KRow<CPL> ring[U];
+    KRow<CPL, Q5> ring[U];
 #pragma unroll
     for (int i = 0; i < U; ++i) load1(ring[i], i);
     __builtin_amdgcn_sched_barrier(0);
 
     static_for<0, R>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        Q4KRow<CPL>& t = ring[j % U];
+        KRow<CPL, Q5>& t = ring[j % U];
         row_priority<PRIO, R, j>();
         // everything read from the slot is read before the slot is refilled
         const float d = f16_bits_to_f32(t.hd.x), dm = f16_bits_to_f32(t.hd.x >> 16);
@@ -206,8 +216,21 @@ __device__ __forceinline__ void gemv_q4_k_body(const uint8_t* __restrict__ w, co
 #pragma unroll
             for (int wd = 0; wd < 4; ++wd) {
                 float f[8];                                       // plane A, plane B
-                if constexpr (CPL == 1) nibbles8_fp8(qw[wd], f);
-                else nibbles8(qw[wd], f);
+                if constexpr (Q5) {
+                    // a 32-bit rotate: bits that wrap land outside bit 4 of every byte
+                    const uint32_t h = wd == 0 ? t.qh.x : wd == 1 ? t.qh.y : wd == 2 ? t.qh.z : t.qh.w;
+                    const uint32_t lo = vand_or(qw[wd], 0x0F0F0F0Fu, vand(__builtin_amdgcn_alignbit(h, h, rot_lo), 0x10101010u));
+                    const uint32_t hi = vand_or(qw[wd] >> 4, 0x0F0F0F0Fu, vand(__builtin_amdgcn_alignbit(h, h, rot_hi), 0x10101010u));
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        f[b] = byte_f(lo, b);
+                        f[4 + b] = byte_f(hi, b);
+                    }
+                } else if constexpr (CPL == 1) {
+                    nibbles8_fp8(qw[wd], f);
+                } else {
+                    nibbles8(qw[wd], f);
+                }
                 const int e = 16 * c + 4 * wd;
                 a0 = __builtin_fmaf(__builtin_fmaf(sa, f[0], -ta), xl[e + 0], a0);
                 a1 = __builtin_fmaf(__builtin_fmaf(sa, f[1], -ta), xl[e + 1], a1);
@@ -251,8 +274,19 @@ gemv_q4_k_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, flo
     gemv_q4_k_body<CPL, U, R, (R >= 14)>(w, x, y, n, nb, blockIdx.x);
 }
 
+// Q5_K through the same ring (U = 3 slots of 48 bytes). Bound by the wave's
+// load -> convert -> FMA chain, as Q4_K. Measured against the batch kernel
+// below, which drains its loads every four rows (us): 14336 x 4096 16.2 -> 11.3
+// (3.6 TB/s), 3584 x 18944 26.6 -> 13.6, 4096 x 4096 9.3 -> 5.3, 1024 x 1024 5.4 -> 4.6.
+// Rows per workgroup as Q4_K.
+template <int U, int R>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4)))
+gemv_q5_k_ring_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, float* __restrict__ y, int64_t n, int nb) {
+    gemv_q4_k_body<1, U, R, (R >= 14), 0, true>(w, x, y, n, nb, blockIdx.x);
+}
+
 // ------------------------------------------------------------------ Q5_K
-// Work unit: one 32-byte qs group g (64 elements, 4 lanes per block). The
+// (explicit geometries only: frq_dev_gemv_tuned with cpl 1.) Work unit: one 32-byte qs group g (64 elements, 4 lanes per block). The
 // 5th bit of element base+i is bit 2g (low nibble) / 2g+1 (high nibble) of
 // qh byte i (gguf.py:252-262).
 template <int U>
@@ -1045,6 +1079,30 @@ bool q6k_rows(int rows, dim3 gd, dim3 bd, hipStream_t s, const uint8_t* w, const
     }
 }
 
+// Q5_K ring kernel: work unit 8 in GemvPlan::cpl (8 lanes per block).
+constexpr int kQ5KRingUnit = 8;
+
+template <int U, int R>
+void q5k_go(dim3 gd, dim3 bd, hipStream_t s, const uint8_t* w, const float* x, float* y, int64_t n, int nb) {
+    gemv_q5_k_ring_kernel<(U < R ? U : R), R><<<gd, bd, 0, s>>>(w, x, y, n, nb);
+}
+
+hipError_t launch_q5k_ring(int rows, int waves, int64_t grid, const uint8_t* w, const float* x, float* y, int64_t n,
+                           int nb, hipStream_t s) {
+    const dim3 gd((unsigned)grid), bd((unsigned)(64 * waves));
+    switch (rows) {
+        case 1: q5k_go<3, 1>(gd, bd, s, w, x, y, n, nb); break;
+        case 2: q5k_go<3, 2>(gd, bd, s, w, x, y, n, nb); break;
+        case 4: q5k_go<3, 4>(gd, bd, s, w, x, y, n, nb); break;
+        case 7: q5k_go<3, 7>(gd, bd, s, w, x, y, n, nb); break;
+        case 8: q5k_go<3, 8>(gd, bd, s, w, x, y, n, nb); break;
+        case 14: q5k_go<3, 14>(gd, bd, s, w, x, y, n, nb); break;
+        case 16: q5k_go<3, 16>(gd, bd, s, w, x, y, n, nb); break;
+        default: return hipErrorInvalidConfiguration;
+    }
+    return hipGetLastError();
+}
+
 // Q8_0 ring kernel: work unit 8 in GemvPlan::cpl (2 lanes per block, 16 int8
 // each); needs a 4-byte aligned weight base and an even block count.
 constexpr int kQ80RingUnit = 8;
@@ -1173,6 +1231,19 @@ hipError_t launch_gemv(int qtype, const uint8_t* w, const float* x, float* y, in
         return launch_q6k_ring(p.unroll, p.rows_per_wg, p.waves, p.grid, w, x, y, n, (int)nb, stream);
     }
     if (qtype == kTypeQ6K && p.cpl == kQ6KRingUnit) return hipErrorInvalidValue;   // layout not eligible
+    if (qtype == kTypeQ5K && nb * 8 <= 1024 &&
+        (p.cpl == kQ5KRingUnit || (p.cpl <= 0 && (p.rows_per_wg <= 0 || q4k_rows_ok(p.rows_per_wg))))) {
+        p.cpl = kQ5KRingUnit;
+        p.waves = (int)((nb * 8 + 63) / 64);
+        if (p.rows_per_wg <= 0) p.rows_per_wg = pick_rows_q4k(n, p.waves);
+        if (!q4k_rows_ok(p.rows_per_wg)) return hipErrorInvalidConfiguration;
+        p.unroll = p.rows_per_wg < 3 ? p.rows_per_wg : 3;
+        p.grid = (n + p.rows_per_wg - 1) / p.rows_per_wg;
+        if (p.grid > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
+        if (plan) *plan = p;
+        return launch_q5k_ring(p.rows_per_wg, p.waves, p.grid, w, x, y, n, (int)nb, stream);
+    }
+    if (qtype == kTypeQ5K && p.cpl == kQ5KRingUnit) return hipErrorInvalidValue;   // row too long
     if (qtype == kTypeQ10 && (p.cpl == kQ10MxUnit || (p.cpl <= 0 && gemv_q10_mx_default(w, n, k)))) {
         p.cpl = kQ10MxUnit;
         if (!gemv_q10_mx_ok(w, k)) return hipErrorInvalidValue;   // layout not eligible

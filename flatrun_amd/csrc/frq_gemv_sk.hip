@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) gemv_q4_k_sk_kernel(const uint8_t* __rest
     const uint8_t* wb = w + (int64_t)blk * kQ4KBytes;
     const int qoff = 16 + 32 * g + 16 * hh;
 
-    auto load = [&](Q4KRow<CPL>(&t)[U], int64_t rfirst) {
+    auto load = [&](KRow<CPL>(&t)[U], int64_t rfirst) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (active && rfirst + u < r1) {
@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(256) gemv_q4_k_sk_kernel(const uint8_t* __rest
     };
 
     // first batch in flight before x is fetched
-    Q4KRow<CPL> A[U], B[U];
+    KRow<CPL> A[U], B[U];
     load(A, r0);
 
     float xl[NE], xh[NE];
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(256) gemv_q4_k_sk_kernel(const uint8_t* __rest
         }
     }
 
-    auto compute = [&](const Q4KRow<CPL>(&t)[U], int64_t rfirst) {
+    auto compute = [&](const KRow<CPL>(&t)[U], int64_t rfirst) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             uint32_t sc0, m0, sc1, m1;
