@@ -456,7 +456,8 @@ int gemv_batched_group(int count, const int* qtypes, const uint8_t* const* w, co
                         if (int rc = pair_rows(qtypes[j], w[j], x, y[j], n[j], k, batch, ldy[j], s, scratch, p[j].bytes,
                                                ready))
                             return rc;
-                        ready = done[j] = true;
+                        done[j] = true;
+                        ready = !p[j].few;
                     }
             }
     }

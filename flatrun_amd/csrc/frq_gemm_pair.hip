@@ -332,6 +332,63 @@ __device__ __forceinline__ T row_reduce(T v, T* lds, int tr, Op op) {
     return t;
 }
 
+// Eight scaled values as pairs; body collects sum |x| capped at 2^-10 of the
+// largest.
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo, float& body) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const f16x2 hv = {(_Float16)v[2 * p], (_Float16)v[2 * p + 1]};
+        const f16x2 lv = {(_Float16)(v[2 * p] - (float)hv[0]), (_Float16)(v[2 * p + 1] - (float)hv[1])};
+        hi[p] = as_u32(hv);
+        lo[p] = as_u32(lv);
+        body += fminf(fabsf(v[2 * p]), 16.0f) + fminf(fabsf(v[2 * p + 1]), 16.0f);
+    }
+}
+// What the pairs of four scaled values lose beyond 2^-23 of each: elements below
+// 2^-16 of the largest only, and at most 2^-25 each, so rows of N elements with
+// N 2^-25 <= 2^-24 body pass without it.
+__device__ __forceinline__ float lost4(const f32x4 v) {
+    float e = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float r = v[i] - (float)(_Float16)v[i];
+        e += fmaxf(fabsf(r - (float)(_Float16)r) - 0x1p-23f * fabsf(v[i]), 0.0f);
+    }
+    return e;
+}
+
+// The largest |x| of v and `big`, as bits (a NaN above inf).
+__device__ __forceinline__ uint32_t largest(uint32_t big, const f32x4 v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) big = max(big, __float_as_uint(v[e]) & 0x7FFFFFFFu);
+    return big;
+}
+
+// The power of two that takes values of at most `big` (bits) to [2^14, 2^15):
+// false where 2^-100 <= big < 2^101 does not hold (exponent fields 27 .. 227).
+__device__ __forceinline__ bool row_scale(uint32_t big, int& e) {
+    const int ef = (int)(big >> 23);
+    const bool ok = big == 0 || (ef >= 27 && ef <= 227);
+    e = big == 0 || !ok ? 0 : 127 + 14 - ef;
+    return ok;
+}
+
+// The two A fragments' parts of a row's sums s0, s1 over two neighbouring
+// sub-blocks: x1 x2 x1 x2 and x3 x1 0 0 (see K4Stage).
+__device__ __forceinline__ void sum_pieces(float s0, float s1, u32x4& f0, u32x4& f1) {
+    const uint32_t p1 = bf16_pair(s0, s1);
+    const float r0 = s0 - bf16_lo(p1), r1 = s1 - bf16_hi(p1);
+    const uint32_t p2 = bf16_pair(r0, r1), p3 = bf16_pair(r0 - bf16_lo(p2), r1 - bf16_hi(p2));
+    f0 = u32x4{p1, p2, p1, p2};
+    f1 = u32x4{p3, p1, 0u, 0u};
+}
+__device__ __forceinline__ float sum8(float v) {       // over eight neighbouring lanes
+    v += dpp_mov<0xB1>(v);
+    v += dpp_mov<0x4E>(v);
+    v += dpp_mov<0x141>(v);
+    return v;
+}
+
 // The pairs of every row of x, the sub-block sums' pieces (Q4_K / Q5_K) and
 // the factor that undoes the row's scale (0 = row computed weight by weight).
 // RW rows per workgroup, TPR threads each, NC pieces of eight elements per
@@ -358,11 +415,6 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
         a = in && ra < K ? *reinterpret_cast<const f32x4*>(xr + ra) : f32x4{};
         b = in && rb < K ? *reinterpret_cast<const f32x4*>(xr + rb) : f32x4{};
     };
-    auto largest = [](uint32_t big, const f32x4 v) __attribute__((always_inline)) {   // |x| as bits, NaN above inf
-#pragma unroll
-        for (int e = 0; e < 4; ++e) big = max(big, __float_as_uint(v[e]) & 0x7FFFFFFFu);
-        return big;
-    };
     f32x4 xa[NC ? NC : 1], xb[NC ? NC : 1];
     uint32_t big = 0;
     if constexpr (NC > 0) {
@@ -375,13 +427,10 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
     }
     big = row_reduce<TPR>(big, reinterpret_cast<uint32_t*>(red[rr]), tr,
                           [](uint32_t a, uint32_t b) { return a > b ? a : b; });
-    // exponent fields 27 .. 227: 2^-100 <= max |x| < 2^101
-    const int ef = (int)(big >> 23);
-    bool ok = big == 0 || (ef >= 27 && ef <= 227);
-    const int e = big == 0 || !ok ? 0 : 127 + 14 - ef;   // max |x| 2^e in [2^14, 2^15)
+    int e;
+    bool ok = row_scale(big, e);                         // max |x| 2^e in [2^14, 2^15)
     const float scale = ok ? ldexpf(1.0f, e) : 0.0f;
-    const float cap = 16.0f;                             // 2^-10 of the largest
-    float err = 0.0f, body = 0.0f;
+    float body = 0.0f;
     const int64_t mt = m >> 5;
     const int nst = units * 4;
     auto split = [&](int c, f32x4 a, f32x4 b) __attribute__((always_inline)) {
@@ -392,18 +441,7 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
         float v[8];
         Order<QT>::order(a, b, v);
         u32x4 hi, lo;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const f16x2 hv = {(_Float16)v[2 * p], (_Float16)v[2 * p + 1]};
-            const float r0 = v[2 * p] - (float)hv[0], r1 = v[2 * p + 1] - (float)hv[1];
-            const f16x2 lv = {(_Float16)r0, (_Float16)r1};
-            hi[p] = as_u32(hv);
-            lo[p] = as_u32(lv);
-            // error beyond 2^-23 of the element (only elements below 2^-16 of the largest have any)
-            err += fmaxf(fabsf(r0 - (float)lv[0]) - 0x1p-23f * fabsf(v[2 * p]), 0.0f) +
-                   fmaxf(fabsf(r1 - (float)lv[1]) - 0x1p-23f * fabsf(v[2 * p + 1]), 0.0f);
-            body += fminf(fabsf(v[2 * p]), cap) + fminf(fabsf(v[2 * p + 1]), cap);
-        }
+        split8(v, hi, lo, body);
         const bool out = live && c < chunks;
         if (out) {
             uint8_t* fp = xf + ((mt * nst + st) * 8 + 2 * i) * 1024 + ((m & 31) + 32 * h) * 16;
@@ -411,20 +449,13 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
             *reinterpret_cast<u32x4*>(fp + 1024) = lo;
         }
         if constexpr (kK4<QT>) {                         // a, b: four elements of each sub-block, eight lanes
-            float s0 = (a[0] + a[1]) + (a[2] + a[3]), s1 = (b[0] + b[1]) + (b[2] + b[3]);
-            s0 += dpp_mov<0xB1>(s0);
-            s1 += dpp_mov<0xB1>(s1);
-            s0 += dpp_mov<0x4E>(s0);
-            s1 += dpp_mov<0x4E>(s1);
-            s0 += dpp_mov<0x141>(s0);
-            s1 += dpp_mov<0x141>(s1);
+            const float s0 = sum8((a[0] + a[1]) + (a[2] + a[3])), s1 = sum8((b[0] + b[1]) + (b[2] + b[3]));
             if ((c & 7) == 0 && out) {
-                const uint32_t p1 = bf16_pair(s0, s1);
-                const float r0 = s0 - bf16_lo(p1), r1 = s1 - bf16_hi(p1);
-                const uint32_t p2 = bf16_pair(r0, r1), p3 = bf16_pair(r0 - bf16_lo(p2), r1 - bf16_hi(p2));
+                u32x4 f0, f1;
+                sum_pieces(s0, s1, f0, f1);
                 uint8_t* sp = xsum + (mt * nst + st) * 1024 + (m & 31) * 16;
-                *reinterpret_cast<u32x4*>(sp) = u32x4{p1, p2, p1, p2};
-                *reinterpret_cast<u32x4*>(sp + 512) = u32x4{p3, p1, 0u, 0u};
+                *reinterpret_cast<u32x4*>(sp) = f0;
+                *reinterpret_cast<u32x4*>(sp + 512) = f1;
             }
         }
     };
@@ -439,9 +470,19 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
         }
     }
     const auto add = [](float a, float b) { return a + b; };
-    err = row_reduce<TPR>(err, red[rr], tr, add);
     body = row_reduce<TPR>(body, red[rr], tr, add);
-    ok = ok && err <= 0x1p-24f * body;
+    // (a workgroup of one row decides alike in all its threads; others always look)
+    if (RW > 1 || (float)(units * kUnit) > 2.0f * body) {
+        float err = 0.0f;
+        if constexpr (NC > 0) {
+#pragma unroll
+            for (int j = 0; j < NC; ++j) err += lost4(xa[j] * scale) + lost4(xb[j] * scale);
+        } else {
+            for (int c = tr; c < K / 4; c += TPR) err += lost4(*reinterpret_cast<const f32x4*>(xr + 4 * c) * scale);
+        }
+        err = row_reduce<TPR>(err, red[rr], tr, add);
+        ok = ok && err <= 0x1p-24f * body;
+    }
     if (tr == 0 && live) inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
 }
 
@@ -451,34 +492,47 @@ __device__ __forceinline__ u32x4 head_words(const Head<QT>& h) {   // d, dmin an
     else return u32x4{};
 }
 
+// A value of each of two lanes that share a pair of sub-blocks (ROW16: 16 lanes
+// apart, else 32), to both: [0] from the lane of the even one, [1] of the odd one.
+template <bool ROW16>
+__device__ __forceinline__ u32x2 both(uint32_t v) {
+    if constexpr (ROW16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return u32x2{r[0], r[1]};
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return u32x2{r[0], r[1]};
+    }
+}
+
 // What Q4_K / Q5_K add to a stage: its two sub-blocks' code constants and the
 // B fragment of (R - dmin m / d) 2^-14, to be multiplied by sum(x) (the pieces
-// of split_kernel's fragment: w1 x1, w1 x2, w2 x1, w2 x2 | w1 x3, w3 x1).
+// of split_kernel's fragment: w1 x1, w1 x2, w2 x1, w2 x2 | w1 x3, w3 x1). Each of
+// the two lanes of a row that share the sub-blocks works out one of them (sc,
+// mn; odd: which).
 struct K4Stage {
     f16x2 mul[2], off[2];
     u32x4 uf;
-    template <int QT, int T>
-    __device__ __forceinline__ void set(const u32x4 hd, int h) {
+    template <int QT, bool ROW16>
+    __device__ __forceinline__ void set(const u32x4 hd, uint32_t sc, uint32_t mn, int odd) {
         const float d = f16_bits_to_f32(hd[0]), dm = f16_bits_to_f32(hd[0] >> 16);
         // d = 0: the codes are 0 and the whole weight, -dmin m, is the second term
         const bool z = d == 0.0f;
         const float rd = z ? 1.0f : __builtin_amdgcn_rcpf(d);
-        float u[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            uint32_t sc, mn;
-            k4_scale_min(hd[1], hd[2], hd[3], 2 * T + j, sc, mn);
-            const float s = z ? 0.0f : (float)sc, tm = dm * (float)mn;      // exact
-            // d non-finite: fmaxf drops a NaN, so R lands in range anyway
-            const float R = fminf(fmaxf(__builtin_rintf(tm * rd), 0.0f), (QT == kTypeQ4K ? 15.0f : 31.0f) * s);
-            u[j] = __builtin_fmaf(d, R, -tm) * (rd * 0x1p-14f);             // d R - tm in one rounding
-            mul[j] = pair_of(s * (j ? 64.0f : 1024.0f));
-            off[j] = pair_of(R * -0x1p-14f);
-        }
-        const uint32_t p1 = bf16_pair(u[0], u[1]);
-        const float r0 = u[0] - bf16_lo(p1), r1 = u[1] - bf16_hi(p1);
-        const uint32_t p2 = bf16_pair(r0, r1), p3 = bf16_pair(r0 - bf16_lo(p2), r1 - bf16_hi(p2));
-        uf = u32x4{p1, h ? p3 : p1, h ? 0u : p2, h ? 0u : p2};
+        const float s = z ? 0.0f : (float)sc, tm = dm * (float)mn;          // exact
+        // d non-finite: fmaxf drops a NaN, so R lands in range anyway
+        const float R = fminf(fmaxf(__builtin_rintf(tm * rd), 0.0f), (QT == kTypeQ4K ? 15.0f : 31.0f) * s);
+        const float u = __builtin_fmaf(d, R, -tm) * (rd * 0x1p-14f);        // d R - tm in one rounding
+        const u32x2 m = both<ROW16>(as_u32(pair_of(s * (odd ? 64.0f : 1024.0f))));
+        const u32x2 o = both<ROW16>(as_u32(pair_of(R * -0x1p-14f)));
+        mul[0] = as_f16x2(m[0]), mul[1] = as_f16x2(m[1]);
+        off[0] = as_f16x2(o[0]), off[1] = as_f16x2(o[1]);
+        const uint32_t u1 = bf16_pair(u, 0.0f);
+        const float r1 = u - bf16_lo(u1);
+        const uint32_t u2 = bf16_pair(r1, 0.0f);
+        const u32x2 p = both<ROW16>(u1 | (u2 << 16)), p3 = both<ROW16>(bf16_pair(r1 - bf16_lo(u2), 0.0f));
+        const uint32_t w1 = __builtin_amdgcn_perm(p[1], p[0], 0x05040100u), w2 = __builtin_amdgcn_perm(p[1], p[0], 0x07060302u);
+        uf = u32x4{w1, odd ? p3[0] | (p3[1] << 16) : w1, odd ? 0u : w2, odd ? 0u : w2};
     }
     __device__ static __forceinline__ float scale(const u32x4 hd) {
         const float d = f16_bits_to_f32(hd[0]);
@@ -603,6 +657,7 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
         for (int nt = 0; nt < NT; ++nt) bb[nt].template load<decltype(pc)::value>(up, wrow[nt], h, left);
     };
 
+    const uint32_t sh8 = 8u * (uint32_t)h;
     // a stage's codes of one 32-row tile of W
     struct Codes {
         f16x8 s[GS];
@@ -614,7 +669,15 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
         Codes c;
         K4Stage ks;
         if constexpr (kK4<QT>) {
-            ks.template set<QT, T>(head_words(hh), h);
+            // (sc, m) of sub-block 2T + h (get_scale_min_k4, gguf.py:135-163)
+            const u32x4 hw = head_words(hh);
+            const uint32_t s0 = hw[1] >> sh8, s1 = hw[2] >> sh8, s2 = hw[3] >> sh8;
+            constexpr int B = 16 * (T & 1);
+            if constexpr (T < 2)
+                ks.template set<QT, false>(hw, (s0 >> B) & 63u, (s1 >> B) & 63u, h);
+            else
+                ks.template set<QT, false>(hw, ((s2 >> B) & 15u) | (((s0 >> (B + 6)) & 3u) << 4),
+                                           ((s2 >> (B + 4)) & 15u) | (((s1 >> (B + 6)) & 3u) << 4), h);
             c.u = __builtin_bit_cast(bf16x8, ks.uf);
         }
         static_for<0, GS>([&](auto ic) {
@@ -876,14 +939,26 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
 }
 
 // S > 1: y = inv * (the planes added in split order, in fp64: free here, and
-// one rounding instead of S). Then, S = 1 too, the rows
-// that the pairs do not carry (inv = 0), weight by weight in fp64, a wave per
-// output over the whole grid.
+// one rounding instead of S). Then, S = 1 too, the rows that the pairs do not
+// carry, weight by weight in fp64, a wave per output over the whole grid: those
+// with inv = 0, or, where every split judged its part of x itself (few_kernel;
+// inv null, the planes in units of y, at most 32 rows), with a flag of any split.
 template <int QT>
 __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ part, float* __restrict__ y, int S,
                                                      int M, int N, int64_t ldy, const float* __restrict__ inv,
-                                                     const uint8_t* __restrict__ w, const float* __restrict__ x,
-                                                     int K) {
+                                                     const uint32_t* __restrict__ flags, const uint8_t* __restrict__ w,
+                                                     const float* __restrict__ x, int K) {
+    const int lane = threadIdx.x & 63, wv = (int)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int)gridDim.x * 4;
+    uint32_t bad = 0;                                    // rows < 32, of any split
+    if (!inv) {
+        for (int i = lane; i < 32 * S; i += 64)
+            if (flags[i] && (i & 31) < M) bad |= 1u << (i & 31);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) bad |= (uint32_t)__shfl_xor((int)bad, o, 64);
+    }
+    auto factor = [&](int m) __attribute__((always_inline)) {
+        return inv ? inv[m] : (bad >> m) & 1u ? 0.0f : 1.0f;
+    };
     const int64_t plane = (int64_t)M * N;
     if (S > 1) {
         if (((N | ldy) & 3) == 0 && !(reinterpret_cast<uintptr_t>(y) & 15)) {
@@ -901,7 +976,7 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
                     for (int q = 0; q < 8; ++q)
                         if (q0 + q < S) v += __builtin_convertvector(t[q], f64x4);
                 }
-                const float f = inv[m];
+                const float f = factor(m);
                 if (f != 0.0f)
                     *reinterpret_cast<f32x4*>(y + (int64_t)m * ldy + n) = __builtin_convertvector(v * (double)f, f32x4);
             }
@@ -910,14 +985,13 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
             for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < plane; e += step) {
                 const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
                 const double v = sum_planes<double>([&](int q) { return (double)part[e + q * plane]; }, S);
-                const float f = inv[m];
+                const float f = factor(m);
                 if (f != 0.0f) y[(int64_t)m * ldy + n] = (float)(v * f);
             }
         }
     }
-    const int lane = threadIdx.x & 63, wv = (int)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int)gridDim.x * 4;
-    for (int m0 = 0; m0 < M; m0 += 64) {                // every wave scans all rows of inv
-        uint64_t hit = __ballot(m0 + lane < M && inv[m0 + lane < M ? m0 + lane : 0] == 0.0f);
+    for (int m0 = 0; m0 < M; m0 += 64) {                // every wave scans all rows
+        uint64_t hit = inv ? __ballot(m0 + lane < M && inv[m0 + lane < M ? m0 + lane : 0] == 0.0f) : bad;
         while (hit) {
             const int m = m0 + __builtin_ctzll(hit);
             hit &= hit - 1;
@@ -932,6 +1006,287 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
             }
         }
     }
+}
+
+// ------------------------------------------------------------ up to 32 rows
+// The same arithmetic for few rows of x, where launches and latency count: one
+// launch splits x and multiplies. A workgroup owns 256 rows of W and a range of
+// at most kFewUnits / MT units of k; its 16 waves are eight of 32 rows of W by two
+// halves (128 elements) of every unit, on v_mfma_f32_16x16x32_f16 (MT tiles of
+// 16 rows of x: half the matrix work and LDS of a padded 32-row tile). All loads
+// of x and the first of W go out at once; wave r splits row r (and r + 16) of the
+// range of x into LDS, scaled by the range's own largest |x|; one barrier; then
+// every wave runs through its halves without another. Lane (c, q) of a tile holds row c of W and the
+// 16 qs bytes (a dword of Q1_0) of k group q: every 64-byte part of a row in one
+// load. The two halves are added through LDS, the splits of k by finish_kernel.
+// 16 waves (four per SIMD) hide each other's chains of decode and products,
+// which bound the 32-row tile of gemm_pair_kernel at two waves per SIMD. Measured
+// (whole call, us, three launches with that tile / here): 16 rows of Q4_K
+// 4096 x 14336 30.3 / 23.8 (1.4 TB/s of W; bound by vector work, about five
+// instructions per weight), 18944 x 3584 30 / 25, Q1_0 8192 x 4096 21 / 17.
+constexpr int kFewUnits = 8;
+constexpr int kFewAside = 128, kFewHead = kFewAside + 2048;   // LDS: factors of the rows, a place for unused writes, x
+
+template <int QT>
+struct FewRaw;                                           // one tile's fields of half a unit
+template <>
+struct FewRaw<kTypeQ4K> {
+    u32x4 hd, v;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int kh, int q, int) {
+        hd = ld<u32x4>(unit, row);
+        v = ld<u32x4>(unit + 16 + 64 * kh, row + 16 * q);
+    }
+};
+template <>
+struct FewRaw<kTypeQ5K> {
+    u32x4 hd, qh, v;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int kh, int q, int) {
+        hd = ld<u32x4>(unit, row);
+        qh = ld<u32x4>(unit + 16, row + 16 * (q & 1));
+        v = ld<u32x4>(unit + 48 + 64 * kh, row + 16 * q);
+    }
+};
+template <>
+struct FewRaw<kTypeQ10> {
+    uint32_t d, v;
+    __device__ __forceinline__ void load(gptr unit, uint32_t row, int kh, int q, int left) {
+        const gptr bp = unit + (kh < left ? kh : left - 1) * kQ10Bytes;
+        const uint32_t dv = ld<uint16_t>(bp, row);
+        d = kh < left ? dv : 0u;
+        v = ld<u32_a2>(bp + 2, row + 4 * q);
+    }
+};
+
+template <int QT, int MT>
+__global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                   float* __restrict__ y, int M, int N, int K, int units, int64_t ldy,
+                                                   int S, float* __restrict__ part, uint32_t* __restrict__ flags) {
+    constexpr int kHalf = 8192 + (kK4<QT> ? 1024 : 0);   // pairs and sums of 16 rows x 128 k
+    constexpr int kUnitBytes = (int)weight_row_bytes<QT>(kUnit);
+    constexpr int DEPTH = QT == kTypeQ5K ? 2 : 3;        // units of W in flight (registers)
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave & 7, kh = wave >> 3, c = lane & 15, q = lane >> 4;
+    const int G = (int)gridDim.x, xcd = (int)blockIdx.x & 7, gq = G >> 3, gr = G & 7;
+    const int id = (xcd < gr ? xcd * (gq + 1) : gr * (gq + 1) + (xcd - gr) * gq) + ((int)blockIdx.x >> 3);
+    const int ntiles = (N + 255) / 256, n0 = id % ntiles * 256, split = id / ntiles;
+    const int u0 = (int)((int64_t)split * units / S), u1 = (int)((int64_t)(split + 1) * units / S), U = u1 - u0;
+    float* inv = reinterpret_cast<float*>(lds);          // of the 16 MT rows
+    uint8_t* xl = lds + kFewHead;
+
+    const uint8_t* wtile = w + (int64_t)n0 * weight_row_bytes<QT>(K);
+    uint32_t wrow[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        const int n = 32 * wn + 16 * nt + c;
+        wrow[nt] = (uint32_t)(n0 + n < N ? n : N - 1 - n0) * (uint32_t)weight_row_bytes<QT>(K);
+    }
+    FewRaw<QT> raw[DEPTH][2];
+    auto load_w = [&](FewRaw<QT> (&r)[2], int u) __attribute__((always_inline)) {
+        const int uu = u < u1 ? u : u1 - 1;
+        const gptr up = scalar_base(wtile + (int64_t)uu * kUnitBytes);
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) r[nt].load(up, wrow[nt], kh, q, K / kQ10Elems - 2 * uu);
+    };
+    // x first (memory returns in order): wave r's rows r and (MT = 2) r + 16, lane
+    // l's pieces l, l + 64, ...; past the range or the row its last elements,
+    // made zeros below
+    constexpr int NC = kFewUnits / MT / 2;               // 32 pieces of eight per unit
+    const int kleft = K - u0 * kUnit, lim = (U * kUnit < kleft ? U * kUnit : kleft) - 4;
+    f32x4 xva[MT][NC], xvb[MT][NC];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = 16 * mt + wave < M ? 16 * mt + wave : M - 1;
+        const gptr xr = scalar_base(reinterpret_cast<const uint8_t*>(x + (int64_t)m * K + (int64_t)u0 * kUnit));
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int p = lane + 64 * j;
+            int ra, rb;
+            Order<QT>::runs(p >> 3, (p >> 1) & 3, p & 1, ra, rb);
+            xva[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(ra < lim ? ra : lim));
+            xvb[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(rb < lim ? rb : lim));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, DEPTH>([&](auto jc) { load_w(raw[decltype(jc)::value], u0 + decltype(jc)::value); });
+    __builtin_amdgcn_sched_barrier(0);
+
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = 16 * mt + wave;
+        if (m < M) {                                     // wave-uniform
+            f32x4 (&xa)[NC] = xva[mt], (&xb)[NC] = xvb[mt];
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int p = lane + 64 * j;
+                int ra, rb;
+                Order<QT>::runs(p >> 3, (p >> 1) & 3, p & 1, ra, rb);
+                if (ra > lim) xa[j] = f32x4{};
+                if (rb > lim) xb[j] = f32x4{};
+            }
+            uint32_t big = 0;
+#pragma unroll
+            for (int j = 0; j < NC; ++j) big = largest(largest(big, xa[j]), xb[j]);
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) big = max(big, (uint32_t)__shfl_xor((int)big, o, 64));
+            __builtin_amdgcn_sched_barrier(0);
+            int e;
+            bool ok = row_scale(big, e);
+            const float scale = ok ? ldexpf(1.0f, e) : 0.0f;
+            float body = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                if (2 * j >= U) break;                   // uniform; an odd last unit's pair writes zeros beyond it
+                const int p = lane + 64 * j, st = p >> 3, i = (p >> 1) & 3, h = p & 1, qq = (st & 1) * 2 + h;
+                f32x4 a = xa[j], b = xb[j];
+                if (!ok) a = b = f32x4{};                // inf * 0 would be NaN
+                a *= scale;
+                b *= scale;
+                float v[8];
+                Order<QT>::order(a, b, v);
+                u32x4 hi, lo;
+                split8(v, hi, lo, body);
+                uint8_t* half = xl + (size_t)((st >> 1) * MT + mt) * kHalf;
+                uint8_t* fp = half + 2 * i * 1024 + (wave + 16 * qq) * 16;
+                *reinterpret_cast<u32x4*>(fp) = hi;
+                *reinterpret_cast<u32x4*>(fp + 1024) = lo;
+                if constexpr (kK4<QT>) {                 // one lane of eight writes the sums, the others aside
+                    u32x4 f0, f1;
+                    sum_pieces(sum8((a[0] + a[1]) + (a[2] + a[3])), sum8((b[0] + b[1]) + (b[2] + b[3])), f0, f1);
+                    uint8_t* sp = (p & 7) == 0 ? half + 8192 + (wave + 16 * qq) * 16 : lds + kFewAside + lane * 32;
+                    *reinterpret_cast<u32x4*>(sp) = f0;
+                    *reinterpret_cast<u32x4*>(sp + ((p & 7) == 0 ? 256 : 16)) = f1;
+                }
+                __builtin_amdgcn_sched_barrier(0);       // one piece at a time: registers
+            }
+            body = wave_sum(body);
+            if ((float)(U * kUnit) > 2.0f * body) {      // wave-uniform
+                float err = 0.0f;
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+                    if (2 * j < U) err += lost4(xa[j] * scale) + lost4(xb[j] * scale);
+                ok = ok && wave_sum(err) <= 0x1p-24f * body;
+            }
+            if (lane == 0) {
+                inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
+                if (n0 == 0) flags[32 * split + m] = ok ? 0u : 1u;
+            }
+        }
+    }
+    __syncthreads();
+
+    f32x4 acc[MT][2] = {};
+    const PairDecode dec(4 * kh + q);                    // this lane's sub-block
+    const int qs = 2 * (2 * kh + (q >> 1));              // the fifth bits of its pair
+    auto compute = [&](const FewRaw<QT> (&r)[2], int u) __attribute__((always_inline)) {
+        const uint8_t* xb = xl + (size_t)(2 * (u - u0) + kh) * MT * kHalf + lane * 16;
+        f16x8 b[2][4];
+        bf16x8 bu[2];
+        float sc[2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            if constexpr (kK4<QT>) {
+                uint32_t s, mn;
+                dec(r[nt].hd[1], r[nt].hd[2], r[nt].hd[3], s, mn);
+                K4Stage ks;
+                ks.template set<QT, true>(r[nt].hd, s, mn, q & 1);
+                bu[nt] = __builtin_bit_cast(bf16x8, ks.uf);
+                sc[nt] = K4Stage::scale(r[nt].hd);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t v = r[nt].v[i], v8 = v >> 8;
+                    u32x4 f = {v & 0x000F000Fu, v & 0x00F000F0u, v8 & 0x000F000Fu, v8 & 0x00F000F0u};
+                    if constexpr (QT == kTypeQ5K) {
+                        const uint32_t g = r[nt].qh[i] >> qs;
+                        f |= u32x4{(g << 4) & 0x00100010u, (g << 7) & 0x01000100u, (g >> 4) & 0x00100010u,
+                                   (g >> 1) & 0x01000100u};
+                    }
+                    f[0] = fma2(f[0], ks.mul[0], ks.off[0]);
+                    f[1] = fma2(f[1], ks.mul[1], ks.off[1]);
+                    f[2] = fma2(f[2], ks.mul[0], ks.off[0]);
+                    f[3] = fma2(f[3], ks.mul[1], ks.off[1]);
+                    b[nt][i] = __builtin_bit_cast(f16x8, f);
+                }
+            } else {
+                sc[nt] = -f16_bits_to_f32(r[nt].d);      // codes negated, as in Body<kTypeQ10>
+                static_for<0, 4>([&](auto ic) {
+                    constexpr int I = decltype(ic)::value;
+                    u32x4 f;
+                    static_for<0, 4>([&](auto jc) {
+                        constexpr int j = decltype(jc)::value;
+                        f[j] = ((r[nt].v << (15 - 4 * I - j)) & 0x80008000u) | 0x3C003C00u;
+                    });
+                    b[nt][I] = __builtin_bit_cast(f16x8, f);
+                });
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const uint8_t* xm = xb + mt * kHalf;
+            f32x4 t[2] = {};
+            if constexpr (kK4<QT>) {
+                const bf16x8 a = *reinterpret_cast<const bf16x8*>(xm + 8192);
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bu[nt], t[nt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int pc = 1; pc >= 0; --pc)              // lo, then hi
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const f16x8 a = *reinterpret_cast<const f16x8*>(xm + (2 * i + pc) * 1024);
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt)
+                        t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[nt][i], t[nt], 0, 0, 0);
+                }
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) acc[mt][nt][r4] = __builtin_fmaf(sc[nt], t[nt][r4], acc[mt][nt][r4]);
+        }
+    };
+    int u = u0;
+    for (; u + DEPTH <= u1; u += DEPTH)
+        static_for<0, DEPTH>([&](auto jc) {
+            constexpr int J = decltype(jc)::value;
+            compute(raw[J], u + J);
+            load_w(raw[J], u + J + DEPTH);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    static_for<0, DEPTH - 1>([&](auto jc) {
+        constexpr int J = decltype(jc)::value;
+        if (u + J < u1) compute(raw[J], u + J);
+    });
+
+    // the second half's sums through LDS (x is done with), then out
+    float f[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f[mt][r] = inv[16 * mt + 4 * q + r];
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(xl) + wn * MT * 2 * 64 + lane;
+    if (kh == 1) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) red[(2 * mt + nt) * 64] = acc[mt][nt];
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    float* out = S == 1 ? y : part + (int64_t)split * M * N;
+    const int64_t ldo = S == 1 ? ldy : N;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const f32x4 v = acc[mt][nt] + red[(2 * mt + nt) * 64];
+            const int n = n0 + 32 * wn + 16 * nt + c;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = 16 * mt + 4 * q + r;
+                if (m < M && n < N) out[(int64_t)m * ldo + n] = v[r] * f[mt][r];
+            }
+        }
 }
 
 template <int QT, int WM, int WN, int MT, int NT, int DEPTH>
@@ -968,6 +1323,28 @@ template <int QT>
 void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int64_t ldy, hipStream_t s,
               uint8_t* scratch, bool x_ready) {
     float* inv = reinterpret_cast<float*>(scratch);
+    if constexpr (QT != kTypeQ6K) {
+        if (p.few) {
+            uint32_t* flags = reinterpret_cast<uint32_t*>(scratch);
+            float* part = reinterpret_cast<float*>(scratch + p.part_off);
+            const unsigned grid = (unsigned)((p.n + 255) / 256 * p.splits);
+            const int mt = p.m <= 16 ? 1 : 2;
+            const int64_t u = (p.units + p.splits - 1) / p.splits;
+            const unsigned bytes = (unsigned)((u + 1) / 2 * 4 * mt * (8192 + (kK4<QT> ? 1024 : 0)));
+            const unsigned red = (unsigned)(8 * mt * 2 * 64 * 16);
+            const unsigned ldsb = kFewHead + (bytes > red ? bytes : red);
+            if (mt == 1)
+                few_kernel<QT, 1><<<dim3(grid), dim3(1024), ldsb, s>>>(w, x, y, (int)p.m, (int)p.n, (int)p.k,
+                                                                       (int)p.units, ldy, p.splits, part, flags);
+            else
+                few_kernel<QT, 2><<<dim3(grid), dim3(1024), ldsb, s>>>(w, x, y, (int)p.m, (int)p.n, (int)p.k,
+                                                                       (int)p.units, ldy, p.splits, part, flags);
+            const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
+            finish_kernel<QT><<<dim3((unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work)), dim3(256), 0, s>>>(
+                part, y, p.splits, (int)p.m, (int)p.n, ldy, nullptr, flags, w, x, (int)p.k);
+            return;
+        }
+    }
     if (!x_ready) split_go<QT>(p, x, s, scratch + p.x_off, scratch + p.sum_off, inv);
     if (p.bm == 32)
         pair_go<QT, 1, 8, 1, 1, 2>(p, w, y, ldy, s, scratch);
@@ -978,7 +1355,7 @@ void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int
     const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
     const unsigned fin = (unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work);
     finish_kernel<QT><<<dim3(fin), dim3(256), 0, s>>>(reinterpret_cast<const float*>(scratch + p.part_off), y,
-                                                      p.splits, (int)p.m, (int)p.n, ldy, inv, w, x, (int)p.k);
+                                                      p.splits, (int)p.m, (int)p.n, ldy, inv, nullptr, w, x, (int)p.k);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -992,6 +1369,7 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
     if (kq == 0 || m <= 0 || n <= 0 || k <= 0 || k % kq || m > kPairRows || n > 0x3FFFFFFF || k > (1 << 22))
         return false;
     const bool k4 = qtype == kTypeQ4K || qtype == kTypeQ5K;
+    p->few = false;
     p->m = m;
     p->n = n;
     p->k = k;
@@ -1031,6 +1409,34 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
                 p->x_off = x_off;
                 p->part_off = part_off;
             }
+        }
+    }
+    if (m <= 32 && qtype != kTypeQ6K) {
+        // few_kernel: one round of 256 workgroups where its LDS lets it, every
+        // split at least two units. Measured (us, both launches): 7 + 6 per
+        // round + 2.2 a unit (3.0 past 16 rows), against three launches and
+        // 6 more than the model above: 18944 x 3584, 16 rows 25 / 30, 32 rows
+        // (two rounds of it) 50 / 32; 4096 x 14336, 16 / 32 rows 26 / 32 against
+        // 35 / 38; 1024 x 1024 14 / 15.
+        const int64_t most = kFewUnits / (m <= 16 ? 1 : 2), need = (p->units + most - 1) / most;
+        int64_t fs = 256 / ntiles < 64 ? 256 / ntiles : 64;
+        if (fs > (p->units + 1) / 2) fs = (p->units + 1) / 2;
+        if (fs < need) fs = need;
+        if (fs < 1) fs = 1;
+        const int64_t share = (p->units + fs - 1) / fs;
+        fs = (p->units + share - 1) / share;             // as few splits as give that share
+        const double few_us = 7.0 + (double)((ntiles * fs + 255) / 256) * (6.0 + (double)share * (m <= 16 ? 2.2 : 3.0));
+        const size_t part_off = align256((size_t)fs * 32 * 4);
+        const size_t bytes = part_off + (fs > 1 ? (size_t)fs * (size_t)m * (size_t)n * 4 : 0);
+        if (bytes <= cap && fs * ntiles <= 0x7FFFFFFF && (!found || few_us < best + 6.0)) {
+            p->few = true;
+            p->splits = (int)fs;
+            p->bm = 32;
+            p->layout = 0;                               // nothing that another launch could use
+            p->sum_off = p->x_off = 0;
+            p->part_off = part_off;
+            p->bytes = bytes;
+            return true;
         }
     }
     if (!found) return false;

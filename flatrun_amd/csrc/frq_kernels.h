@@ -239,6 +239,7 @@ constexpr int64_t kPairRows = 1024;
 struct PairPlan {
     int64_t m = 0, n = 0, k = 0, units = 0;
     int bm = 0, bn = 0, splits = 1, layout = 0;
+    bool few = false;       // up to 32 rows: the one-launch kernel, which shares nothing
     size_t sum_off = 0, x_off = 0, part_off = 0, bytes = 0;
 };
 bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, PairPlan* p);

@@ -43,6 +43,8 @@ def check(q, raw, xs, n, k, y, what):
 @pytest.mark.parametrize("q,n,k,rows", [
     ("Q5_K", 1, 256, 4), ("Q5_K", 255, 512, 31), ("Q5_K", 257, 1280, 32), ("Q5_K", 289, 768, 33),
     ("Q5_K", 300, 4352, 64), ("Q5_K", 513, 256, 65), ("Q5_K", 256, 2304, 97), ("Q5_K", 33, 20992, 7),
+    ("Q5_K", 257, 1280, 16), ("Q5_K", 70, 768, 17), ("Q5_K", 2100, 2304, 15), ("Q1_0", 511, 896, 16),
+    ("Q4_K", 1500, 16384, 16), ("Q4_K", 18000, 1536, 17), ("Q4_K", 9000, 2816, 9),
     ("Q1_0", 1, 128, 4), ("Q1_0", 31, 384, 5), ("Q1_0", 257, 640, 32), ("Q1_0", 300, 4224, 63),
     ("Q1_0", 256, 2048, 130), ("Q1_0", 65, 18944, 33),
     ("Q4_K", 255, 256, 65), ("Q4_K", 257, 1280, 129), ("Q4_K", 300, 2816, 100), ("Q4_K", 64, 1024, 1030),
