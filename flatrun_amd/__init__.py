@@ -107,6 +107,30 @@ def _raw_bytes(weight) -> np.ndarray:
 
 _GIB = 1 << 30
 
+# Page-locked memory that activations and results of resident-weight calls go
+# through (larger results, or x over 1 MiB, are copied without it). A call
+# takes one buffer and gives it back; at most two are kept between calls.
+_PINNED_BYTES = 4 << 20
+_pinned_free: list = []
+
+
+def _take_pinned():
+    """A buffer no other call holds, or None where there is none to have."""
+    from . import device
+    try:
+        return _pinned_free.pop()
+    except IndexError:
+        pass
+    try:
+        return device.PinnedBuffer(_PINNED_BYTES)
+    except FrqDeviceError:
+        return None
+
+
+def _give_pinned(buf) -> None:
+    if buf is not None and len(_pinned_free) < 2:
+        _pinned_free.append(buf)
+
 
 def _cache_capacity(setting) -> int:
     """Bytes of device weight cache from a constructor argument or the
@@ -251,12 +275,10 @@ class NativeBackend:
         if seq and n:
             xb = (seq * k * 4 + 255) // 256 * 256
             with self._lock:
-                scratch = self._scratch_for(xb + seq * n * 4)
-                base = scratch.ptr
-                if x_c.size:
-                    _lib.check(_lib.lib().frq_memcpy_h2d(base, x_c.ctypes.data, x_c.nbytes))
-                device.gemv(qname, weight, base, base + xb, n, k, batch=seq, w_bytes=weight.nbytes)
-                _lib.check(_lib.lib().frq_memcpy_d2h(out.ctypes.data, base + xb, out.nbytes))
+                scratch = self._scratch_for(xb + (seq * n * 4 + 15) // 16 * 16)
+                pinned = _take_pinned()
+                device.gemv_host(qname, weight, x_c, out, n, k, seq, scratch, pinned, w_bytes=weight.nbytes)
+                _give_pinned(pinned)      # not after an error: a copy may still be pending, and freeing waits for it
         return out[0] if x_c.ndim == 1 else out
 
     def upload(self, weight) -> DeviceWeight:

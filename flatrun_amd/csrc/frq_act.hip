@@ -26,7 +26,21 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const float* __restrict__
     }
 }
 
+__global__ void __launch_bounds__(256) copy16_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                     int64_t count) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < count) dst[i] = src[i];
+}
+
 }  // namespace
+
+hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream) {
+    const int64_t count = (int64_t)((bytes + 15) / 16);
+    if (count == 0) return hipSuccess;
+    copy16_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(static_cast<const uint4*>(src),
+                                                                       static_cast<uint4*>(dst), count);
+    return hipGetLastError();
+}
 
 hipError_t launch_silu_mul(const float* gateup, int64_t ld_in, float* out, int64_t ld_out, int64_t rows,
                            int64_t inter, hipStream_t stream) {

@@ -256,6 +256,10 @@ bool gemv_swiglu_fusable(int qtype_gate, const uint8_t* wgate, int qtype_up, con
 hipError_t launch_gemv_swiglu(const uint8_t* wgate, const uint8_t* wup, const float* x, float* gateup, float* act,
                               int64_t inter, int64_t k, hipStream_t s);
 
+// dst = src, whole 16-byte units (both rounded up to them and 16-byte aligned,
+// device memory or pinned host memory).
+hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
+
 hipError_t launch_silu_mul(const float* gateup, int64_t ld_in, float* out, int64_t ld_out, int64_t rows,
                            int64_t inter, hipStream_t stream);
 

@@ -255,6 +255,21 @@ def gemv(qtype, w, x, y, n: int, k: int, batch: int = 1, stream=None, w_bytes: i
     check(lib().frq_dev_gemv(q, _addr(w), wb, _addr(x), _addr(y), int(n), int(k), int(batch), _stream(stream)))
 
 
+def gemv_host(qtype, w, x: np.ndarray, y: np.ndarray, n: int, k: int, batch: int, scratch: DeviceBuffer,
+              pinned: PinnedBuffer | None = None, w_bytes: int | None = None) -> None:
+    """gemv with x and y in host memory (contiguous float32, (batch, k) and
+    (batch, n)), synchronous, on the null stream (frq_dev_gemv_host)."""
+    q = qtype_id(qtype)
+    wb = _nbytes(w) if w_bytes is None else int(w_bytes)
+    if x.dtype != np.float32 or y.dtype != np.float32 or not (x.flags.c_contiguous and y.flags.c_contiguous):
+        raise ValueError("gemv_host: x and y must be contiguous float32")
+    if x.size < batch * k or y.size < batch * n:
+        raise ValueError(f"gemv_host: x or y holds fewer than {batch} rows")
+    check(lib().frq_dev_gemv_host(q, _addr(w), wb, x.ctypes.data, y.ctypes.data, int(n), int(k), int(batch),
+                                  scratch.ptr, scratch.nbytes, pinned.ptr if pinned else 0,
+                                  pinned.nbytes if pinned else 0))
+
+
 GROUP_MAX = 4
 
 

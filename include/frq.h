@@ -194,6 +194,15 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
 int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
                  int64_t batch, void* stream);
 
+/* frq_dev_gemv with x and y in host memory, synchronous, on the null stream.
+ * `scratch`: device memory for both, at least 4 k batch rounded up to 256,
+ * plus 4 n batch bytes (16-byte aligned). `pinned`: page-locked host memory
+ * (frq_host_alloc; null for none) that x up to 1 MiB and y go through where
+ * they fit; larger ones are copied with hipMemcpy. One call at a time per
+ * scratch or pinned memory. Same kernels and bits as frq_dev_gemv. */
+int frq_dev_gemv_host(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
+                      int64_t batch, void* scratch, size_t scratch_bytes, void* pinned, size_t pinned_bytes);
+
 /* frq_dev_gemv that allocates nothing. No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
