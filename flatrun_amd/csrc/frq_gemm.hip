@@ -13,7 +13,8 @@
 // X is taken as given in bf16; products and sums are fp32. The result equals
 // fp64 X . bf16(W)^T to fp32 accumulation error.
 //
-// Tiling: a workgroup (8 waves, two per SIMD) owns a 256 (M) x 128 (N) tile of
+// Tiling (gemm_big_tile below has its own, for large Q4_K products): a
+// workgroup (8 waves, two per SIMD) owns a 256 (M) x 128 (N) tile of
 // Y and walks K in steps of 64 (one Q4_K group: 32 qs bytes per row). Wave
 // (wm, wn) owns the 64 x 64 sub-tile at (64 wm, 64 wn): 2 x 2 MFMA tiles of
 // 32 x 32, 64 fp32 accumulators per lane. Per K-step the X tile [256][64]
@@ -35,6 +36,8 @@
 // l is row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #include "frq_common.h"
 #include "frq_kernels.h"
+
+#include <type_traits>
 
 namespace frq {
 namespace {
@@ -490,6 +493,195 @@ __global__ void __launch_bounds__(512) gemm_bf16_group_kernel(GemmGroup g, const
     }
 }
 
+// The 256 x 256 tile (Q4_K; see big_tiles below for where it is taken): wave
+// (wm, wn) owns the 128 x 64 sub-tile at (128 wm, 64 wn), 4 x 2 MFMA tiles, so
+// that a K-step's 32 MFMAs take 24 fragment reads from LDS, where the 64 x 64
+// sub-tiles take 16 for 16 MFMAs, and W is dequantized once per 256 rows of Y
+// by 512 threads (512 x 28672 x 4096: 133 -> 117 us, 1027 TFLOP/s on 224 of
+// 256 CUs, with W cold in the caches 137 -> 128; a large library product
+// reaches 1305 TFLOP/s. The tile has one round in which nothing hides the
+// 59 MB of results at its end). X goes from memory straight to LDS. A K-step has two halves
+// of 32 k (the low and the high nibbles of a Q4_K group), each with its own
+// X and W buffers [256 rows][32 k] and one barrier. Half (t, 0) fills half
+// (t + 1, 1), half (t, 1) fills (t + 2, 0): a half is complete one barrier
+// before its first fragments are read, so these are read ahead, under the
+// MFMAs before the barrier, and nothing waits at the start of a half.
+// The 16-byte chunk c of row r is at place c ^ (r / 2 % 4): eight consecutive
+// rows' fragments then lie on different banks without padding, which copies
+// straight to LDS could not leave. The order of products and sums is that of
+// gemm_tile: the same bits.
+constexpr int kBigM = 256, kBigN = 256, kBigHalf = 256 * 64;
+__device__ __forceinline__ void gemm_big_tile(const uint8_t* __restrict__ w, const uint16_t* __restrict__ x,
+                                              float* __restrict__ y, int ldy, int M, int N, int K, int mt0, int nt0,
+                                              uint8_t* __restrict__ lds) {
+    using F = WFmt<kTypeQ4K>;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1, h = lane >> 5;
+    const int m0 = mt0 * kBigM, n0 = nt0 * kBigN;
+    const int64_t row_bytes = (int64_t)(K / F::kElems) * F::kBytes;
+    const int ksteps = K / kBK, last = ksteps - 1;
+    const int mrows = M - m0 < kBigM ? M - m0 : kBigM, nrows = N - n0 < kBigN ? N - n0 : kBigN;
+    const auto xrs = buffer_rsrc(x + (int64_t)m0 * K, (uint32_t)((int64_t)mrows * K * 2));
+    const auto wrs = buffer_rsrc(w + (int64_t)n0 * row_bytes, (uint32_t)((int64_t)nrows * row_bytes));
+    // X: copy j of a wave moves rows 32 wave + 16 j .. + 15 (rows past M: the last one)
+    uint32_t xoff[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int r = 32 * wave + 16 * j + (lane >> 2);
+        xoff[j] = (uint32_t)(((int64_t)(r < mrows ? r : mrows - 1) * K + 8 * ((lane & 3) ^ ((lane >> 3) & 3))) * 2);
+    }
+    // W: row 32 wave + lane % 32 (past N: the last one), 16 h .. + 15 of a step's 32 bytes of codes
+    const int wr = 32 * wave + (lane & 31);
+    const uint32_t wvoff = (uint32_t)((int64_t)(wr < nrows ? wr : nrows - 1) * row_bytes);
+    const uint32_t place = (uint32_t)((lane >> 1) & 3);
+    uint32_t wput[2], xget[2], wget[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        wput[j] = 4 * kBigHalf + 64 * wr + 16 * ((2 * h + j) ^ place);
+        const uint32_t at = 64 * (lane & 31) + 16 * ((2 * j + h) ^ place);
+        xget[j] = 64 * 128 * wm + at;
+        wget[j] = 4 * kBigHalf + 64 * 64 * wn + at;
+    }
+    // half H of step u (past the last one: the last, into a half nothing reads)
+    auto copy_x = [&](int u, int H, int buf) __attribute__((always_inline)) {
+        const int kb = (u < last ? u : last) * kBK + 32 * H;
+        static_for<0, 2>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                xrs, (__attribute__((address_space(3))) void*)&lds[buf * kBigHalf + 1024 * (2 * wave + j)], 16, (int)xoff[j],
+                kb * 2, 0, 0);
+        });
+    };
+    struct Raw {
+        u32x4 h, q;
+    };
+    auto load_w = [&](Raw& r, int u) __attribute__((always_inline)) {
+        const int kb = (u < last ? u : last) * kBK, sblk = (kb >> 8) * kQ4KBytes;
+        r.h = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)wvoff, sblk, 0));
+        r.q = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)(wvoff + 16 + 16 * h),
+                                                                             sblk + 32 * ((kb >> 6) & 3), 0));
+    };
+    const float u_inv = 1.0f / fp8_unit();
+    auto put_w = [&](const Raw& r, int u, auto hc, int buf) __attribute__((always_inline)) {
+        typename F::Raw f;
+        f.h = r.h;
+        const f32x4 sc = F::scales(f, (u < last ? u : last) * kBK, u_inv);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            u32x4 a, b;
+            f.q = u32x2{r.q[2 * j], r.q[2 * j + 1]};
+            F::weights(f, sc, a, b);
+            *reinterpret_cast<u32x4*>(&lds[buf * kBigHalf + wput[j]]) = decltype(hc)::value ? b : a;
+        }
+    };
+
+    f32x16 acc[4][2];
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.0f;
+
+    bf16x8 fa[2][4], fb[2][2];                            // of even and odd 16 k
+    auto frags = [&](int buf, auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+            fb[j][ni] = *reinterpret_cast<const bf16x8*>(&lds[buf * kBigHalf + wget[j] + 32 * 64 * ni]);
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi)
+            fa[j][mi] = *reinterpret_cast<const bf16x8*>(&lds[buf * kBigHalf + xget[j] + 32 * 64 * mi]);
+    };
+    auto mfmas = [&](auto jc) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[j][mi], fb[j][ni], acc[mi][ni], 0, 0, 0);
+    };
+
+    Raw raw[2];                                          // of even and odd steps
+    auto half = [&](auto bc, auto hc, int t) __attribute__((always_inline)) {
+        constexpr int B = decltype(bc)::value, H = decltype(hc)::value;
+        constexpr int here = 2 * B + H, next = H ? 2 * (B ^ 1) : here + 1, fill = H ? 2 * B : 2 * (B ^ 1) + 1;
+        constexpr int S = H ? B : B ^ 1;                 // the filled step's raw set
+        const int u = H ? t + 2 : t + 1;
+        copy_x(u, H ^ 1, fill);
+        asm volatile("" ::: "memory");                  // the loads of W stay behind the copies
+        if constexpr (H) load_w(raw[B ^ 1], t + 3);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        frags(here, std::integral_constant<int, 1>{});
+        mfmas(std::integral_constant<int, 0>{});
+        frags(next, std::integral_constant<int, 0>{});
+        mfmas(std::integral_constant<int, 1>{});
+        put_w(raw[S], u, std::integral_constant<int, H ^ 1>{}, fill);
+        static_for<0, 16>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // VALU
+            if constexpr (i % 8 < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);        // LDS read
+            if constexpr (i == 10 || i == 14) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS write
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        // Vector memory instructions finish in order: all but this half's are
+        // done, so the half filled during the half before is in LDS (its
+        // writes of W too: fragments read after them have been used).
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(H ? 4 : 2) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    const std::integral_constant<int, 0> c0{};
+    const std::integral_constant<int, 1> c1{};
+    copy_x(0, 0, 0);
+    copy_x(0, 1, 1);
+    copy_x(1, 0, 2);
+    load_w(raw[0], 0);
+    load_w(raw[1], 1);
+    put_w(raw[0], 0, c0, 0);
+    put_w(raw[0], 0, c1, 1);
+    put_w(raw[1], 1, c0, 2);
+    load_w(raw[0], 2);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    frags(0, c0);
+    for (int t = 0; t < ksteps; t += 2) {                // an even count
+        half(c0, c0, t);
+        half(c0, c1, t);
+        half(c1, c0, t + 1);
+        half(c1, c1, t + 1);
+    }
+
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni) {
+            const int n = n0 + 64 * wn + 32 * ni + (lane & 31);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + 128 * wm + 32 * mi + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (m < M && n < N) y[(int64_t)m * ldy + n] = acc[mi][ni][r];
+            }
+        }
+}
+
+__global__ void __launch_bounds__(512) gemm_big_kernel(GemmGroup g, const uint16_t* __restrict__ x, int M, int K) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[8 * kBigHalf];
+    const int64_t b = blockIdx.x;
+    int i = 0;
+#pragma unroll
+    for (int t = 1; t < kGemmGroupMax; ++t)
+        if (t < g.count && b >= g.wg_begin[t]) i = t;
+    const int mtiles = (M + kBigM - 1) / kBigM;
+    const int local = (int)(b - g.wg_begin[i]);
+    gemm_big_tile(g.w[i], x, g.y[i], (int)g.ldy[i], M, (int)g.n[i], K, local % mtiles, local / mtiles, lds);
+}
+
 // y[i] = part[0][i] + part[1][i] + ... + part[S-1][i], in that order (the
 // same bits however the splits were scheduled); 4 elements per thread, the
 // planes loaded eight at a time (sum_planes).
@@ -595,6 +787,34 @@ size_t gemm_bf16_scratch(int64_t m, int64_t n, int64_t k) {
     return sp > 1 ? (size_t)sp * (size_t)m * (size_t)n * sizeof(float) : 0;
 }
 
+// 256 x 256 tiles for Q4_K where their rounds over the 256 CUs take less time:
+// a round of them measured 117 us at k = 4096, one of 256 x 128 tiles 67 (the
+// larger tile does 8 to 15 % more per second, which a last round with few
+// tiles loses again). 512 x 28672: one round of 224 instead of two of 448, 133 ->
+// 117 us; 1000 x 28672: two instead of four, 257 -> 230; 333 x 22016: 113 ->
+// 99; but 512 x 14336: one round either way, 67 us with the smaller tiles.
+// Shapes that split K have one round of the smaller tiles.
+static bool big_tiles(int count, const int* qtypes, const int64_t* n, int64_t m) {
+    int64_t small = 0, big = 0;
+    for (int i = 0; i < count; ++i) {
+        if (qtypes[i] != kTypeQ4K) return false;
+        small += ((n[i] + kBN - 1) / kBN) * ((m + kBM - 1) / kBM);
+        big += ((n[i] + kBigN - 1) / kBigN) * ((m + kBigM - 1) / kBigM);
+    }
+    return ((big + 255) / 256) * 117 < ((small + 255) / 256) * 67;
+}
+
+// g: w, y, n, ldy of the matrices
+static hipError_t launch_big(GemmGroup g, const uint16_t* x, int64_t m, int64_t k, hipStream_t stream) {
+    int64_t wg = 0;
+    for (int i = 0; i < g.count; ++i) {
+        g.wg_begin[i] = wg;
+        wg += ((g.n[i] + kBigN - 1) / kBigN) * ((m + kBigM - 1) / kBigM);
+    }
+    gemm_big_kernel<<<dim3((unsigned)wg), dim3(512), 0, stream>>>(g, x, (int)m, (int)k);
+    return hipGetLastError();
+}
+
 hipError_t launch_split_reduce(const float* part, float* y, int splits, int64_t rows, int64_t cols, int64_t ldy,
                                hipStream_t stream) {
     const int64_t count = rows * cols;
@@ -617,6 +837,14 @@ hipError_t launch_gemm_bf16(int qtype, const uint8_t* w, const uint16_t* x, floa
     if (sp > 1 && !part) sp = 1;                           // no scratch: one split
     const int64_t tiles = ((n + kBN - 1) / kBN) * ((m + kBM - 1) / kBM);
     if (tiles * sp > 0x7FFFFFFF) return hipErrorInvalidValue;
+    if (big_tiles(1, &qtype, &n, m)) {
+        GemmGroup g{};
+        g.count = 1;
+        g.w[0] = w;
+        g.y[0] = y;
+        g.n[0] = g.ldy[0] = n;
+        return launch_big(g, x, m, k, stream);
+    }
     const dim3 grid((unsigned)(tiles * sp)), block(512);
     // loads two K-steps ahead where the step count per split is a multiple of four
     const bool ahead2 = (k / kBK / sp) % 4 == 0;
@@ -670,6 +898,7 @@ hipError_t launch_gemm_bf16_group(int count, const int* qtypes, const uint8_t* c
         if (sp > 1) pp += (int64_t)sp * m * n[i];
     }
     if (wg > 0x7FFFFFFF) return hipErrorInvalidValue;
+    if (big_tiles(count, qtypes, n, m)) return launch_big(g, x, m, k, stream);
     const bool ahead2 = (k / kBK / sp) % 4 == 0;
     if (ahead2) gemm_bf16_group_kernel<2><<<dim3((unsigned)wg), dim3(512), 0, stream>>>(g, x, (int)m, (int)k, sp);
     else gemm_bf16_group_kernel<1><<<dim3((unsigned)wg), dim3(512), 0, stream>>>(g, x, (int)m, (int)k, sp);
