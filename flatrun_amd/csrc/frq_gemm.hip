@@ -497,10 +497,7 @@ __global__ void __launch_bounds__(512) gemm_bf16_group_kernel(GemmGroup g, const
 // (wm, wn) owns the 128 x 64 sub-tile at (128 wm, 64 wn), 4 x 2 MFMA tiles, so
 // that a K-step's 32 MFMAs take 24 fragment reads from LDS, where the 64 x 64
 // sub-tiles take 16 for 16 MFMAs, and W is dequantized once per 256 rows of Y
-// by 512 threads (512 x 28672 x 4096: 133 -> 117 us, 1027 TFLOP/s on 224 of
-// 256 CUs, with W cold in the caches 137 -> 128; a large library product
-// reaches 1305 TFLOP/s. The tile has one round in which nothing hides the
-// 59 MB of results at its end). X goes from memory straight to LDS. A K-step has two halves
+// by 512 threads. X goes from memory straight to LDS. A K-step has two halves
 // of 32 k (the low and the high nibbles of a Q4_K group), each with its own
 // X and W buffers [256 rows][32 k] and one barrier. Half (t, 0) fills half
 // (t + 1, 1), half (t, 1) fills (t + 2, 0): a half is complete one barrier
@@ -509,7 +506,11 @@ __global__ void __launch_bounds__(512) gemm_bf16_group_kernel(GemmGroup g, const
 // The 16-byte chunk c of row r is at place c ^ (r / 2 % 4): eight consecutive
 // rows' fragments then lie on different banks without padding, which copies
 // straight to LDS could not leave. The order of products and sums is that of
-// gemm_tile: the same bits.
+// gemm_tile: the same bits. Results are stored past the caches: all tiles of
+// a round end together, and nothing hides the stores (the call below 129.6 ->
+// 117.6 us). 512 x (14336 | 14336) x 4096, W cold in the caches: 137 -> 118 us,
+// 1020 TFLOP/s on 224 of 256 CUs (a large library product: 1305); bound by the
+// matrix cores and the clock that their power leaves.
 constexpr int kBigM = 256, kBigN = 256, kBigHalf = 256 * 64;
 __device__ __forceinline__ void gemm_big_tile(const uint8_t* __restrict__ w, const uint16_t* __restrict__ x,
                                               float* __restrict__ y, int ldy, int M, int N, int K, int mt0, int nt0,
@@ -665,7 +666,7 @@ __device__ __forceinline__ void gemm_big_tile(const uint8_t* __restrict__ w, con
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + 128 * wm + 32 * mi + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (m < M && n < N) y[(int64_t)m * ldy + n] = acc[mi][ni][r];
+                if (m < M && n < N) __builtin_nontemporal_store(acc[mi][ni][r], &y[(int64_t)m * ldy + n]);
             }
         }
 }
@@ -788,12 +789,13 @@ size_t gemm_bf16_scratch(int64_t m, int64_t n, int64_t k) {
 }
 
 // 256 x 256 tiles for Q4_K where their rounds over the 256 CUs take less time:
-// a round of them measured 117 us at k = 4096, one of 256 x 128 tiles 67 (the
-// larger tile does 8 to 15 % more per second, which a last round with few
-// tiles loses again). 512 x 28672: one round of 224 instead of two of 448, 133 ->
-// 117 us; 1000 x 28672: two instead of four, 257 -> 230; 333 x 22016: 113 ->
-// 99; but 512 x 14336: one round either way, 67 us with the smaller tiles.
-// Shapes that split K have one round of the smaller tiles.
+// at k = 4096 a round of 256 x 128 tiles takes 67 us, one of the larger ones
+// about 110 (they do 10 to 20 % more per second, which a last round with few
+// tiles loses again). Measured, smaller / larger tiles: 512 x 28672, two rounds
+// or one, 133 / 119 us; 1000 x 28672, four or two, 258 / 232; 333 x 22016,
+// 113 / 99; 257 x 28672 113 / 112; 512 x 80000 x 1024, five or three, 115 / 110;
+// but 512 x 14336, one round either way, 67 us with the smaller tiles. Shapes
+// that split K have one round of the smaller tiles.
 static bool big_tiles(int count, const int* qtypes, const int64_t* n, int64_t m) {
     int64_t small = 0, big = 0;
     for (int i = 0; i < count; ++i) {
@@ -801,7 +803,7 @@ static bool big_tiles(int count, const int* qtypes, const int64_t* n, int64_t m)
         small += ((n[i] + kBN - 1) / kBN) * ((m + kBM - 1) / kBM);
         big += ((n[i] + kBigN - 1) / kBigN) * ((m + kBigM - 1) / kBigM);
     }
-    return ((big + 255) / 256) * 117 < ((small + 255) / 256) * 67;
+    return ((big + 255) / 256) * 110 < ((small + 255) / 256) * 67;
 }
 
 // g: w, y, n, ldy of the matrices
