@@ -42,7 +42,8 @@
 // (837 TFLOP/s of matrix work on rows padded to 384, about 1300 in a large
 // library product), Q6_K 3584 x 18944 351 / 173 (its scale per 16 elements:
 // eight times the vector work); whole calls, 97 rows of Q5_K 14336 x 4096 1391
-// (a GEMV per row) / 53, 16 rows of Q4_K 4096 x 14336 35.5 / 30.3. 128-row tiles
+// (a GEMV per row) / 52, 16 rows of Q4_K 4096 x 14336 35.5 / 30.3 (few_kernel
+// 23.8). 128-row tiles
 // are bound by the matrix cores' issue and power, few rows by the chain of
 // decode and products per wave (2.9 us per 256 of k) and the three launches.
 // MFMA operand layouts (32x32x16, 8 values per lane): A lane l holds row l%32,

@@ -168,7 +168,8 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  *   Q4_K, Q5_K, Q6_K, Q1_0 (frq_gemm_pair.hip): fp16 matrix cores on exact
  * integer codes (Q4_K / Q5_K sc q - R with R the integer nearest dmin*m / d,
  * so every term stays within 3 |w_j x_j|) and on x as hi + lo, two fp16 values
- * under a power of two per row of x: every element down to 2^-16 of the row's
+ * under a power of two per row of x (up to 32 rows of Q4_K, Q5_K and Q1_0: per
+ * row and range of k, which a workgroup sums): every element down to 2^-16 of the row's
  * largest to within 2^-23 of itself, smaller ones to within 2^-40 of the
  * largest. A row whose elements that loses more than 2^-24 of its sum |x|
  * (outliers capped at 2^-10 of the largest), or with an inf, a NaN or a largest
