@@ -106,6 +106,7 @@ SIGNATURES: dict[str, list] = {
     "frq_dev_dequant": [_i32, _vp, _sz, _i64, _vp, _vp],
     "frq_dev_dequant_f16": [_i32, _vp, _sz, _i64, _vp, _vp],
     "frq_dev_gemv": [_i32, _vp, _sz, _vp, _vp, _i64, _i64, _i64, _vp],
+    "frq_gemv_batch_plan": [_i32, _i64, _i64, _i64, _i64p],
     "frq_dev_gemv_host": [_i32, _vp, _sz, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp, _sz],
     "frq_dev_gemv_noalloc": [_i32, _vp, _sz, _vp, _vp, _i64, _i64, _i64, _vp],
     "frq_dev_gemv_group": [_i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _vp],

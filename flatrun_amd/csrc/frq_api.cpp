@@ -731,6 +731,28 @@ int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float
     return dev_gemv(qtype, w, w_bytes, x, y, n, k, batch, stream, nullptr);
 }
 
+int frq_gemv_batch_plan(int qtype, int64_t n, int64_t k, int64_t batch, int64_t plan[4]) {
+    Fmt f;
+    if (!plan) return fail(FRQ_ERR_INVALID, "null plan");
+    if (!fmt_of(qtype, &f)) return fail(FRQ_ERR_INVALID, "unknown qtype %d", qtype);
+    if (n <= 0 || k <= 0 || batch < 2 || k % f.belems) return fail(FRQ_ERR_SHAPE, "batch plan: shape");
+    for (int i = 0; i < 4; ++i) plan[i] = 0;
+    switch (batch_route(qtype, nullptr, nullptr, batch, n, k, kPairScratchMax)) {
+        case BatchRoute::SmallM: plan[0] = FRQ_BATCH_SMALL; break;
+        case BatchRoute::Gemm: plan[0] = FRQ_BATCH_GEMM; break;
+        case BatchRoute::Rows: plan[0] = FRQ_BATCH_ROWS; break;
+        case BatchRoute::Pair: {
+            frq::PairPlan p;
+            pair_plan(qtype, nullptr, nullptr, batch, n, k, kPairScratchMax, &p);
+            plan[0] = p.few ? FRQ_BATCH_FEW : FRQ_BATCH_PAIR;
+            plan[1] = p.bm;
+            plan[2] = p.splits;
+            plan[3] = (int64_t)p.bytes;
+        }
+    }
+    return FRQ_OK;
+}
+
 int frq_dev_gemv_host(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
                       int64_t batch, void* scratch, size_t scratch_bytes, void* pinned, size_t pinned_bytes) {
     if (n < 0 || k < 0 || batch < 0) return fail(FRQ_ERR_SHAPE, "host gemv: negative shape");

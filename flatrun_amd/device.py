@@ -255,6 +255,17 @@ def gemv(qtype, w, x, y, n: int, k: int, batch: int = 1, stream=None, w_bytes: i
     check(lib().frq_dev_gemv(q, _addr(w), wb, _addr(x), _addr(y), int(n), int(k), int(batch), _stream(stream)))
 
 
+BATCH_ROUTES = ("rows", "small", "pair", "few", "gemm")
+
+
+def batch_plan(qtype, n: int, k: int, batch: int) -> tuple[str, int, int, int]:
+    """(route, rows per tile, splits of k, scratch bytes) of a batched gemv
+    (frq_gemv_batch_plan); needs no GPU."""
+    plan = (ctypes.c_int64 * 4)()
+    check(lib().frq_gemv_batch_plan(qtype_id(qtype), int(n), int(k), int(batch), plan))
+    return BATCH_ROUTES[plan[0]], plan[1], plan[2], plan[3]
+
+
 def gemv_host(qtype, w, x: np.ndarray, y: np.ndarray, n: int, k: int, batch: int, scratch: DeviceBuffer,
               pinned: PinnedBuffer | None = None, w_bytes: int | None = None) -> None:
     """gemv with x and y in host memory (contiguous float32, (batch, k) and

@@ -195,6 +195,17 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
 int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
                  int64_t batch, void* stream);
 
+/* Which kernel a batch (two or more rows, aligned x and w) takes and how it
+ * splits the work: plan[0] = FRQ_BATCH_*, and for the pair kernels plan[1] =
+ * rows of x per tile, plan[2] = splits of k, plan[3] = bytes of scratch of the
+ * first 1024 rows (0 for the others). A function of its arguments only. */
+#define FRQ_BATCH_ROWS 0    /* one GEMV per row */
+#define FRQ_BATCH_SMALL 1   /* a small-M matvec */
+#define FRQ_BATCH_PAIR 2    /* frq_gemm_pair.hip, tiles of 32, 64 or 128 rows */
+#define FRQ_BATCH_FEW 3     /* frq_gemm_pair.hip, up to 32 rows in one kernel */
+#define FRQ_BATCH_GEMM 4    /* frq_gemm_f32.hip */
+int frq_gemv_batch_plan(int qtype, int64_t n, int64_t k, int64_t batch, int64_t plan[4]);
+
 /* frq_dev_gemv with x and y in host memory, synchronous, on the null stream.
  * `scratch`: device memory for both, at least 4 k batch rounded up to 256,
  * plus 4 n batch bytes (16-byte aligned). `pinned`: page-locked host memory
