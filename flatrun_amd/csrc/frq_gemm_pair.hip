@@ -5,13 +5,15 @@
 // The reference's batched entry points (matmul_<q>_batched, _C.cpp:154-283)
 // run one fp32 matvec per row of X. Here the products run on
 // v_mfma_f32_32x32x16_f16, two per product:
-//   * x enters as hi + lo, hi = f16(x 2^e), lo = f16(x 2^e - hi), with 2^e a
-//     power of two per row that puts the row's largest |x| in [2^14, 2^15).
-//     The pair carries every element down to 2^-16 of the row's largest to
-//     within 2^-23 of itself, smaller ones to within 2^-40 of the largest.
-//   * W enters as integers that f16 holds exactly (times 2^-14): Q4_K / Q5_K
-//     sc q - R with R the integer nearest dmin m / d, Q6_K q - 32, Q1_0 +-1.
-//     A nibble masked in place is the f16 subnormal
+//   * x enters as hi + lo 2^-12, hi = f16(x 2^e), lo = f16((x 2^e - hi) 2^12),
+//     with 2^e a power of two per row that puts the row's largest |x| in
+//     [2^14, 2^15). The pair carries every element down to 2^-28 of the row's
+//     largest to within 2^-23 of itself, smaller ones to within 2^-51 of the
+//     largest: its own 2^-19 down to 2^-32.
+//   * W enters as integers that f16 holds exactly (times 2^-14 for the products
+//     with lo, 2^-2 for those with hi: one v_pk_mul_f16 per two codes apart):
+//     Q4_K / Q5_K sc q - R with R the integer nearest dmin m / d, Q6_K q - 32,
+//     Q1_0 +-1 (2^-12 and 1). A nibble masked in place is the f16 subnormal
 //     q 2^-24 (or 16 q 2^-24), so one v_pk_fma_f16 turns two of them into
 //     codes, scale and centre included.
 //   * the matrix cores sum 64 elements (Q6_K 16, one sub-block) in fp32, then
@@ -25,12 +27,14 @@
 //   large x on a weight that is exactly zero leaves the others their bits.
 //
 // split_kernel writes the pairs once per call in the order the matrix cores
-// take them, with the scale per row. It also measures, per row, the error
-// of the split beyond 2^-23 of each element, against 2^-24 of sum |x| with
-// elements capped at 2^-10 of the largest: a row beyond that (an outlier some
-// 2^17 above the rest), one whose largest |x| is outside [2^-100, 2^100], and
-// one with an inf or NaN are computed weight by weight in fp64 instead
-// (finish_kernel), as gemm_f32's are.
+// take them, with the scale per row. A row whose largest |x| is outside
+// [2^-100, 2^101) and one with an inf or NaN are computed weight by weight in
+// fp64 instead (finish_kernel), as gemm_f32's are. What the pairs miss of
+// elements by more than 2^-19 of the element itself (SwiGLU makes some: 1e-20
+// beside 1e2) is added up per row; times the largest weight of a row of W that
+// bounds what an output lost. It only counts where the weights of all the larger
+// x are zero or nearly so, that is in an output that small itself: an output
+// below 2^19 of that bound is computed weight by weight in fp64 too.
 //
 // Tiling: BM x BN of Y per workgroup; a wave owns 32 MT x 32 NT. W goes from
 // memory to registers to the matrix cores (lane = one row of W; both halves
@@ -53,6 +57,8 @@
 #include "frq_common.h"
 #include "frq_kernels.h"
 #include "frq_weight_at.h"
+
+#include <type_traits>
 
 namespace frq {
 namespace {
@@ -79,6 +85,14 @@ constexpr int kStageBytes = 8192;        // 32 rows x 64 k x 2 pieces x 2 bytes
 template <int QT>
 constexpr bool kK4 = QT == kTypeQ4K || QT == kTypeQ5K;
 
+constexpr uint32_t kSignCode = 0x0C000C00u;   // +2^-12 twice
+// The largest |code| under a scale d: an output's limit is a row's `lim` (2^19 of
+// what its pairs miss) times this and the largest |d| of a row of W.
+template <int QT>
+constexpr float kMaxCode = QT == kTypeQ4K ? 63.0f * 15.0f : QT == kTypeQ5K ? 63.0f * 31.0f : QT == kTypeQ6K ? 4096.0f : 1.0f;
+// Whether an output stands as computed.
+__device__ __forceinline__ bool stands(float y, float limit) { return !(fabsf(y) < limit); }
+
 __device__ __forceinline__ f16x2 as_f16x2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ uint32_t as_u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ uint32_t fma2(uint32_t a, f16x2 b, f16x2 c) {
@@ -90,6 +104,12 @@ __device__ __forceinline__ f16x2 pair_of(float v) {   // v exact in f16
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
     const f32x2 v = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+// Codes for hi from those for lo (exact).
+__device__ __forceinline__ f16x8 for_hi(f16x8 c) { return c * (_Float16)4096.0f; }
+__device__ __forceinline__ float add_scaled(float s, float t, float acc) { return __builtin_fmaf(s, t, acc); }
+__device__ __forceinline__ double add_scaled(float s, float t, double acc) {
+    return __builtin_fma((double)s, (double)t, acc);
 }
 __device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
@@ -233,7 +253,7 @@ struct Body<kTypeQ6K> {
     __device__ __forceinline__ u32x4 frag(const Head<kTypeQ6K>& hh) const {
         constexpr int p = T & 1, c = I >> 1, g = I & 1;
         u32x4 r;
-        const f16x2 m = c ? pair_of(64.0f) : pair_of(1024.0f), o = pair_of(-32.0f / 16384.0f);
+        const f16x2 m = c ? pair_of(64.0f) : pair_of(1024.0f), o = pair_of(-32.0f * 0x1p-14f);
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const uint32_t v = shifted(ql[T][g][e], ql[T][g][e + 1], hh.sh), v8 = v >> 8;
@@ -251,7 +271,7 @@ struct Body<kTypeQ6K> {
     __device__ __forceinline__ float scale(const Head<kTypeQ6K>& hh) const {
         constexpr int j = (I & 1) + 2 * ((T & 1) + 2 * (I >> 1)), e = j >> 2;
         const uint32_t v = shifted(sc[T >> 1][e], sc[T >> 1][e + 1], hh.sh);
-        return f16_bits_to_f32(hh.d) * 16384.0f * (float)(int)(int8_t)(v >> (8 * (j & 3)));
+        return f16_bits_to_f32(hh.d) * 4.0f * (float)(int)(int8_t)(v >> (8 * (j & 3)));
     }
 };
 
@@ -281,7 +301,7 @@ struct Body<kTypeQ10> {
         u32x4 r;
         static_for<0, 4>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
-            r[j] = ((q[T] << (15 - 4 * I - j)) & 0x80008000u) | 0x3C003C00u;
+            r[j] = ((q[T] << (15 - 4 * I - j)) & 0x80008000u) | kSignCode;
         });
         return r;
     }
@@ -333,29 +353,38 @@ __device__ __forceinline__ T row_reduce(T v, T* lds, int tr, Op op) {
     return t;
 }
 
-// Eight scaled values as pairs; body collects sum |x| capped at 2^-10 of the
-// largest.
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo, float& body) {
+// Eight scaled values as pairs.
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const f16x2 hv = {(_Float16)v[2 * p], (_Float16)v[2 * p + 1]};
-        const f16x2 lv = {(_Float16)(v[2 * p] - (float)hv[0]), (_Float16)(v[2 * p + 1] - (float)hv[1])};
+        const f16x2 lv = {(_Float16)((v[2 * p] - (float)hv[0]) * 4096.0f), (_Float16)((v[2 * p + 1] - (float)hv[1]) * 4096.0f)};
         hi[p] = as_u32(hv);
         lo[p] = as_u32(lv);
-        body += fminf(fabsf(v[2 * p]), 16.0f) + fminf(fabsf(v[2 * p + 1]), 16.0f);
     }
 }
-// What the pairs of four scaled values lose beyond 2^-23 of each: elements below
-// 2^-16 of the largest only, and at most 2^-25 each, so rows of N elements with
-// N 2^-25 <= 2^-24 body pass without it.
-__device__ __forceinline__ float lost4(const f32x4 v) {
-    float e = 0.0f;
+// What the pairs of four values x, scaled by s, miss of those that they miss by
+// more than 2^-19 of the value. Only values below 2^-18 can be (the error is at
+// most 2^-37 there and 2^-23 of the value above): those `least` finds. A value that
+// the scale takes to zero counts as 2^-60.
+__device__ __forceinline__ float lost4(const f32x4 x, float s) {
+    float lost = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float r = v[i] - (float)(_Float16)v[i];
-        e += fmaxf(fabsf(r - (float)(_Float16)r) - 0x1p-23f * fabsf(v[i]), 0.0f);
+        const float v = x[i] * s, r = v - (float)(_Float16)v;
+        const float e = fabsf(r - (float)(_Float16)(r * 4096.0f) * 0x1p-12f);
+        lost += v == 0.0f ? (x[i] != 0.0f ? 0x1p-60f : 0.0f) : e > 0x1p-19f * fabsf(v) ? e : 0.0f;
     }
-    return e;
+    return lost;
+}
+// The least nonzero |x| of v and `small`, as bits doubled less one.
+__device__ __forceinline__ uint32_t least(uint32_t small, const f32x4 v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) small = min(small, (__float_as_uint(v[e]) << 1) - 1u);
+    return small;
+}
+__device__ __forceinline__ bool below(uint32_t small, int e) {   // least's value under a scale 2^e: below 2^-18
+    return small < (__float_as_uint(ldexpf(1.0f, -18 - e)) << 1) - 1u;
 }
 
 // The largest |x| of v and `big`, as bits (a NaN above inf).
@@ -391,7 +420,8 @@ __device__ __forceinline__ float sum8(float v) {       // over eight neighbourin
 }
 
 // The pairs of every row of x, the sub-block sums' pieces (Q4_K / Q5_K) and
-// the factor that undoes the row's scale (0 = row computed weight by weight).
+// the factor that undoes the row's scale (0 = row computed weight by weight),
+// and lim, 2^19 of what the row's pairs miss.
 // RW rows per workgroup, TPR threads each, NC pieces of eight elements per
 // thread: x is read once, into registers (NC = 0: rows too long for that are
 // read twice). Eight neighbouring rows, whose 16-byte parts share lines of
@@ -399,7 +429,7 @@ __device__ __forceinline__ float sum8(float v) {       // over eight neighbourin
 template <int QT, int RW, int TPR, int NC>
 __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict__ x, int M, int K, int units,
                                                          uint8_t* __restrict__ xf, uint8_t* __restrict__ xsum,
-                                                         float* __restrict__ inv) {
+                                                         float* __restrict__ inv, float* __restrict__ lim) {
     __shared__ float red[RW][TPR / 64];
     static_assert(RW <= 8, "rows of a workgroup share an XCD's eight");
     constexpr int WR = 8 / RW;                         // workgroups of eight rows
@@ -431,7 +461,6 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
     int e;
     bool ok = row_scale(big, e);                         // max |x| 2^e in [2^14, 2^15)
     const float scale = ok ? ldexpf(1.0f, e) : 0.0f;
-    float body = 0.0f;
     const int64_t mt = m >> 5;
     const int nst = units * 4;
     auto split = [&](int c, f32x4 a, f32x4 b) __attribute__((always_inline)) {
@@ -442,7 +471,7 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
         float v[8];
         Order<QT>::order(a, b, v);
         u32x4 hi, lo;
-        split8(v, hi, lo, body);
+        split8(v, hi, lo);
         const bool out = live && c < chunks;
         if (out) {
             uint8_t* fp = xf + ((mt * nst + st) * 8 + 2 * i) * 1024 + ((m & 31) + 32 * h) * 16;
@@ -470,21 +499,36 @@ __global__ void __launch_bounds__(RW * TPR) split_kernel(const float* __restrict
             split(c, a, b);
         }
     }
-    const auto add = [](float a, float b) { return a + b; };
-    body = row_reduce<TPR>(body, red[rr], tr, add);
-    // (a workgroup of one row decides alike in all its threads; others always look)
-    if (RW > 1 || (float)(units * kUnit) > 2.0f * body) {
-        float err = 0.0f;
+    float lost = 0.0f;
+    if (ok) {                                            // (a row decides alike in all its threads)
         if constexpr (NC > 0) {
+            uint32_t small = ~0u;
 #pragma unroll
-            for (int j = 0; j < NC; ++j) err += lost4(xa[j] * scale) + lost4(xb[j] * scale);
+            for (int j = 0; j < NC; ++j) small = least(least(small, xa[j]), xb[j]);
+            if (below(small, e)) {
+#pragma unroll
+                for (int j = 0; j < NC; ++j) lost += lost4(xa[j], scale) + lost4(xb[j], scale);
+            }
         } else {
-            for (int c = tr; c < K / 4; c += TPR) err += lost4(*reinterpret_cast<const f32x4*>(xr + 4 * c) * scale);
+            for (int c = tr; c < K / 4; c += TPR) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(xr + 4 * c);
+                if (below(least(~0u, v), e)) lost += lost4(v, scale);
+            }
         }
-        err = row_reduce<TPR>(err, red[rr], tr, add);
-        ok = ok && err <= 0x1p-24f * body;
     }
-    if (tr == 0 && live) inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
+    lost = row_reduce<TPR>(lost, red[rr], tr, [](float a, float b) { return a + b; });
+    if (tr == 0 && live) {
+        inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
+        lim[m] = ldexpf(lost, 19 - e);
+    }
+}
+
+// The largest |d| of a unit (of its second half's block too: Q1_0).
+template <int QT>
+__device__ __forceinline__ float largest_scale(const Head<QT>& h, const Body<QT>& b) {
+    if constexpr (QT == kTypeQ10) return fmaxf(fabsf(f16_bits_to_f32(b.d[0])), fabsf(f16_bits_to_f32(b.d[1])));
+    else if constexpr (QT == kTypeQ6K) return fabsf(f16_bits_to_f32(h.d));
+    else return fabsf(f16_bits_to_f32(h.hd[0]));
 }
 
 template <int QT>
@@ -507,11 +551,13 @@ __device__ __forceinline__ u32x2 both(uint32_t v) {
 }
 
 // What Q4_K / Q5_K add to a stage: its two sub-blocks' code constants and the
-// B fragment of (R - dmin m / d) 2^-14, to be multiplied by sum(x) (the pieces
+// B fragment of (R - dmin m / d) 2^-E, to be multiplied by sum(x) (the pieces
 // of split_kernel's fragment: w1 x1, w1 x2, w2 x1, w2 x2 | w1 x3, w3 x1). Each of
 // the two lanes of a row that share the sub-blocks works out one of them (sc,
-// mn; odd: which).
+// mn; odd: which). 2^-E is the unit of the codes that meet hi.
+template <int E>
 struct K4Stage {
+    static constexpr float kUnit = 1.0f / (1 << E), kInv = 1 << E;
     f16x2 mul[2], off[2];
     u32x4 uf;
     template <int QT, bool ROW16>
@@ -523,7 +569,7 @@ struct K4Stage {
         const float s = z ? 0.0f : (float)sc, tm = dm * (float)mn;          // exact
         // d non-finite: fmaxf drops a NaN, so R lands in range anyway
         const float R = fminf(fmaxf(__builtin_rintf(tm * rd), 0.0f), (QT == kTypeQ4K ? 15.0f : 31.0f) * s);
-        const float u = __builtin_fmaf(d, R, -tm) * (rd * 0x1p-14f);        // d R - tm in one rounding
+        const float u = __builtin_fmaf(d, R, -tm) * (rd * kUnit);          // d R - tm in one rounding
         const u32x2 m = both<ROW16>(as_u32(pair_of(s * (odd ? 64.0f : 1024.0f))));
         const u32x2 o = both<ROW16>(as_u32(pair_of(R * -0x1p-14f)));
         mul[0] = as_f16x2(m[0]), mul[1] = as_f16x2(m[1]);
@@ -537,7 +583,7 @@ struct K4Stage {
     }
     __device__ static __forceinline__ float scale(const u32x4 hd) {
         const float d = f16_bits_to_f32(hd[0]);
-        return d == 0.0f ? 16384.0f : d * 16384.0f;
+        return d == 0.0f ? kInv : d * kInv;
     }
 };
 
@@ -565,8 +611,8 @@ __device__ __forceinline__ void interleave() {
 template <int QT, int WM, int WN, int MT, int NT, int DEPTH>
 __global__ void __launch_bounds__(512) gemm_pair_kernel(
     const uint8_t* __restrict__ w, const uint8_t* __restrict__ xf, const uint8_t* __restrict__ xsum,
-    const float* __restrict__ inv, float* __restrict__ y, int M, int N, int K, int units, int64_t ldy, int S,
-    float* __restrict__ part) {
+    const float* __restrict__ inv, const float* __restrict__ lim, float* __restrict__ y, int M, int N, int K, int units,
+    int64_t ldy, int S, float* __restrict__ part, uint32_t* __restrict__ aux) {
     static_assert(WM * WN == 8, "eight waves");
     constexpr bool DB = DEPTH > 1;
     constexpr int BT = WM * MT, BM = 32 * BT, BN = 32 * WN * NT;
@@ -624,8 +670,12 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
         return *reinterpret_cast<const bf16x8*>(&xs[buf + kSumOff + (MT * wm + mt) * (LS * 1024) + st * 1024 + lane * 16]);
     };
 
+    constexpr int kE = MT * NT > 2 ? 14 : 2;
+    constexpr bool kScaleT = kK4<QT> && MT * NT > 2;
     constexpr bool kTwo = MT * NT <= 2;                // room for a second level
-    f32x16 acc[MT][NT], tot[kTwo ? MT : 1][NT], t[2];
+    typedef float Sum;
+    Sum acc[MT][NT][16];
+    f32x16 tot[kTwo ? MT : 1][NT], t[2];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -644,7 +694,7 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
     constexpr int HS = DB ? DEPTH : kK4<QT> ? 1 : 2, UR = DB ? DEPTH : 2;   // sets, units per round of the loop
     Head<QT> hd[HS][NT];
     Body<QT> bd[DEPTH][NT];
-    float d14[NT] = {};
+    float d4[NT] = {}, dmax = 0.0f;                    // dmax: the largest |d| of the lane's rows of W
     auto load_head = [&](Head<QT> (&hh)[NT], int u) __attribute__((always_inline)) {
         const gptr up = scalar_base(wtile + (int64_t)(u < u1 ? u : u1 - 1) * kUnitBytes);
 #pragma unroll
@@ -668,7 +718,7 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
     auto decode = [&](auto tc, auto gc, const Head<QT>& hh, const Body<QT>& bb) __attribute__((always_inline)) {
         constexpr int T = decltype(tc)::value, I0 = decltype(gc)::value * GS;
         Codes c;
-        K4Stage ks;
+        K4Stage<kE> ks;
         if constexpr (kK4<QT>) {
             // (sc, m) of sub-block 2T + h (get_scale_min_k4, gguf.py:135-163)
             const u32x4 hw = head_words(hh);
@@ -720,7 +770,11 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
             }
             if constexpr (kK4<QT> && T == 0) {
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) d14[nt] = K4Stage::scale(head_words(hh[nt]));
+                for (int nt = 0; nt < NT; ++nt) d4[nt] = K4Stage<kE>::scale(head_words(hh[nt]));
+            }
+            if constexpr (T == 2) {
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) dmax = fmaxf(dmax, largest_scale(hh[nt], bb[nt]));
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (GS == 4) {
@@ -747,18 +801,27 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
                     }
                     constexpr int C = (T * MT * NT + PH) & 1;          // this chain's set
                     const f32x16 zero = {};
-                    if constexpr (kK4<QT>) t[C] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sx, b[nt].u, zero, 0, 0, 0);
+                    if constexpr (kK4<QT> && !kScaleT) t[C] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sx, b[nt].u, zero, 0, 0, 0);
 #pragma unroll
-                    for (int q = 1; q >= 0; --q)                        // lo, then hi
+                    for (int q = 1; q >= 0; --q) {                      // lo, then hi
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
                             t[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                a[i][q], b[nt].s[i], !kK4<QT> && q == 1 && i == 0 ? zero : t[C], 0, 0, 0);
+                                a[i][q], q || kScaleT ? b[nt].s[i] : for_hi(b[nt].s[i]),
+                                (!kK4<QT> || kScaleT) && q == 1 && i == 0 ? zero : t[C], 0, 0, 0);
+                        if constexpr (kScaleT) {
+                            if (q) {
+#pragma unroll
+                                for (int r = 0; r < 16; ++r) t[C][r] *= 0x1p-12f;
+                                t[C] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sx, b[nt].u, t[C], 0, 0, 0);
+                            }
+                        }
+                    }
                     constexpr int PP = (PH + MT * NT - 1) % (MT * NT);  // the chain before this one
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
-                        acc[PP / NT][PP % NT][r] = __builtin_fmaf(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
-                    if constexpr (kK4<QT>) tsc = d14[nt];
+                        acc[PP / NT][PP % NT][r] = add_scaled(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
+                    if constexpr (kK4<QT>) tsc = d4[nt];
                     else tsc = bb[nt].template scale<T, 3>(hh[nt]);
                     if constexpr (last) b[0] = b0;
                     if constexpr (lastnt) {
@@ -768,7 +831,14 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
                             for (int i = 0; i < 4; ++i) a[i][q] = an[i][q];
                         sx = sn;
                     }
-                    interleave<8 + (kK4<QT> ? 1 : 0), 2 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0)>();
+                    if constexpr (kScaleT) {
+                        constexpr int V = 2 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0);
+                        interleave<4, V>();
+                        __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+                        interleave<5, V>();
+                    } else {
+                        interleave<8 + (kK4<QT> ? 1 : 0), 4 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0)>();
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (!DB && PH == (QT == kTypeQ5K && MT * NT > 2 ? 1 : 0)) {
                         if constexpr (T == (HS == 1 ? 3 : 2)) load_head(hn, u + 1);
@@ -805,12 +875,12 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
                         for (int q = 1; q >= 0; --q)
 #pragma unroll
                             for (int i = 0; i < GS; ++i)
-                                t[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i][q], b[nt].s[i],
+                                t[C] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i][q], q ? b[nt].s[i] : for_hi(b[nt].s[i]),
                                                                               q == 1 && i == 0 ? zero : t[C], 0, 0, 0);
                         constexpr int PP = (mt * NT + nt + MT * NT - 1) % (MT * NT);
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
-                            acc[PP / NT][PP % NT][r] = __builtin_fmaf(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
+                            acc[PP / NT][PP % NT][r] = add_scaled(tsc, t[C ^ 1][r], acc[PP / NT][PP % NT][r]);
                         if constexpr (mt == 0) gsc[nt] = bb[nt].template scale<T, G_ * GS>(hh[nt]);
                         tsc = gsc[nt];
                     });
@@ -822,7 +892,7 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
                     for (int q = 0; q < 2; ++q)
 #pragma unroll
                         for (int i = 0; i < GS; ++i) a[i][q] = an[i][q];
-                    interleave<2 * GS * NT, (GS == 1 ? 9 : 5) + (lastmt ? (GS == 1 ? 9 : 7) : 0)>();
+                    interleave<2 * GS * NT, (GS == 1 ? 11 : 7) + (lastmt ? (GS == 1 ? 9 : 7) : 0)>();
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (!DB && G_ == 0 && mt == 0) {
                         if constexpr (T == 2) load_head(hn, u + 1);
@@ -886,9 +956,11 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
-                    tot[mt][nt] += acc[mt][nt];
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+                    for (int r = 0; r < 16; ++r) {
+                        tot[mt][nt][r] += acc[mt][nt][r];
+                        acc[mt][nt][r] = 0.0f;
+                    }
                 }
         }
     };
@@ -912,82 +984,176 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
         }
     });
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[MT - 1][NT - 1][r] = __builtin_fmaf(tsc, t[1][r], acc[MT - 1][NT - 1][r]);
+    for (int r = 0; r < 16; ++r) acc[MT - 1][NT - 1][r] = add_scaled(tsc, t[1][r], acc[MT - 1][NT - 1][r]);
     if constexpr (kTwo) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] += tot[mt][nt];
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[mt][nt][r] += tot[mt][nt][r];
     }
 
-    float* out = S == 1 ? y : part + (int64_t)split * M * N;
-    const int64_t ld = S == 1 ? ldy : N;
+    if (S > 1) {
+        float* out = part + (int64_t)split * M * N;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int n = n0 + 32 * (NT * wn + nt) + (lane & 31);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = 32 * (mt0 + MT * wm + mt) + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (m < M && n < N) out[(int64_t)m * N + n] = (float)acc[mt][nt][r];
+                }
+            }
+        if (mt0 == 0 && wm == 0 && h == 0) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int n = n0 + 32 * (NT * wn + nt) + lane;
+                if (n < N) aux[split * N + n] = __float_as_uint(dmax * kMaxCode<QT>);
+            }
+        }
+        return;
+    }
+    // S = 1: outputs that do not stand leave as NaN, and the wave's word of aux tells finish_kernel
+    uint32_t redo = 0;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int m = 32 * (mt0 + MT * wm + mt) + 8 * i + 4 * h;
-            f32x4 f = {1.0f, 1.0f, 1.0f, 1.0f};
-            if (S == 1) f = *reinterpret_cast<const f32x4*>(inv + m);   // inv is padded to whole tiles
+            const f32x4 f = *reinterpret_cast<const f32x4*>(inv + m);   // (padded to whole tiles, as lim)
+            const f32x4 g = *reinterpret_cast<const f32x4*>(lim + m);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 const int n = n0 + 32 * (NT * wn + nt) + (lane & 31);
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (m + r < M && n < N) out[(int64_t)(m + r) * ld + n] = acc[mt][nt][4 * i + r] * f[r];
+                for (int r = 0; r < 4; ++r) {
+                    float v = (float)acc[mt][nt][4 * i + r] * f[r];
+                    if (!stands(v, g[r] * (dmax * kMaxCode<QT>))) {
+                        v = __builtin_nanf("");
+                        redo |= m + r < M && n < N;
+                    }
+                    if (m + r < M && n < N) y[(int64_t)(m + r) * ldy + n] = v;
+                }
             }
         }
+    const bool any = __ballot(redo) != 0;
+    if (lane == 0) aux[(mt0 / MT + wm) * (ntiles * WN) + n0 / (32 * NT) + wn] = any;
+}
+
+// A row of x times one of W by a wave in fp64, the sum in every lane.
+template <int QT>
+__device__ __forceinline__ float exact_dot(const uint8_t* __restrict__ wr, const float* __restrict__ xr, int K, int lane) {
+    double s = 0.0;
+    for (int j = lane; j < K; j += 64) s = __builtin_fma((double)weight_at<QT>(wr, j), (double)xr[j], s);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+    return (float)s;
 }
 
 // S > 1: y = inv * (the planes added in split order, in fp64: free here, and
-// one rounding instead of S). Then, S = 1 too, the rows that the pairs do not
-// carry, weight by weight in fp64, a wave per output over the whole grid: those
-// with inv = 0, or, where every split judged its part of x itself (few_kernel;
-// inv null, the planes in units of y, at most 32 rows), with a flag of any split.
+// one rounding instead of S). Then, S = 1 too, what the pairs do not carry,
+// weight by weight in fp64, a wave per row of W over the whole grid:
+//   * rows with inv = 0, or, where every split judged its part of x itself
+//     (few_kernel; inv null, the planes in units of y, at most 32 rows, lim [S][32]),
+//     an infinite lim of any split;
+//   * single outputs that do not stand, marked as NaN: with S > 1 by the planes'
+//     sum and the largest scales that aux [S][N] holds, with S = 1 those in the
+//     tiles of tm x tn outputs (one wave's) that aux marks.
 template <int QT>
 __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ part, float* __restrict__ y, int S,
                                                      int M, int N, int64_t ldy, const float* __restrict__ inv,
-                                                     const uint32_t* __restrict__ flags, const uint8_t* __restrict__ w,
+                                                     const float* __restrict__ lim, const uint32_t* __restrict__ aux,
+                                                     int tm, int tn, const uint8_t* __restrict__ w,
                                                      const float* __restrict__ x, int K) {
     const int lane = threadIdx.x & 63, wv = (int)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int)gridDim.x * 4;
-    uint32_t bad = 0;                                    // rows < 32, of any split
+    uint32_t bad = 0;                                    // few_kernel's rows, of any split
+    float few_lim = 0.0f;                                // of row lane % 32
     if (!inv) {
-        for (int i = lane; i < 32 * S; i += 64)
-            if (flags[i] && (i & 31) < M) bad |= 1u << (i & 31);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) bad |= (uint32_t)__shfl_xor((int)bad, o, 64);
+        for (int i = lane; i < 32 * S; i += 64) few_lim += (i & 31) < M ? lim[i] : 0.0f;
+        few_lim += __shfl_xor(few_lim, 32, 64);
+        bad = (uint32_t)__ballot(few_lim == __builtin_inff());
     }
-    auto factor = [&](int m) __attribute__((always_inline)) {
-        return inv ? inv[m] : (bad >> m) & 1u ? 0.0f : 1.0f;
+    const int64_t row_bytes = weight_row_bytes<QT>(K);
+    // the lane's output (m, n), where it is a NaN and `in`
+    auto redo_nans = [&](bool in, int m, int n) __attribute__((always_inline)) {
+        const float v = in ? y[(int64_t)m * ldy + n] : 0.0f;
+        for (uint64_t redo = __ballot(v != v); redo; redo &= redo - 1) {
+            const int l = __builtin_ctzll(redo), ml = __builtin_amdgcn_readlane(m, l), nl = __builtin_amdgcn_readlane(n, l);
+            const float o = exact_dot<QT>(w + (int64_t)nl * row_bytes, x + (int64_t)ml * K, K, lane);
+            if (lane == l) y[(int64_t)m * ldy + n] = o;
+        }
     };
-    const int64_t plane = (int64_t)M * N;
     if (S > 1) {
-        if (((N | ldy) & 3) == 0 && !(reinterpret_cast<uintptr_t>(y) & 15)) {
-            const int nq = N >> 2;
-            const int64_t total = (int64_t)M * nq, step = (int64_t)gridDim.x * 256;
-            for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += step) {
-                const int m = (int)(e / nq), n = 4 * (int)(e - (int64_t)m * nq);
+        // V neighbouring outputs per lane; rows computed below are left alone
+        auto add = [&](auto vc) __attribute__((always_inline)) {
+            constexpr int V = decltype(vc)::value;
+            typedef float fv __attribute__((ext_vector_type(V)));
+            typedef double dv __attribute__((ext_vector_type(V)));
+            const int64_t plane = (int64_t)M * N, total = plane / V, step = (int64_t)gridDim.x * 256;
+            const int nq = N / V;
+            bool again = false;
+            for (int64_t e0 = (int64_t)wv * 64; e0 < total; e0 += step) {
+                const int64_t e = e0 + lane < total ? e0 + lane : total - 1;
+                const int m = (int)(e / nq), n = V * (int)(e - (int64_t)m * nq);
                 const float* p = part + (int64_t)m * N + n;
-                f64x4 v = {};
+                dv v = {};
                 for (int q0 = 0; q0 < S; q0 += 8) {      // eight loads in flight
-                    f32x4 t[8];
+                    fv t[8];
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) t[q] = *reinterpret_cast<const f32x4*>(p + (q0 + q < S ? q0 + q : 0) * plane);
+                    for (int q = 0; q < 8; ++q) t[q] = *reinterpret_cast<const fv*>(p + (q0 + q < S ? q0 + q : 0) * plane);
 #pragma unroll
                     for (int q = 0; q < 8; ++q)
-                        if (q0 + q < S) v += __builtin_convertvector(t[q], f64x4);
+                        if (q0 + q < S) v += __builtin_convertvector(t[q], dv);
                 }
-                const float f = factor(m);
-                if (f != 0.0f)
-                    *reinterpret_cast<f32x4*>(y + (int64_t)m * ldy + n) = __builtin_convertvector(v * (double)f, f32x4);
+                const float f = inv ? inv[m] : (bad >> m) & 1u ? 0.0f : 1.0f;
+                const float g = inv ? lim[m] : __shfl(few_lim, m, 64);
+                fv r = __builtin_convertvector(v * (double)f, fv);
+                const bool in = e0 + lane < total && f != 0.0f;
+                fv c = {};                                // the largest scales, where the limit is not zero
+                if (__ballot(g != 0.0f)) {
+                    const float* a = reinterpret_cast<const float*>(aux) + n;
+#pragma unroll 1
+                    for (int q0 = 0; q0 < S; q0 += 8) {
+                        fv t[8];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) t[q] = *reinterpret_cast<const fv*>(a + (int64_t)(q0 + q < S ? q0 + q : 0) * N);
+#pragma unroll
+                        for (int q = 0; q < 8; ++q)
+#pragma unroll
+                            for (int i = 0; i < V; ++i) c[i] = fmaxf(c[i], t[q][i]);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    if (!stands(r[i], g * c[i])) {
+                        r[i] = __builtin_nanf("");
+                        again |= in;
+                    }
+                if (in) *reinterpret_cast<fv*>(y + (int64_t)m * ldy + n) = r;
             }
-        } else {
-            const int64_t step = (int64_t)gridDim.x * 256;
-            for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < plane; e += step) {
-                const int m = (int)(e / N), n = (int)(e - (int64_t)m * N);
-                const double v = sum_planes<double>([&](int q) { return (double)part[e + q * plane]; }, S);
-                const float f = factor(m);
-                if (f != 0.0f) y[(int64_t)m * ldy + n] = (float)(v * f);
+            if (!__ballot(again)) return;
+            for (int64_t e0 = (int64_t)wv * 64; e0 < total; e0 += step) {   // every lane its own outputs again
+                const int64_t e = e0 + lane < total ? e0 + lane : total - 1;
+                const int m = (int)(e / nq), n = V * (int)(e - (int64_t)m * nq);
+                const bool in = e0 + lane < total && (inv ? inv[m] != 0.0f : !((bad >> m) & 1u));
+#pragma unroll 1
+                for (int i = 0; i < V; ++i) redo_nans(in, m, n + i);
+            }
+        };
+        if (((N | ldy) & 3) == 0 && !(reinterpret_cast<uintptr_t>(y) & 15)) add(Int<4>{});
+        else add(Int<1>{});
+    } else {
+        const int ct = (N + tn - 1) / tn, tiles = (M + tm - 1) / tm * ct, pitch = (N + 255) / 256 * (256 / tn);
+        for (int i = wv; i < tiles; i += waves) {
+            const int rt = i / ct, n0 = (i - rt * ct) * tn;
+            if (!aux[rt * pitch + n0 / tn]) continue;
+            for (int e0 = 0; e0 < tm * tn; e0 += 64) {   // a tile's width divides 64
+                const int m = rt * tm + (e0 + lane) / tn, n = n0 + (e0 + lane) % tn;
+                const bool in = m < M && n < N && (inv ? inv[m] != 0.0f : !((bad >> m) & 1u));
+                redo_nans(in, m, n);
             }
         }
     }
@@ -996,14 +1162,9 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
         while (hit) {
             const int m = m0 + __builtin_ctzll(hit);
             hit &= hit - 1;
-            const float* xr = x + (int64_t)m * K;
             for (int n = wv; n < N; n += waves) {
-                const uint8_t* wr = w + (int64_t)n * weight_row_bytes<QT>(K);
-                double s = 0.0;
-                for (int j = lane; j < K; j += 64) s = __builtin_fma((double)weight_at<QT>(wr, j), (double)xr[j], s);
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
-                if (lane == 0) y[(int64_t)m * ldy + n] = (float)s;
+                const float o = exact_dot<QT>(w + (int64_t)n * row_bytes, x + (int64_t)m * K, K, lane);
+                if (lane == 0) y[(int64_t)m * ldy + n] = o;
             }
         }
     }
@@ -1026,7 +1187,7 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
 // 4096 x 14336 30.3 / 23.8 (1.4 TB/s of W; bound by vector work, about five
 // instructions per weight), 18944 x 3584 30 / 25, Q1_0 8192 x 4096 21 / 17.
 constexpr int kFewUnits = 8;
-constexpr int kFewAside = 128, kFewHead = kFewAside + 2048;   // LDS: factors of the rows, a place for unused writes, x
+constexpr int kFewAside = 256, kFewHead = kFewAside + 2048;   // LDS: factors and limits of the rows, a place for unused writes, x
 
 template <int QT>
 struct FewRaw;                                           // one tile's fields of half a unit
@@ -1058,10 +1219,17 @@ struct FewRaw<kTypeQ10> {
     }
 };
 
+template <int QT>
+__device__ __forceinline__ uint32_t few_scale(const FewRaw<QT>& r) {
+    if constexpr (kK4<QT>) return r.hd[0];
+    else return r.d;
+}
+
 template <int QT, int MT>
 __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                    float* __restrict__ y, int M, int N, int K, int units, int64_t ldy,
-                                                   int S, float* __restrict__ part, uint32_t* __restrict__ flags) {
+                                                   int S, float* __restrict__ part, float* __restrict__ lim,
+                                                   uint32_t* __restrict__ aux) {
     constexpr int kHalf = 8192 + (kK4<QT> ? 1024 : 0);   // pairs and sums of 16 rows x 128 k
     constexpr int kUnitBytes = (int)weight_row_bytes<QT>(kUnit);
     constexpr int DEPTH = QT == kTypeQ5K ? 2 : 3;        // units of W in flight (registers)
@@ -1072,7 +1240,7 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
     const int id = (xcd < gr ? xcd * (gq + 1) : gr * (gq + 1) + (xcd - gr) * gq) + ((int)blockIdx.x >> 3);
     const int ntiles = (N + 255) / 256, n0 = id % ntiles * 256, split = id / ntiles;
     const int u0 = (int)((int64_t)split * units / S), u1 = (int)((int64_t)(split + 1) * units / S), U = u1 - u0;
-    float* inv = reinterpret_cast<float*>(lds);          // of the 16 MT rows
+    float *inv = reinterpret_cast<float*>(lds), *row_lim = inv + 32;   // of the 16 MT rows
     uint8_t* xl = lds + kFewHead;
 
     const uint8_t* wtile = w + (int64_t)n0 * weight_row_bytes<QT>(K);
@@ -1093,7 +1261,7 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
     // l's pieces l, l + 64, ...; past the range or the row its last elements,
     // made zeros below
     constexpr int NC = kFewUnits / MT / 2;               // 32 pieces of eight per unit
-    const int kleft = K - u0 * kUnit, lim = (U * kUnit < kleft ? U * kUnit : kleft) - 4;
+    const int kleft = K - u0 * kUnit, last = (U * kUnit < kleft ? U * kUnit : kleft) - 4;
     f32x4 xva[MT][NC], xvb[MT][NC];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -1104,8 +1272,8 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
             const int p = lane + 64 * j;
             int ra, rb;
             Order<QT>::runs(p >> 3, (p >> 1) & 3, p & 1, ra, rb);
-            xva[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(ra < lim ? ra : lim));
-            xvb[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(rb < lim ? rb : lim));
+            xva[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(ra < last ? ra : last));
+            xvb[mt][j] = ld<f32x4>(xr, 4u * (uint32_t)(rb < last ? rb : last));
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1122,8 +1290,8 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                 const int p = lane + 64 * j;
                 int ra, rb;
                 Order<QT>::runs(p >> 3, (p >> 1) & 3, p & 1, ra, rb);
-                if (ra > lim) xa[j] = f32x4{};
-                if (rb > lim) xb[j] = f32x4{};
+                if (ra > last) xa[j] = f32x4{};
+                if (rb > last) xb[j] = f32x4{};
             }
             uint32_t big = 0;
 #pragma unroll
@@ -1134,7 +1302,6 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
             int e;
             bool ok = row_scale(big, e);
             const float scale = ok ? ldexpf(1.0f, e) : 0.0f;
-            float body = 0.0f;
 #pragma unroll
             for (int j = 0; j < NC; ++j) {
                 if (2 * j >= U) break;                   // uniform; an odd last unit's pair writes zeros beyond it
@@ -1146,7 +1313,7 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                 float v[8];
                 Order<QT>::order(a, b, v);
                 u32x4 hi, lo;
-                split8(v, hi, lo, body);
+                split8(v, hi, lo);
                 uint8_t* half = xl + (size_t)((st >> 1) * MT + mt) * kHalf;
                 uint8_t* fp = half + 2 * i * 1024 + (wave + 16 * qq) * 16;
                 *reinterpret_cast<u32x4*>(fp) = hi;
@@ -1160,23 +1327,27 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                 }
                 __builtin_amdgcn_sched_barrier(0);       // one piece at a time: registers
             }
-            body = wave_sum(body);
-            if ((float)(U * kUnit) > 2.0f * body) {      // wave-uniform
-                float err = 0.0f;
+            uint32_t small = ~0u;
 #pragma unroll
-                for (int j = 0; j < NC; ++j)
-                    if (2 * j < U) err += lost4(xa[j] * scale) + lost4(xb[j] * scale);
-                ok = ok && wave_sum(err) <= 0x1p-24f * body;
+            for (int j = 0; j < NC; ++j) small = least(least(small, xa[j]), xb[j]);
+            float lost = 0.0f;
+            if (ok && __ballot(below(small, e))) {       // wave-uniform
+#pragma unroll
+                for (int j = 0; j < NC; ++j) lost += lost4(xa[j], scale) + lost4(xb[j], scale);
+                lost = wave_sum(lost);
             }
             if (lane == 0) {
                 inv[m] = ok ? ldexpf(1.0f, -e) : 0.0f;
-                if (n0 == 0) flags[32 * split + m] = ok ? 0u : 1u;
+                row_lim[m] = ok ? ldexpf(lost, 19 - e) : __builtin_inff();
+                if (n0 == 0) lim[32 * split + m] = row_lim[m];
             }
         }
     }
     __syncthreads();
 
-    f32x4 acc[MT][2] = {};
+    typedef f32x4 Sum;
+    Sum acc[MT][2] = {};
+    float dmax = 0.0f;                                   // the largest |d| of the lane's rows of W
     const PairDecode dec(4 * kh + q);                    // this lane's sub-block
     const int qs = 2 * (2 * kh + (q >> 1));              // the fifth bits of its pair
     auto compute = [&](const FewRaw<QT> (&r)[2], int u) __attribute__((always_inline)) {
@@ -1186,13 +1357,14 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
         float sc[2];
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
+            dmax = fmaxf(dmax, fabsf(f16_bits_to_f32(few_scale(r[nt]))));
             if constexpr (kK4<QT>) {
                 uint32_t s, mn;
                 dec(r[nt].hd[1], r[nt].hd[2], r[nt].hd[3], s, mn);
-                K4Stage ks;
+                K4Stage<14> ks;
                 ks.template set<QT, true>(r[nt].hd, s, mn, q & 1);
                 bu[nt] = __builtin_bit_cast(bf16x8, ks.uf);
-                sc[nt] = K4Stage::scale(r[nt].hd);
+                sc[nt] = K4Stage<14>::scale(r[nt].hd);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const uint32_t v = r[nt].v[i], v8 = v >> 8;
@@ -1209,13 +1381,13 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                     b[nt][i] = __builtin_bit_cast(f16x8, f);
                 }
             } else {
-                sc[nt] = -f16_bits_to_f32(r[nt].d);      // codes negated, as in Body<kTypeQ10>
+                sc[nt] = f16_bits_to_f32(r[nt].d) * -4096.0f;   // codes negated and 2^-12, as in Body<kTypeQ10>
                 static_for<0, 4>([&](auto ic) {
                     constexpr int I = decltype(ic)::value;
                     u32x4 f;
                     static_for<0, 4>([&](auto jc) {
                         constexpr int j = decltype(jc)::value;
-                        f[j] = ((r[nt].v << (15 - 4 * I - j)) & 0x80008000u) | 0x3C003C00u;
+                        f[j] = ((r[nt].v << (15 - 4 * I - j)) & 0x80008000u) | kSignCode;
                     });
                     b[nt][I] = __builtin_bit_cast(f16x8, f);
                 });
@@ -1225,13 +1397,8 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
         for (int mt = 0; mt < MT; ++mt) {
             const uint8_t* xm = xb + mt * kHalf;
             f32x4 t[2] = {};
-            if constexpr (kK4<QT>) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(xm + 8192);
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bu[nt], t[nt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int pc = 1; pc >= 0; --pc)              // lo, then hi
+            for (int pc = 1; pc >= 0; --pc) {            // lo, then hi
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const f16x8 a = *reinterpret_cast<const f16x8*>(xm + (2 * i + pc) * 1024);
@@ -1239,10 +1406,22 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                     for (int nt = 0; nt < 2; ++nt)
                         t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[nt][i], t[nt], 0, 0, 0);
                 }
+                if (pc) {                                // the same codes for both here: eight sums, 32 pairs of codes
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                        for (int r4 = 0; r4 < 4; ++r4) t[nt][r4] *= 0x1p-12f;
+                    if constexpr (kK4<QT>) {
+                        const bf16x8 a = *reinterpret_cast<const bf16x8*>(xm + 8192);
+#pragma unroll
+                        for (int nt = 0; nt < 2; ++nt) t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bu[nt], t[nt], 0, 0, 0);
+                    }
+                }
+            }
 #pragma unroll
             for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4) acc[mt][nt][r4] = __builtin_fmaf(sc[nt], t[nt][r4], acc[mt][nt][r4]);
+                for (int r4 = 0; r4 < 4; ++r4) acc[mt][nt][r4] = add_scaled(sc[nt], t[nt][r4], acc[mt][nt][r4]);
         }
     };
     int u = u0;
@@ -1259,74 +1438,99 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
     });
 
     // the second half's sums through LDS (x is done with), then out
-    float f[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) f[mt][r] = inv[16 * mt + 4 * q + r];
     __syncthreads();
     f32x4* red = reinterpret_cast<f32x4*>(xl) + wn * MT * 2 * 64 + lane;
+    float* dred = reinterpret_cast<float*>(lds + kFewAside) + wn * 16 + c;
     if (kh == 1) {
+        if (q == 0) *dred = dmax;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int nt = 0; nt < 2; ++nt) {
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) red[(2 * mt + nt) * 64] = acc[mt][nt];
+            for (int mt = 0; mt < MT; ++mt) red[(2 * mt + nt) * 64] = __builtin_convertvector(acc[mt][nt], f32x4);
+        }
     }
     __syncthreads();
     if (kh == 1) return;
     float* out = S == 1 ? y : part + (int64_t)split * M * N;
     const int64_t ldo = S == 1 ? ldy : N;
+    const float dm = fmaxf(dmax, *dred) * kMaxCode<QT>;
+    uint32_t redo = 0;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int nt = 0; nt < 2; ++nt) {
+        const int n = n0 + 32 * wn + 16 * nt + c;
+        if (S > 1 && q == 0 && n < N) aux[split * N + n] = __float_as_uint(dm);
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            const f32x4 v = acc[mt][nt] + red[(2 * mt + nt) * 64];
-            const int n = n0 + 32 * wn + 16 * nt + c;
+        for (int mt = 0; mt < MT; ++mt) {
+            const f32x4 v = __builtin_convertvector(acc[mt][nt] + __builtin_convertvector(red[(2 * mt + nt) * 64], Sum), f32x4);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = 16 * mt + 4 * q + r;
-                if (m < M && n < N) out[(int64_t)m * ldo + n] = v[r] * f[mt][r];
+                float o = v[r] * inv[m];
+                if (S == 1 && !stands(o, row_lim[m] * dm)) {   // as in gemm_pair_kernel
+                    o = __builtin_nanf("");
+                    redo |= m < M && n < N;
+                }
+                if (m < M && n < N) out[(int64_t)m * ldo + n] = o;
             }
         }
+    }
+    if (S == 1) {
+        const bool any = __ballot(redo) != 0;
+        if (lane == 0) aux[n0 / 32 + wn] = any;
+    }
+}
+
+template <int QT>
+void finish_go(const PairPlan& p, const float* part, const float* inv, const float* lim, const uint32_t* aux, int tm,
+               int tn, const uint8_t* w, const float* x, float* y, int64_t ldy, hipStream_t s) {
+    const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
+    finish_kernel<QT><<<dim3((unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work)), dim3(256), 0, s>>>(
+        part, y, p.splits, (int)p.m, (int)p.n, ldy, inv, lim, aux, tm, tn, w, x, (int)p.k);
 }
 
 template <int QT, int WM, int WN, int MT, int NT, int DEPTH>
-void pair_go(const PairPlan& p, const uint8_t* w, float* y, int64_t ldy, hipStream_t s, uint8_t* scratch) {
+void pair_go(const PairPlan& p, const uint8_t* w, const float* x, float* y, int64_t ldy, hipStream_t s,
+             uint8_t* scratch) {
     const int64_t ntiles = (p.n + 32 * WN * NT - 1) / (32 * WN * NT), mtiles = (p.m + 32 * WM * MT - 1) / (32 * WM * MT);
+    const float *inv = reinterpret_cast<const float*>(scratch), *lim = reinterpret_cast<const float*>(scratch + p.lim_off);
+    float* part = reinterpret_cast<float*>(scratch + p.part_off);
+    uint32_t* aux = reinterpret_cast<uint32_t*>(scratch + p.aux_off);
     gemm_pair_kernel<QT, WM, WN, MT, NT, DEPTH><<<dim3((unsigned)(ntiles * mtiles * p.splits)), dim3(512), 0, s>>>(
-        w, scratch + p.x_off, scratch + p.sum_off, reinterpret_cast<const float*>(scratch), y, (int)p.m, (int)p.n,
-        (int)p.k, (int)p.units, ldy, p.splits, reinterpret_cast<float*>(scratch + p.part_off));
+        w, scratch + p.x_off, scratch + p.sum_off, inv, lim, y, (int)p.m, (int)p.n, (int)p.k, (int)p.units, ldy, p.splits,
+        part, aux);
+    finish_go<QT>(p, part, inv, lim, aux, 32 * MT, 32 * NT, w, x, y, ldy, s);
 }
 
 // Few rows: 1024 threads each, for latency; more: enough threads that every
 // one holds two to five pieces of the row in registers.
 template <int QT, int RW, int TPR, int NC>
-void split_launch(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv) {
+void split_launch(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv, float* lim) {
     const unsigned grid = (unsigned)((p.m + 63) / 64 * 64 / RW);
-    split_kernel<QT, RW, TPR, NC><<<dim3(grid), dim3(RW * TPR), 0, s>>>(x, (int)p.m, (int)p.k, (int)p.units, xf, xsum, inv);
+    split_kernel<QT, RW, TPR, NC><<<dim3(grid), dim3(RW * TPR), 0, s>>>(x, (int)p.m, (int)p.k, (int)p.units, xf, xsum, inv,
+                                                                                lim);
 }
 template <int QT>
-void split_go(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv) {
+void split_go(const PairPlan& p, const float* x, hipStream_t s, uint8_t* xf, uint8_t* xsum, float* inv, float* lim) {
     const int64_t chunks = p.units * 32;
     if (p.m <= 64 && chunks > 512) {
-        if (chunks <= 1024) return split_launch<QT, 1, 1024, 1>(p, x, s, xf, xsum, inv);
-        if (chunks <= 2048) return split_launch<QT, 1, 1024, 2>(p, x, s, xf, xsum, inv);
-        if (chunks <= 3072) return split_launch<QT, 1, 1024, 3>(p, x, s, xf, xsum, inv);
+        if (chunks <= 1024) return split_launch<QT, 1, 1024, 1>(p, x, s, xf, xsum, inv, lim);
+        if (chunks <= 2048) return split_launch<QT, 1, 1024, 2>(p, x, s, xf, xsum, inv, lim);
+        if (chunks <= 3072) return split_launch<QT, 1, 1024, 3>(p, x, s, xf, xsum, inv, lim);
     }
-    if (chunks <= 256) return split_launch<QT, 4, 128, 2>(p, x, s, xf, xsum, inv);
-    if (chunks <= 512) return split_launch<QT, 2, 256, 2>(p, x, s, xf, xsum, inv);
-    if (chunks <= 1024) return split_launch<QT, 2, 256, 4>(p, x, s, xf, xsum, inv);
-    if (chunks <= 2560) return split_launch<QT, 1, 512, 5>(p, x, s, xf, xsum, inv);
-    split_launch<QT, 1, 1024, 0>(p, x, s, xf, xsum, inv);
+    if (chunks <= 256) return split_launch<QT, 4, 128, 2>(p, x, s, xf, xsum, inv, lim);
+    if (chunks <= 512) return split_launch<QT, 2, 256, 2>(p, x, s, xf, xsum, inv, lim);
+    if (chunks <= 1024) return split_launch<QT, 2, 256, 4>(p, x, s, xf, xsum, inv, lim);
+    if (chunks <= 2560) return split_launch<QT, 1, 512, 5>(p, x, s, xf, xsum, inv, lim);
+    split_launch<QT, 1, 1024, 0>(p, x, s, xf, xsum, inv, lim);
 }
 
 template <int QT>
 void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int64_t ldy, hipStream_t s,
               uint8_t* scratch, bool x_ready) {
-    float* inv = reinterpret_cast<float*>(scratch);
+    float *inv = reinterpret_cast<float*>(scratch), *lim = reinterpret_cast<float*>(scratch + p.lim_off);
     if constexpr (QT != kTypeQ6K) {
         if (p.few) {
-            uint32_t* flags = reinterpret_cast<uint32_t*>(scratch);
+            uint32_t* aux = reinterpret_cast<uint32_t*>(scratch + p.aux_off);
             float* part = reinterpret_cast<float*>(scratch + p.part_off);
             const unsigned grid = (unsigned)((p.n + 255) / 256 * p.splits);
             const int mt = p.m <= 16 ? 1 : 2;
@@ -1336,27 +1540,20 @@ void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int
             const unsigned ldsb = kFewHead + (bytes > red ? bytes : red);
             if (mt == 1)
                 few_kernel<QT, 1><<<dim3(grid), dim3(1024), ldsb, s>>>(w, x, y, (int)p.m, (int)p.n, (int)p.k,
-                                                                       (int)p.units, ldy, p.splits, part, flags);
+                                                                       (int)p.units, ldy, p.splits, part, lim, aux);
             else
                 few_kernel<QT, 2><<<dim3(grid), dim3(1024), ldsb, s>>>(w, x, y, (int)p.m, (int)p.n, (int)p.k,
-                                                                       (int)p.units, ldy, p.splits, part, flags);
-            const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
-            finish_kernel<QT><<<dim3((unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work)), dim3(256), 0, s>>>(
-                part, y, p.splits, (int)p.m, (int)p.n, ldy, nullptr, flags, w, x, (int)p.k);
-            return;
+                                                                       (int)p.units, ldy, p.splits, part, lim, aux);
+            return finish_go<QT>(p, part, nullptr, lim, aux, 16 * mt, 32, w, x, y, ldy, s);
         }
     }
-    if (!x_ready) split_go<QT>(p, x, s, scratch + p.x_off, scratch + p.sum_off, inv);
+    if (!x_ready) split_go<QT>(p, x, s, scratch + p.x_off, scratch + p.sum_off, inv, lim);
     if (p.bm == 32)
-        pair_go<QT, 1, 8, 1, 1, 2>(p, w, y, ldy, s, scratch);
+        pair_go<QT, 1, 8, 1, 1, 2>(p, w, x, y, ldy, s, scratch);
     else if (p.bm == 64)
-        pair_go<QT, 1, 8, 2, 1, QT == kTypeQ10 ? 2 : 1>(p, w, y, ldy, s, scratch);
+        pair_go<QT, 1, 8, 2, 1, QT == kTypeQ10 ? 2 : 1>(p, w, x, y, ldy, s, scratch);
     else if constexpr (QT == kTypeQ4K || QT == kTypeQ6K)
-        pair_go<QT, 2, 4, 2, 2, 1>(p, w, y, ldy, s, scratch);
-    const int64_t work = p.splits > 1 ? (p.m * p.n + 1023) / 1024 : 0;
-    const unsigned fin = (unsigned)(work < 256 ? 256 : work > 2048 ? 2048 : work);
-    finish_kernel<QT><<<dim3(fin), dim3(256), 0, s>>>(reinterpret_cast<const float*>(scratch + p.part_off), y,
-                                                      p.splits, (int)p.m, (int)p.n, ldy, inv, nullptr, w, x, (int)p.k);
+        pair_go<QT, 2, 4, 2, 2, 1>(p, w, x, y, ldy, s, scratch);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -1392,13 +1589,16 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
     for (int c = 0; c < 2; ++c) {
         const int bm = bms[c];
         const int64_t mtiles = (m + bm - 1) / bm, mpad = mtiles * bm;
-        const size_t sum_off = align256((size_t)mpad * 4), x_off = sum_off + (k4 ? (size_t)(mpad / 32 * p->units) * 4096 : 0);
+        const size_t lim_off = (size_t)mpad * 4, sum_off = align256(2 * lim_off);
+        const size_t x_off = sum_off + (k4 ? (size_t)(mpad / 32 * p->units) * 4096 : 0);
         const size_t part_off = x_off + (size_t)mpad * (size_t)p->units * kUnit * 4;
         if (part_off > cap) continue;
         const double unit_us = bm == 32 ? 2.9 : bm == 64 ? 3.9 : qtype == kTypeQ6K ? 9.0 : 7.0, start_us = 6.0;
         for (int64_t s = 1; s <= 64 && s <= p->units; ++s) {
-            const size_t bytes = s > 1 ? (size_t)s * (size_t)m * (size_t)n * 4 : 0;
-            if (part_off + bytes > cap) break;
+            // the planes and the largest scales [s][n], or a word per wave of every tile
+            const size_t planes = s > 1 ? align256((size_t)s * (size_t)m * (size_t)n * 4) : 0;
+            const size_t aux = s > 1 ? (size_t)s * (size_t)n * 4 : (size_t)(mtiles * ntiles) * 8 * 4;
+            if (part_off + planes + aux > cap) break;
             const double rounds = (double)((mtiles * ntiles * s + 255) / 256);
             const double us = rounds * (start_us + (double)((p->units + s - 1) / s) * unit_us) + (s > 1 ? s * plane_us + 1.0 : 0.0);
             if (!found || us < best) {
@@ -1406,9 +1606,12 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
                 best = us;
                 p->bm = bm;
                 p->splits = (int)s;
+                p->lim_off = lim_off;
                 p->sum_off = sum_off;
                 p->x_off = x_off;
                 p->part_off = part_off;
+                p->aux_off = part_off + planes;
+                p->bytes = p->aux_off + aux;
             }
         }
     }
@@ -1428,21 +1631,21 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
         fs = (p->units + share - 1) / share;             // as few splits as give that share
         const double few_us = 7.0 + (double)((ntiles * fs + 255) / 256) * (6.0 + (double)share * (m <= 16 ? 2.2 : 3.0));
         const size_t part_off = align256((size_t)fs * 32 * 4);
-        const size_t bytes = part_off + (fs > 1 ? (size_t)fs * (size_t)m * (size_t)n * 4 : 0);
+        const size_t aux_off = part_off + (fs > 1 ? align256((size_t)fs * (size_t)m * (size_t)n * 4) : 0);
+        const size_t bytes = aux_off + (fs > 1 ? (size_t)fs * (size_t)n * 4 : (size_t)ntiles * 8 * 4);
         if (bytes <= cap && fs * ntiles <= 0x7FFFFFFF && (!found || few_us < best + 6.0)) {
             p->few = true;
             p->splits = (int)fs;
             p->bm = 32;
             p->layout = 0;                               // nothing that another launch could use
-            p->sum_off = p->x_off = 0;
+            p->lim_off = p->sum_off = p->x_off = 0;
             p->part_off = part_off;
+            p->aux_off = aux_off;
             p->bytes = bytes;
             return true;
         }
     }
-    if (!found) return false;
-    p->bytes = p->part_off + (p->splits > 1 ? (size_t)p->splits * (size_t)m * (size_t)n * 4 : 0);
-    return true;
+    return found;
 }
 
 hipError_t launch_gemm_pair(int qtype, const uint8_t* w, const float* x, float* y, int64_t ldy, const PairPlan& p,

@@ -230,9 +230,9 @@ hipError_t launch_gemm_f32(int qtype, const uint8_t* w, const float* x, float* y
 // (frq_gemm_pair.hip): y[m, n] = x[m, k] . W[n, k]^T for raw Q4_K, Q5_K, Q6_K
 // or Q1_0 blocks, rows of y ldy >= n floats apart; x 16-byte aligned, w
 // 16-byte (Q4_K, Q5_K) / 2-byte aligned. At most kPairRows rows a launch.
-// `scratch` (p.bytes, 256-byte aligned) holds the row factors, the sub-block
-// sums, the pairs and the partial planes of a split k; launches sharing it must
-// be ordered. With x_ready the first three are those of an earlier launch of the same x,
+// `scratch` (p.bytes, 256-byte aligned) holds the row factors and limits, the
+// sub-block sums, the pairs, the partial planes of a split k and marks for the
+// last kernel; launches sharing it must be ordered. With x_ready the first three are those of an earlier launch of the same x,
 // m, k, p.layout and p.bm on the same scratch. The plan is a function of its
 // arguments only; false where it does not fit `cap` bytes.
 constexpr int64_t kPairRows = 1024;
@@ -240,7 +240,7 @@ struct PairPlan {
     int64_t m = 0, n = 0, k = 0, units = 0;
     int bm = 0, bn = 0, splits = 1, layout = 0;
     bool few = false;       // up to 32 rows: the one-launch kernel, which shares nothing
-    size_t sum_off = 0, x_off = 0, part_off = 0, bytes = 0;
+    size_t lim_off = 0, sum_off = 0, x_off = 0, part_off = 0, aux_off = 0, bytes = 0;
 };
 bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, PairPlan* p);
 hipError_t launch_gemm_pair(int qtype, const uint8_t* w, const float* x, float* y, int64_t ldy, const PairPlan& p,

@@ -167,14 +167,14 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  * time, by one of two fp32-contract GEMMs:
  *   Q4_K, Q5_K, Q6_K, Q1_0 (frq_gemm_pair.hip): fp16 matrix cores on exact
  * integer codes (Q4_K / Q5_K sc q - R with R the integer nearest dmin*m / d,
- * so every term stays within 3 |w_j x_j|) and on x as hi + lo, two fp16 values
- * under a power of two per row of x (up to 32 rows of Q4_K, Q5_K and Q1_0: per
- * row and range of k, which a workgroup sums): every element down to 2^-16 of the row's
- * largest to within 2^-23 of itself, smaller ones to within 2^-40 of the
- * largest. A row whose elements that loses more than 2^-24 of its sum |x|
- * (outliers capped at 2^-10 of the largest), or with an inf, a NaN or a largest
- * |x| outside [2^-100, 2^101), is computed weight by weight in fp64 (one
- * rounding; inf and NaN as IEEE arithmetic has them).
+ * so every term stays within 3 |w_j x_j|) and on x as hi + lo 2^-12, two fp16
+ * values under a power of two per row of x (up to 32 rows of Q4_K, Q5_K and
+ * Q1_0: per row and range of k, which a workgroup sums): every element down to
+ * 2^-28 of the row's largest to within 2^-23 of itself, down to 2^-32 to within
+ * 2^-19, smaller ones to within 2^-51 of the largest. An output that the last
+ * ones could take beyond the bound (it hangs on them alone), is computed
+ * weight by weight in fp64, as is a row with an inf, a NaN or a largest |x|
+ * outside [2^-100, 2^101) (one rounding; inf and NaN as IEEE arithmetic has them).
  *   Q8_0, small Q4_K and Q6_K matrices (n k < 24 M; Q4_K up to 64 rows), and
  * Q4_K / Q6_K where the former's scratch cannot be had (frq_gemm_f32.hip): x as
  * three bf16 pieces (all 24 bits of every x in {0} U [2^-100, 2^100]); rows

@@ -3,9 +3,9 @@ oracle, at the sizes where its tiles, units and splits end.
 
 Rows around the 32-, 64- and 128-row tiles, columns around the 256-column tile
 (one wave, one lane short of it), rows of W from one block to several units
-with a remainder in every split, each format, and rows of x that the pairs do
-not carry (outliers far above the rest, non-finite values), which are computed
-weight by weight. The bound is the matvec's: 1e-5 of sum |w_j x_j| per output
+with a remainder in every split, each format, and what the pairs do not carry
+and is computed weight by weight: rows of x with non-finite values, outputs that
+hang on x far below their row's largest. The bound is the matvec's: 1e-5 of sum |w_j x_j| per output
 and of max |y| per row (conftest.assert_matvec_close).
 """
 
@@ -84,6 +84,59 @@ def test_rows_beyond_the_pairs(frq, q, n, k, rows):
         assert np.all(err[ok] <= bound[ok]), r
     assert not np.any(np.isfinite(y[6][W[:, 11] != 0])) and np.all(np.isnan(y[7]))
     assert bits_equal(y[8:], run(q, raw, calm, n, k)[8:])
+
+
+def zero_weights(q, raw, n, k, keep):
+    """raw with every weight zero but, in the rows `keep[i]` true, those of one
+    sub-block (Q1_0: block) near the middle of the row; where that is in the row."""
+    nb, b0 = k // G.BLOCK[q][1], k // G.BLOCK[q][1] // 2
+    r = raw.reshape(n, nb, -1).copy()
+    if q == "Q1_0":
+        r[:, :b0, :2] = r[:, b0 + 1:, :2] = 0
+        r[~keep, b0, :2] = 0
+        return r.reshape(-1), slice(b0 * 128, b0 * 128 + 128)
+    sc = slice(4, 16) if q in ("Q4_K", "Q5_K") else slice(192, 208)
+    one = r[:, b0, sc].copy()
+    r[:, :, sc] = 0
+    if q == "Q6_K":
+        r[:, b0, 197] = np.where(one[:, 5] == 0, 9, one[:, 5])     # elements 80 .. 95
+        r[~keep, b0, 197] = 0
+        return r.reshape(-1), slice(b0 * 256 + 80, b0 * 256 + 96)
+    r[:, b0, 6] = (one[:, 2] & 63) | 1                             # sub-block 2's scale and minimum
+    r[:, b0, 10] = one[:, 6] & 63
+    r[~keep, b0, sc] = 0
+    return r.reshape(-1), slice(b0 * 256 + 64, b0 * 256 + 96)
+
+
+@pytest.mark.parametrize("q,n,k,rows,plan", [
+    ("Q4_K", 8192, 4096, 16, ("few", 32, 8)), ("Q5_K", 14336, 4096, 20, ("few", 32, 4)),
+    ("Q1_0", 8192, 4096, 9, ("few", 32, 8)), ("Q5_K", 65537, 512, 9, ("few", 32, 1)),
+    ("Q5_K", 70, 4096, 9, ("pair", 32, 16)), ("Q6_K", 66000, 512, 11, ("pair", 32, 1)),
+    ("Q4_K", 70, 2048, 66, ("pair", 64, 8)), ("Q6_K", 1500, 16384, 40, ("pair", 64, 32)),
+    ("Q1_0", 65600, 512, 40, ("pair", 64, 1)), ("Q4_K", 33000, 1024, 66, ("pair", 128, 1)),
+    ("Q6_K", 33000, 1024, 66, ("pair", 128, 1)),
+])
+def test_small_x_beside_large_on_zero_weights(frq, q, n, k, rows, plan):
+    """x of a row 2^-15 to 2^-80 below its largest decide outputs whose other
+    weights are all zero: the bound is componentwise, so what the row's scale
+    costs them counts; dense rows of W and rows that are zero stay as they are."""
+    assert device.batch_plan(q, n, k, rows)[:3] == plan
+    dense = synth.make_blocks(q, n, k, seed=n + k)
+    rng = np.random.default_rng(n)
+    pick = np.sort(rng.choice(n, min(n, 40), replace=False))
+    thin, at = zero_weights(q, dense, n, k, np.arange(n) % 3 != 0)
+    raw = dense.reshape(n, -1)
+    raw[pick] = thin.reshape(n, -1)[pick]
+    raw = raw.reshape(-1)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    for r in range(rows):
+        xs[r, at] *= np.float32(2.0 ** -(15 + 5 * (r % 14)))
+    y = run(q, raw, xs, n, k)
+    some = np.unique(np.r_[pick, rng.choice(n, min(n, 60), replace=False)])
+    part = np.ascontiguousarray(raw.reshape(n, -1)[some]).reshape(-1)
+    y64, a64 = G.matmul_f64(q, xs, part, some.size, k), G.abs_matmul_f64(q, xs, part, some.size, k)
+    for r in range(rows):
+        assert_matvec_close(y[r, some], y64[r], a64[r], what=f"{q} {n}x{k} row {r}")
 
 
 def test_group_shares_the_pairs(frq):
