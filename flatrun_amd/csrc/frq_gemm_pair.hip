@@ -34,7 +34,8 @@
 // beside 1e2) is added up per row; times the largest weight of a row of W that
 // bounds what an output lost. It only counts where the weights of all the larger
 // x are zero or nearly so, that is in an output that small itself: an output
-// below 2^19 of that bound is computed weight by weight in fp64 too.
+// below 2^19 of that bound, and one that is not finite (a scale of W may not
+// be), is computed weight by weight in fp64 too.
 //
 // Tiling: BM x BN of Y per workgroup; a wave owns 32 MT x 32 NT. W goes from
 // memory to registers to the matrix cores (lane = one row of W; both halves
@@ -90,8 +91,8 @@ constexpr uint32_t kSignCode = 0x0C000C00u;   // +2^-12 twice
 // what its pairs miss) times this and the largest |d| of a row of W.
 template <int QT>
 constexpr float kMaxCode = QT == kTypeQ4K ? 63.0f * 15.0f : QT == kTypeQ5K ? 63.0f * 31.0f : QT == kTypeQ6K ? 4096.0f : 1.0f;
-// Whether an output stands as computed.
-__device__ __forceinline__ bool stands(float y, float limit) { return !(fabsf(y) < limit); }
+// Whether an output stands as computed, |y| not below its limit and finite.
+__device__ __forceinline__ bool stands(float y, float limit) { return !(fabsf(y) < limit) && fabsf(y) < __builtin_inff(); }
 
 __device__ __forceinline__ f16x2 as_f16x2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ uint32_t as_u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }

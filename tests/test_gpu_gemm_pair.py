@@ -5,7 +5,7 @@ Rows around the 32-, 64- and 128-row tiles, columns around the 256-column tile
 (one wave, one lane short of it), rows of W from one block to several units
 with a remainder in every split, each format, and what the pairs do not carry
 and is computed weight by weight: rows of x with non-finite values, outputs that
-hang on x far below their row's largest. The bound is the matvec's: 1e-5 of sum |w_j x_j| per output
+hang on x far below their row's largest, weights with non-finite scales. The bound is the matvec's: 1e-5 of sum |w_j x_j| per output
 and of max |y| per row (conftest.assert_matvec_close).
 """
 
@@ -137,6 +137,42 @@ def test_small_x_beside_large_on_zero_weights(frq, q, n, k, rows, plan):
     y64, a64 = G.matmul_f64(q, xs, part, some.size, k), G.abs_matmul_f64(q, xs, part, some.size, k)
     for r in range(rows):
         assert_matvec_close(y[r, some], y64[r], a64[r], what=f"{q} {n}x{k} row {r}")
+
+
+@pytest.mark.parametrize("q,n,k,rows,plan", [
+    ("Q4_K", 8192, 4096, 16, ("few", 32, 8)), ("Q5_K", 65537, 512, 9, ("few", 32, 1)),
+    ("Q1_0", 8192, 4096, 20, ("few", 32, 8)), ("Q5_K", 300, 2048, 9, ("pair", 32, 8)),
+    ("Q6_K", 66000, 512, 11, ("pair", 32, 1)), ("Q4_K", 70, 2048, 66, ("pair", 64, 8)),
+    ("Q1_0", 65600, 512, 40, ("pair", 64, 1)), ("Q4_K", 33000, 1024, 66, ("pair", 128, 1)),
+])
+def test_scales_that_are_not_finite(frq, q, n, k, rows, plan):
+    """Blocks whose scale (Q4_K, Q5_K: or minimum) is an infinity or a NaN: each
+    output is the infinity or the NaN that the dequantized weights give, whether
+    x has one sign, both or zeros, and the other rows of W are as without them."""
+    assert device.batch_plan(q, n, k, rows)[:3] == plan
+    bad = synth.make_blocks(q, n, k, seed=n).reshape(n, k // G.BLOCK[q][1], -1)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    xs[0::3] = np.abs(xs[0::3])
+    xs[1::3] = -np.abs(xs[1::3])
+    xs[2, ::2] = 0.0
+    clean = run(q, bad.reshape(-1), xs, n, k)
+    at = {"Q6_K": (208,), "Q1_0": (0,)}.get(q, (0, 2))
+    hit = []
+    for i, (off, bits) in enumerate((o, b) for o in at for b in (0x7C00, 0xFC00, 0x7E00)):
+        row, blk = (7 + 41 * i) % n, (3 * i) % bad.shape[1]
+        if q == "Q6_K":
+            bad[row, blk, :192], bad[row, blk, 192:208] = 0, 5      # codes -32
+        if q == "Q1_0":
+            bad[row, blk, 2:] = 255
+        bad[row, blk, off:off + 2] = (bits & 255, bits >> 8)
+        hit.append(row)
+    y = run(q, bad.reshape(-1), xs, n, k)
+    with np.errstate(invalid="ignore"):
+        want = G.matmul_f64(q, xs, np.ascontiguousarray(bad[hit]).reshape(-1), len(hit), k)
+    assert np.isinf(want).any() and np.isnan(want).any() and not np.isfinite(want).all(axis=0).any()
+    assert np.array_equal(y[:, hit], want.astype(np.float32), equal_nan=True)
+    rest = np.setdiff1d(np.arange(n), hit)
+    assert bits_equal(y[:, rest], clean[:, rest])
 
 
 def test_group_shares_the_pairs(frq):
