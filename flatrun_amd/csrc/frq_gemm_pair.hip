@@ -1044,14 +1044,70 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
     if (lane == 0) aux[(mt0 / MT + wm) * (ntiles * WN) + n0 / (32 * NT) + wn] = any;
 }
 
-// A row of x times one of W by a wave in fp64, the sum in every lane.
+// Weights j .. j + 7 (j a multiple of eight) of a row, weight_at's bits.
 template <int QT>
-__device__ __forceinline__ float exact_dot(const uint8_t* __restrict__ wr, const float* __restrict__ xr, int K, int lane) {
-    double s = 0.0;
-    for (int j = lane; j < K; j += 64) s = __builtin_fma((double)weight_at<QT>(wr, j), (double)xr[j], s);
+__device__ __forceinline__ void weights8(const uint8_t* __restrict__ wrow, int j, float (&v)[8]) {
+    if constexpr (kK4<QT>) {
+        const uint8_t* bp = wrow + (int64_t)(j >> 8) * (QT == kTypeQ4K ? kQ4KBytes : kQ5KBytes);
+        const int sb = (j >> 5) & 7, l = j & 31;
+        const uint4 h = *reinterpret_cast<const uint4*>(bp);
+        const u32x2 q = *reinterpret_cast<const u32x2*>(bp + (QT == kTypeQ4K ? 16 : 48) + 32 * (sb >> 1) + l);
+        u32x2 qh = {};
+        if constexpr (QT == kTypeQ5K) qh = *reinterpret_cast<const u32x2*>(bp + 16 + l);
+        uint32_t sc, mn;
+        k4_scale_min(h.y, h.z, h.w, sb, sc, mn);
+        const float s = f16_bits_to_f32(h.x) * (float)sc, t = f16_bits_to_f32(h.x >> 16) * (float)mn;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
-    return (float)s;
+        for (int i = 0; i < 8; ++i) {
+            uint32_t c = (q[i >> 2] >> (8 * (i & 3) + 4 * (sb & 1))) & 15u;
+            if constexpr (QT == kTypeQ5K) c |= ((qh[i >> 2] >> (8 * (i & 3) + sb)) & 1u) << 4;
+            v[i] = s * (float)c - t;
+        }
+    } else if constexpr (QT == kTypeQ6K) {
+        const uint8_t* bp = wrow + (int64_t)(j >> 8) * kQ6KBytes;
+        const int e = j & 255, hh = e >> 7, ks = (e >> 5) & 3, l = e & 31;
+        const float s = f16_bits_to_f32(ld_u16(bp + 208)) * (float)(int)(int8_t)bp[192 + 8 * hh + (l >> 4) + 2 * ks];
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            const uint32_t ql = ld_u16(bp + 64 * hh + 32 * (ks & 1) + l + i) >> (ks >= 2 ? 4 : 0);
+            const uint32_t qh = ld_u16(bp + 128 + 32 * hh + l + i) >> (2 * ks);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                v[i + b] = s * (float)((int)(((ql >> (8 * b)) & 15u) | (((qh >> (8 * b)) & 3u) << 4)) - 32);
+        }
+    } else {
+        const uint8_t* bp = wrow + (int64_t)(j >> 7) * kQ10Bytes;
+        const float d = f16_bits_to_f32(ld_u16(bp));
+        const uint32_t bits = bp[2 + ((j & 127) >> 3)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (bits >> i) & 1u ? d : -d;
+    }
+}
+
+// R rows of x times one row of W by a wave in fp64, the sums in every lane.
+template <int QT, int R>
+__device__ __forceinline__ void exact_dots(const uint8_t* __restrict__ wr, const float* const (&xr)[R], int K, int lane,
+                                           double (&s)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = 0.0;
+#pragma unroll 1
+    for (int j = 8 * lane; j < K; j += 512) {
+        float v[8];
+        weights8<QT>(wr, j, v);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const f32x4 a = *reinterpret_cast<const f32x4*>(xr[r] + j), b = *reinterpret_cast<const f32x4*>(xr[r] + j + 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[r] = __builtin_fma((double)v[i], (double)a[i], s[r]);
+                s[r] = __builtin_fma((double)v[4 + i], (double)b[i], s[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) s[r] += __shfl_xor(s[r], o, 64);
 }
 
 // S > 1: y = inv * (the planes added in split order, in fp64: free here, and
@@ -1059,7 +1115,7 @@ __device__ __forceinline__ float exact_dot(const uint8_t* __restrict__ wr, const
 // weight by weight in fp64, a wave per row of W over the whole grid:
 //   * rows with inv = 0, or, where every split judged its part of x itself
 //     (few_kernel; inv null, the planes in units of y, at most 32 rows, lim [S][32]),
-//     an infinite lim of any split;
+//     an infinite lim of any split; up to four at a time, W decoded once;
 //   * single outputs that do not stand, marked as NaN: with S > 1 by the planes'
 //     sum and the largest scales that aux [S][N] holds, with S = 1 those in the
 //     tiles of tm x tn outputs (one wave's) that aux marks.
@@ -1083,8 +1139,10 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
         const float v = in ? y[(int64_t)m * ldy + n] : 0.0f;
         for (uint64_t redo = __ballot(v != v); redo; redo &= redo - 1) {
             const int l = __builtin_ctzll(redo), ml = __builtin_amdgcn_readlane(m, l), nl = __builtin_amdgcn_readlane(n, l);
-            const float o = exact_dot<QT>(w + (int64_t)nl * row_bytes, x + (int64_t)ml * K, K, lane);
-            if (lane == l) y[(int64_t)m * ldy + n] = o;
+            const float* xr[1] = {x + (int64_t)ml * K};
+            double s[1];
+            exact_dots<QT, 1>(w + (int64_t)nl * row_bytes, xr, K, lane, s);
+            if (lane == l) y[(int64_t)m * ldy + n] = (float)s[0];
         }
     };
     if (S > 1) {
@@ -1161,11 +1219,22 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
     for (int m0 = 0; m0 < M; m0 += 64) {                // every wave scans all rows
         uint64_t hit = inv ? __ballot(m0 + lane < M && inv[m0 + lane < M ? m0 + lane : 0] == 0.0f) : bad;
         while (hit) {
-            const int m = m0 + __builtin_ctzll(hit);
-            hit &= hit - 1;
+            int m[4];
+            const float* xr[4];
+            int count = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {                // past the last one: it again
+                m[r] = hit ? m0 + __builtin_ctzll(hit) : m[r ? r - 1 : 0];
+                count += hit != 0;
+                hit &= hit - 1;
+                xr[r] = x + (int64_t)m[r] * K;
+            }
             for (int n = wv; n < N; n += waves) {
-                const float o = exact_dot<QT>(w + (int64_t)n * row_bytes, x + (int64_t)m * K, K, lane);
-                if (lane == 0) y[(int64_t)m * ldy + n] = o;
+                double s[4];
+                exact_dots<QT, 4>(w + (int64_t)n * row_bytes, xr, K, lane, s);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (lane == 0 && r < count) y[(int64_t)m[r] * ldy + n] = (float)s[r];
             }
         }
     }

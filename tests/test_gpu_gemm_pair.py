@@ -175,6 +175,17 @@ def test_scales_that_are_not_finite(frq, q, n, k, rows, plan):
     assert bits_equal(y[:, rest], clean[:, rest])
 
 
+@pytest.mark.parametrize("q,n,k,rows,bad", [("Q5_K", 1030, 2048, 9, 9), ("Q1_0", 300, 4224, 70, 67),
+                                            ("Q4_K", 70, 2048, 66, 5), ("Q6_K", 1500, 16384, 40, 6)])
+def test_many_rows_weight_by_weight(frq, q, n, k, rows, bad):
+    """Rows of x below the pairs' range, which are computed several at a time,
+    their number one to three past a multiple of that and beyond 64."""
+    raw = synth.make_blocks(q, n, k, seed=n)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    xs[np.random.default_rng(1).choice(rows, bad, replace=False)] *= np.float32(2.0 ** -110)
+    check(q, raw, xs, n, k, run(q, raw, xs, n, k), q)
+
+
 def test_group_shares_the_pairs(frq):
     """A group whose matrices take both element orders (Q5_K and Q6_K / Q1_0):
     each has the bits it has alone."""
