@@ -18,9 +18,9 @@
 //     codes, scale and centre included.
 //   * the matrix cores sum 64 elements (Q6_K 16, one sub-block) in fp32, then
 //     acc += scale * sum in fp32 (the scale of a Q4_K / Q5_K block alone, since
-//     sc is in the code). With up to 64 rows a wave, acc is added to the result's
-//     accumulator every 256 elements, so that the sums round less often at
-//     full size. Q4_K / Q5_K add -(dmin m - d R) sum(x) per 32-element sub-block
+//     sc is in the code). With up to 64 rows a wave, Q5_K and Q1_0 keep acc in
+//     fp64, and the others add it to the result's accumulator every 256
+//     elements, so that the sums round less often at full size. Q4_K / Q5_K add -(dmin m - d R) sum(x) per 32-element sub-block
 //     on the matrix cores as well: three bf16 pieces of each factor, the six
 //     products down to 2^-24 of their product.
 //   With R the nearest integer, |d (sc q - R)| + |dmin m - d R| <= 3 |w|, so a
@@ -673,8 +673,12 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
 
     constexpr int kE = MT * NT > 2 ? 14 : 2;
     constexpr bool kScaleT = kK4<QT> && MT * NT > 2;
-    constexpr bool kTwo = MT * NT <= 2;                // room for a second level
-    typedef float Sum;
+    // With up to 64 rows a wave there is room for two registers per sum: a second
+    // level in fp32, every 256 elements, or one sum in fp64 for Q5_K and Q1_0, whose
+    // rows one GEMV each would give: 97 rows of Q5_K 14336 x 4096, error against 64
+    // bits 1.12e-7 and 0.89e-7 (one GEMV per row 1.05e-7), 58 and 61 us.
+    constexpr bool kF64 = QT == kTypeQ5K || QT == kTypeQ10, kTwo = !kF64 && MT * NT <= 2;
+    typedef typename std::conditional<kF64, double, float>::type Sum;
     Sum acc[MT][NT][16];
     f32x16 tot[kTwo ? MT : 1][NT], t[2];
 #pragma unroll
@@ -1415,7 +1419,9 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
     }
     __syncthreads();
 
-    typedef f32x4 Sum;
+    // sums in fp64 for Q5_K and Q1_0 (as in gemm_pair_kernel) where the registers
+    // allow: two tiles of Q5_K add at most four units
+    typedef typename std::conditional<(QT == kTypeQ5K && MT == 1) || QT == kTypeQ10, f64x4, f32x4>::type Sum;
     Sum acc[MT][2] = {};
     float dmax = 0.0f;                                   // the largest |d| of the lane's rows of W
     const PairDecode dec(4 * kh + q);                    // this lane's sub-block

@@ -186,6 +186,23 @@ def test_many_rows_weight_by_weight(frq, q, n, k, rows, bad):
     check(q, raw, xs, n, k, run(q, raw, xs, n, k), q)
 
 
+@pytest.mark.parametrize("q,n,k,rows,plan", [
+    ("Q5_K", 8192, 4096, 12, ("few", 32, 8)), ("Q5_K", 4096, 11008, 40, ("pair", 64, 15)),
+    ("Q5_K", 8192, 4096, 97, ("pair", 64, 4)), ("Q1_0", 8192, 4096, 97, ("pair", 64, 4)),
+])
+def test_error_no_larger_than_one_gemv_per_row(frq, q, n, k, rows, plan):
+    """The formats whose rows otherwise run one GEMV each: the batch is no
+    further from 64 bits (2-norms over all outputs; 4 % for the samples')."""
+    assert device.batch_plan(q, n, k, rows)[:3] == plan
+    raw = synth.make_blocks(q, n, k, seed=n + k)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    xs *= np.where(np.random.default_rng(1).random(xs.shape) < 1 / 300, 20, 1).astype(np.float32)
+    y64 = G.matmul_f64(q, xs, raw, n, k)
+    alone = np.stack([run(q, raw, xs[r:r + 1], n, k)[0] for r in range(rows)])
+    err, err_alone = (np.linalg.norm(y - y64) for y in (run(q, raw, xs, n, k), alone))
+    assert err <= 1.04 * err_alone, (err / np.linalg.norm(y64), err_alone / np.linalg.norm(y64))
+
+
 def test_group_shares_the_pairs(frq):
     """A group whose matrices take both element orders (Q5_K and Q6_K / Q1_0):
     each has the bits it has alone."""
