@@ -1634,6 +1634,41 @@ void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// A call's estimated time (us): its launches + rounds of 256 workgroups (one per
+// CU), each a start and a workgroup's units of k, + the planes of a split k,
+// written and read (8 bytes of each output and split, in 3.1 MB). With few CUs
+// busy a unit takes up to 15 % less. The numbers fit 8900 measured calls: every tile of
+// each format at 1 to 64 splits, eleven matrices of 0.5 to 80 M weights, 2 to 512
+// rows, W cold in the caches. The plans chosen take 0.4 % more than the fastest
+// measured ones on average; one unit time for all formats, and few_kernel wherever
+// within 6 us of the tile, took 2.1 %. Some (us, both sides measured): 64- / 128-row
+// tile, Q6_K 18944 x 3584 at 200 rows 141 / 138, 3584 x 18944 at 333 172 / 174,
+// 14336 x 4096 at 128 61 / 68, Q4_K 18944 x 3584 at 200 119 / 113, at 333 149 / 140,
+// 4096 x 4096 at 333 54 / 56; few_kernel / 32-row tile, Q4_K 4096 x 14336 at 16
+// rows 25 / 32, 24 rows 29 / 32, Q5_K 1024 x 1024 at 12 13 / 15, Q1_0 8192 x 1024
+// at 8 12 / 15, 1024 x 4096 at 32 19 / 17.
+struct PairCost {
+    double launches, start, unit, plane;
+    double us(int64_t workgroups, int64_t units, int64_t splits, double plane_us) const {
+        const double busy = workgroups < 256 ? (double)workgroups / 256 : 1.0;
+        return launches + (double)((workgroups + 255) / 256) * (start + (double)units * unit * (0.85 + 0.15 * busy)) +
+               (splits > 1 ? (double)splits * plane_us * plane : 0.0);
+    }
+};
+// bm 16: few_kernel with up to 16 rows, 17: with more
+PairCost pair_cost(int qtype, int bm) {
+    const int f = qtype == kTypeQ4K ? 0 : qtype == kTypeQ5K ? 1 : qtype == kTypeQ10 ? 2 : 3;
+    static constexpr double unit[5][4] = {
+        {2.1, 2.9, 1.7, 0.0}, {2.8, 3.6, 2.4, 0.0}, {3.2, 4.1, 3.0, 5.1}, {4.2, 5.3, 4.3, 5.3}, {8.2, 0.0, 0.0, 10.6}};
+    switch (bm) {
+        case 16: return {5.3, 6.2, unit[0][f], 1.8};
+        case 17: return {9.2, 3.8, unit[1][f], 1.1};
+        case 32: return {8.7, 4.0, unit[2][f], 0.8};
+        case 64: return {12.8, 0.8, unit[3][f], 0.7};
+        default: return {12.8, 0.8, unit[4][f], 0.7};
+    }
+}
+
 }  // namespace
 
 bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, PairPlan* p) {
@@ -1651,13 +1686,10 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
     p->bn = 256;
     p->layout = k4 ? kTypeQ4K : qtype;
     const int64_t ntiles = (n + p->bn - 1) / p->bn;
-    // The row tile and the split of k with the least estimated time: rounds of
-    // 256 workgroups (one per CU), each its share of units and a fixed start,
-    // and every plane written and read. Per unit, measured with k unsplit (us):
-    // 2.9 for 32 rows, 3.9 for 64, 7.0 for 128 (Q6_K 9.0).
-    const double plane_us = (double)m * (double)n * 8.0 / 2.5e6;
+    // The row tile and the split of k with the least estimated time.
+    const double plane_us = (double)m * (double)n * 8.0 / 3.1e6;
     // Q5_K and Q1_0, whose rows otherwise run one GEMV each, keep to the tiles
-    // with two-level sums, which match a GEMV's error.
+    // with fp64 sums, which match a GEMV's error.
     const bool wide = qtype == kTypeQ4K || qtype == kTypeQ6K;
     const int bms[2] = {m <= 32 ? 32 : 64, m <= 32 ? 32 : m <= 64 || !wide ? 64 : 128};
     double best = 0.0;
@@ -1669,14 +1701,13 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
         const size_t x_off = sum_off + (k4 ? (size_t)(mpad / 32 * p->units) * 4096 : 0);
         const size_t part_off = x_off + (size_t)mpad * (size_t)p->units * kUnit * 4;
         if (part_off > cap) continue;
-        const double unit_us = bm == 32 ? 2.9 : bm == 64 ? 3.9 : qtype == kTypeQ6K ? 9.0 : 7.0, start_us = 6.0;
+        const PairCost cost = pair_cost(qtype, bm);
         for (int64_t s = 1; s <= 64 && s <= p->units; ++s) {
             // the planes and the largest scales [s][n], or a word per wave of every tile
             const size_t planes = s > 1 ? align256((size_t)s * (size_t)m * (size_t)n * 4) : 0;
             const size_t aux = s > 1 ? (size_t)s * (size_t)n * 4 : (size_t)(mtiles * ntiles) * 8 * 4;
             if (part_off + planes + aux > cap) break;
-            const double rounds = (double)((mtiles * ntiles * s + 255) / 256);
-            const double us = rounds * (start_us + (double)((p->units + s - 1) / s) * unit_us) + (s > 1 ? s * plane_us + 1.0 : 0.0);
+            const double us = cost.us(mtiles * ntiles * s, (p->units + s - 1) / s, s, plane_us);
             if (!found || us < best) {
                 found = true;
                 best = us;
@@ -1693,11 +1724,7 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
     }
     if (m <= 32 && qtype != kTypeQ6K) {
         // few_kernel: one round of 256 workgroups where its LDS lets it, every
-        // split at least two units. Measured (us, both launches): 7 + 6 per
-        // round + 2.2 a unit (3.0 past 16 rows), against three launches and
-        // 6 more than the model above: 18944 x 3584, 16 rows 25 / 30, 32 rows
-        // (two rounds of it) 50 / 32; 4096 x 14336, 16 / 32 rows 26 / 32 against
-        // 35 / 38; 1024 x 1024 14 / 15.
+        // split at least two units
         const int64_t most = kFewUnits / (m <= 16 ? 1 : 2), need = (p->units + most - 1) / most;
         int64_t fs = 256 / ntiles < 64 ? 256 / ntiles : 64;
         if (fs > (p->units + 1) / 2) fs = (p->units + 1) / 2;
@@ -1705,11 +1732,11 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
         if (fs < 1) fs = 1;
         const int64_t share = (p->units + fs - 1) / fs;
         fs = (p->units + share - 1) / share;             // as few splits as give that share
-        const double few_us = 7.0 + (double)((ntiles * fs + 255) / 256) * (6.0 + (double)share * (m <= 16 ? 2.2 : 3.0));
+        const double few_us = pair_cost(qtype, m <= 16 ? 16 : 17).us(ntiles * fs, share, fs, plane_us);
         const size_t part_off = align256((size_t)fs * 32 * 4);
         const size_t aux_off = part_off + (fs > 1 ? align256((size_t)fs * (size_t)m * (size_t)n * 4) : 0);
         const size_t bytes = aux_off + (fs > 1 ? (size_t)fs * (size_t)n * 4 : (size_t)ntiles * 8 * 4);
-        if (bytes <= cap && fs * ntiles <= 0x7FFFFFFF && (!found || few_us < best + 6.0)) {
+        if (bytes <= cap && fs * ntiles <= 0x7FFFFFFF && (!found || few_us < best)) {
             p->few = true;
             p->splits = (int)fs;
             p->bm = 32;
