@@ -141,7 +141,7 @@ def test_small_x_beside_large_on_zero_weights(frq, q, n, k, rows, plan):
 
 @pytest.mark.parametrize("q,n,k,rows,plan", [
     ("Q4_K", 8192, 4096, 16, ("few", 32, 8)), ("Q5_K", 65537, 512, 9, ("few", 32, 1)),
-    ("Q1_0", 8192, 4096, 20, ("few", 32, 8)), ("Q5_K", 300, 2048, 9, ("pair", 32, 8)),
+    ("Q1_0", 8200, 4224, 30, ("few", 32, 6)), ("Q5_K", 300, 2048, 9, ("pair", 32, 8)),
     ("Q6_K", 66000, 512, 11, ("pair", 32, 1)), ("Q4_K", 70, 2048, 66, ("pair", 64, 8)),
     ("Q1_0", 65600, 512, 40, ("pair", 64, 1)), ("Q4_K", 33000, 1024, 66, ("pair", 128, 1)),
 ])
