@@ -307,10 +307,15 @@ bool mb_takes(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_
 constexpr int64_t kRowsBeforeGemm = 3;
 
 // Formats without a small-M kernel and gemm_f32 (Q5_K, Q1_0): one GEMV per row
-// below this many rows, the pair GEMM from there on (us, rows 2 / 4 / 8: Q5_K
-// 4096 x 4096 10.6 / 21 / 42 by rows, 18.6 from 4 by the pair GEMM; Q1_0
-// 2048 x 2048 6.5 / 12.9 / 28 and 15).
-constexpr int64_t kPairRowsMin = 4;
+// below this many rows, the pair GEMM from there on (us, rows 2 / 3 / 4: Q5_K
+// 4096 x 4096 9.8 / 14.7 / 19.5 by rows, 18.1 by the pair GEMM; 14336 x 4096
+// 19.6 / 28.9 / 38.4 and 25). Four rows of a Q1_0 matrix that one row's
+// matrix-core kernel runs in some 3 us stay by rows too (rows 4 / 5: 2048 x 2048
+// 12.2 / 15.3 by rows, 15.3 by the pair GEMM; 4096 x 4096 14.8 / 18.2 and 16.1;
+// but 1024 x 1024 12.8 / 15.7 and 12.3, 896 x 4864 20.1 and 14.8).
+int64_t pair_rows_min(int qtype, const uint8_t* w, int64_t n, int64_t k) {
+    return qtype == FRQ_Q1_0 && k >= 2048 && k <= 4096 && n * k <= (1 << 24) && frq::gemv_q10_mx_ok(w, k) ? 5 : 4;
+}
 
 // Where gemm_f32 is the faster one of the two: its two launches against the
 // pair GEMM's three decide on small matrices. Measured (us, gemm_f32 / pair):
@@ -351,7 +356,7 @@ BatchRoute batch_route(int qtype, const uint8_t* w, const float* x, int64_t batc
         return BatchRoute::SmallM;
     const bool own = qtype == FRQ_Q5_K || qtype == FRQ_Q1_0;
     frq::PairPlan p;
-    if (batch >= (own ? kPairRowsMin : kRowsBeforeGemm + 1) &&
+    if (batch >= (own ? pair_rows_min(qtype, w, n, k) : kRowsBeforeGemm + 1) &&
         !(f32_before_pair(qtype, batch, n, k) && batched_gemm(qtype, w, x, batch, n, k)) && pair_plan(qtype, w, x, batch, n, k, pair_cap, &p))
         return BatchRoute::Pair;
     if (batch > kRowsBeforeGemm && batched_gemm(qtype, w, x, batch, n, k)) return BatchRoute::Gemm;
