@@ -347,17 +347,18 @@ bool pair_plan(int qtype, const uint8_t* w, const float* x, int64_t batch, int64
 // Which kernels a batch of x rows takes: the small-M kernel for two to
 // mr_rows_before_gemm rows, else one GEMV per row up to kRowsBeforeGemm
 // rows, else a GEMM where there is one (the pair GEMM, or gemm_f32 where its
-// scratch does not fit), else one GEMV per row.
+// scratch does not fit), else one GEMV per row. `p`: the plan of the pair GEMM
+// (of the first kPairRows rows), where that is the route.
 enum class BatchRoute { SmallM, Pair, Gemm, Rows };
 BatchRoute batch_route(int qtype, const uint8_t* w, const float* x, int64_t batch, int64_t n, int64_t k,
-                       size_t pair_cap) {
+                       size_t pair_cap, frq::PairPlan* p) {
     if (mb_takes(qtype, w, x, batch, n, k) ||
         (batch >= 2 && batch <= mr_rows_before_gemm(qtype) && frq::gemv_mr_ok(qtype, w, x, k)))
         return BatchRoute::SmallM;
     const bool own = qtype == FRQ_Q5_K || qtype == FRQ_Q1_0;
-    frq::PairPlan p;
     if (batch >= (own ? pair_rows_min(qtype, w, n, k) : kRowsBeforeGemm + 1) &&
-        !(f32_before_pair(qtype, batch, n, k) && batched_gemm(qtype, w, x, batch, n, k)) && pair_plan(qtype, w, x, batch, n, k, pair_cap, &p))
+        !(f32_before_pair(qtype, batch, n, k) && batched_gemm(qtype, w, x, batch, n, k)) &&
+        pair_plan(qtype, w, x, batch, n, k, pair_cap, p))
         return BatchRoute::Pair;
     if (batch > kRowsBeforeGemm && batched_gemm(qtype, w, x, batch, n, k)) return BatchRoute::Gemm;
     return BatchRoute::Rows;
@@ -376,14 +377,14 @@ uint8_t* pair_scratch_locked(hipStream_t s, size_t bytes) {
     return nullptr;
 }
 
-// The pair GEMM over all rows, kPairRows at a time. x_ready: the scratch holds
-// the pairs of these rows (one chunk) already.
+// The pair GEMM over all rows, kPairRows at a time, by the plan `p` of the first
+// ones (the last, if fewer, by their own). x_ready: the scratch holds the pairs
+// of these rows (one chunk) already.
 int pair_rows(int qtype, const uint8_t* w, const float* x, float* y, int64_t n, int64_t k, int64_t batch, int64_t ldy,
-              hipStream_t s, uint8_t* scratch, size_t cap, bool x_ready) {
+              hipStream_t s, uint8_t* scratch, size_t cap, frq::PairPlan p, bool x_ready) {
     for (int64_t b = 0; b < batch; b += frq::kPairRows) {
-        frq::PairPlan p;
         const int64_t m = batch - b < frq::kPairRows ? batch - b : frq::kPairRows;
-        if (!frq::plan_gemm_pair(qtype, m, n, k, cap, &p)) return fail(FRQ_ERR_UNSUPPORTED, "gemm: no plan");
+        if (m != p.m && !frq::plan_gemm_pair(qtype, m, n, k, cap, &p)) return fail(FRQ_ERR_UNSUPPORTED, "gemm: no plan");
         FRQ_HIP(frq::launch_gemm_pair(qtype, w, x + b * k, y + b * ldy, ldy, p, s, scratch, x_ready));
     }
     return FRQ_OK;
@@ -393,7 +394,8 @@ int pair_rows(int qtype, const uint8_t* w, const float* x, float* y, int64_t n, 
 // gemv_device (the small-M kernel uses none).
 int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t n, int64_t k, int64_t batch,
                  int64_t ldy, hipStream_t s, const frq::FixedScratch* fixed = nullptr) {
-    BatchRoute route = batch_route(qtype, w, x, batch, n, k, pair_cap(fixed));
+    frq::PairPlan pp;
+    BatchRoute route = batch_route(qtype, w, x, batch, n, k, pair_cap(fixed), &pp);
     if (route == BatchRoute::SmallM && mb_takes(qtype, w, x, batch, n, k)) {
         frq::MbPlan p;
         frq::plan_gemv_mb(n, k, (int)batch, &p);
@@ -411,12 +413,10 @@ int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t 
     if (route == BatchRoute::Pair) {
         if (fixed)
             return pair_rows(qtype, w, x, y, n, k, batch, ldy, s, reinterpret_cast<uint8_t*>(fixed->part),
-                             fixed->part_bytes, false);
-        frq::PairPlan p;
-        pair_plan(qtype, w, x, batch, n, k, kPairScratchMax, &p);
+                             fixed->part_bytes, pp, false);
         std::lock_guard<std::mutex> lk(g_sk_mu);
-        if (uint8_t* scratch = pair_scratch_locked(s, p.bytes))
-            return pair_rows(qtype, w, x, y, n, k, batch, ldy, s, scratch, p.bytes, false);
+        if (uint8_t* scratch = pair_scratch_locked(s, pp.bytes))
+            return pair_rows(qtype, w, x, y, n, k, batch, ldy, s, scratch, pp.bytes, pp, false);
         route = batched_gemm(qtype, w, x, batch, n, k) ? BatchRoute::Gemm : BatchRoute::Rows;
     }
     if (route == BatchRoute::Gemm) {
@@ -442,26 +442,27 @@ int gemv_batched(int qtype, const uint8_t* w, const float* x, float* y, int64_t 
 // of its elements. Same bits as separate calls.
 int gemv_batched_group(int count, const int* qtypes, const uint8_t* const* w, const float* x, float* const* y,
                        const int64_t* n, int64_t k, int64_t batch, const int64_t* ldy, hipStream_t s) {
-    bool done[frq::kGemvGroupMax] = {};
+    bool done[frq::kGemvGroupMax] = {}, pair[frq::kGemvGroupMax] = {};
     frq::PairPlan p[frq::kGemvGroupMax];
     size_t need = 0;
     for (int i = 0; i < count; ++i) {
         done[i] = n[i] == 0;
         if (!done[i] && batch <= frq::kPairRows &&
-            batch_route(qtypes[i], w[i], x, batch, n[i], k, kPairScratchMax) == BatchRoute::Pair &&
-            pair_plan(qtypes[i], w[i], x, batch, n[i], k, kPairScratchMax, &p[i]) && p[i].bytes > need)
-            need = p[i].bytes;
+            batch_route(qtypes[i], w[i], x, batch, n[i], k, kPairScratchMax, &p[i]) == BatchRoute::Pair) {
+            pair[i] = true;
+            if (p[i].bytes > need) need = p[i].bytes;
+        }
     }
     if (need) {
         std::lock_guard<std::mutex> lk(g_sk_mu);
         if (uint8_t* scratch = pair_scratch_locked(s, need))
             for (int i = 0; i < count; ++i) {
-                if (done[i] || !p[i].bytes) continue;
+                if (done[i] || !pair[i]) continue;
                 bool ready = false;
                 for (int j = i; j < count; ++j)          // every matrix of this element order
-                    if (!done[j] && p[j].bytes && p[j].layout == p[i].layout && p[j].bm == p[i].bm) {
+                    if (!done[j] && pair[j] && p[j].layout == p[i].layout && p[j].bm == p[i].bm) {
                         if (int rc = pair_rows(qtypes[j], w[j], x, y[j], n[j], k, batch, ldy[j], s, scratch, p[j].bytes,
-                                               ready))
+                                               p[j], ready))
                             return rc;
                         done[j] = true;
                         ready = !p[j].few;
@@ -720,7 +721,8 @@ static int dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, fl
         size_t sb = 0, pb = 0;
         // the small-M kernel needs no scratch and the batched GEMM splits K
         // within what is there; rows that run one GEMV each need theirs
-        if (batch_route(qtype, wp, x, batch, n, k, pair_cap(fixed)) == BatchRoute::Rows)
+        frq::PairPlan p;
+        if (batch_route(qtype, wp, x, batch, n, k, pair_cap(fixed), &p) == BatchRoute::Rows)
             gemv_scratch_need(qtype, wp, x, n, k, &sb, &pb);
         if (sb > fixed->slot_bytes || pb > fixed->part_bytes)
             return fail(FRQ_ERR_UNSUPPORTED,
@@ -742,18 +744,16 @@ int frq_gemv_batch_plan(int qtype, int64_t n, int64_t k, int64_t batch, int64_t 
     if (!fmt_of(qtype, &f)) return fail(FRQ_ERR_INVALID, "unknown qtype %d", qtype);
     if (n <= 0 || k <= 0 || batch < 2 || k % f.belems) return fail(FRQ_ERR_SHAPE, "batch plan: shape");
     for (int i = 0; i < 4; ++i) plan[i] = 0;
-    switch (batch_route(qtype, nullptr, nullptr, batch, n, k, kPairScratchMax)) {
+    frq::PairPlan p;
+    switch (batch_route(qtype, nullptr, nullptr, batch, n, k, kPairScratchMax, &p)) {
         case BatchRoute::SmallM: plan[0] = FRQ_BATCH_SMALL; break;
         case BatchRoute::Gemm: plan[0] = FRQ_BATCH_GEMM; break;
         case BatchRoute::Rows: plan[0] = FRQ_BATCH_ROWS; break;
-        case BatchRoute::Pair: {
-            frq::PairPlan p;
-            pair_plan(qtype, nullptr, nullptr, batch, n, k, kPairScratchMax, &p);
+        case BatchRoute::Pair:
             plan[0] = p.few ? FRQ_BATCH_FEW : FRQ_BATCH_PAIR;
             plan[1] = p.bm;
             plan[2] = p.splits;
             plan[3] = (int64_t)p.bytes;
-        }
     }
     return FRQ_OK;
 }
