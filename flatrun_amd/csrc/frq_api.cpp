@@ -125,8 +125,10 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // on that stream still launches kernels on the old address; the counters of
 // a retired buffer stay zero, since every launch leaves them so. The registry
 // lock is held from the lookup through the launch, so one thread cannot
-// retire a buffer another is about to launch with. Capacities grow at least
-// twofold, so a stream retires O(log size) buffers.
+// retire a buffer another is about to launch with. Capacities up to 1 GiB (the
+// pair GEMM never needs more) are powers of two, larger ones grow at least
+// twofold, so a stream retires O(log size) buffers, and less than 1 GiB of them
+// below that. Where the size cannot be had, what the launch needs is tried.
 struct SkScratch {
     void* part = nullptr;
     size_t part_cap = 0;
@@ -137,6 +139,7 @@ struct SkScratch {
 std::mutex g_sk_mu;
 std::map<std::pair<int, hipStream_t>, SkScratch> g_sk;
 
+constexpr size_t kScratchPow2Max = (size_t)1 << 30;
 int grow(void** ptr, size_t* cap, size_t bytes, bool zero, std::vector<void*>* retired, hipStream_t stream) {
     if (*cap >= bytes) return FRQ_OK;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -144,12 +147,18 @@ int grow(void** ptr, size_t* cap, size_t bytes, bool zero, std::vector<void*>* r
     if (cs != hipStreamCaptureStatusNone)
         return fail(FRQ_ERR_UNSUPPORTED, "scratch for this shape must exist before graph capture: run the call once "
                                          "on the stream before capturing it");
-    size_t want = bytes < ((size_t)1 << 16) ? ((size_t)1 << 16) : bytes;
-    if (want < 2 * *cap) want = 2 * *cap;
+    size_t want = (size_t)1 << 16;
+    while (want < bytes && want < kScratchPow2Max) want *= 2;
+    if (want < bytes) want = bytes < 2 * *cap ? 2 * *cap : bytes;
     void* p = nullptr;
-    FRQ_HIP(hipMalloc(&p, want));
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && want > bytes) {
+        (void)hipGetLastError();
+        e = hipMalloc(&p, want = bytes);
+    }
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc(scratch)");
     if (zero) {   // on the launch stream: ordered before the kernel that first reads it
-        const hipError_t e = hipMemsetAsync(p, 0, want, stream);
+        e = hipMemsetAsync(p, 0, want, stream);
         if (e != hipSuccess) {
             (void)hipFree(p);
             return hip_fail(e, "hipMemsetAsync(scratch)");
@@ -332,7 +341,7 @@ bool f32_before_pair(int qtype, int64_t batch, int64_t n, int64_t k) {
 
 // Scratch a pair launch may hold per stream; shapes beyond it take the kernels
 // that need less (gemm_f32, one GEMV per row).
-constexpr size_t kPairScratchMax = (size_t)1 << 30;
+constexpr size_t kPairScratchMax = kScratchPow2Max;
 
 // The pair GEMM's plan for up to kPairRows rows of x, false where it does not
 // take the shape, the alignment or the scratch.

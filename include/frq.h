@@ -190,8 +190,10 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  * batch-1 call); up to 3 rows that neither takes run one GEMV per row. Few output
  * tiles split k over workgroups whose fp32 partials a second kernel adds in
  * a fixed order. Scratch of the stream: the pairs (4 bytes per element of up to
- * 1024 rows of x, padded to the tile) and the partials, at most 1 GiB; a
- * stream under capture that has less runs the kernels that need less. */
+ * 1024 rows of x, padded to the tile) and the partials, rounded up to a power of
+ * two of at most 1 GiB; buffers that it grew out of, less than 1 GiB together,
+ * stay until frq_stream_destroy, since captured graphs may use them. A stream
+ * under capture that has less runs the kernels that need less. */
 int frq_dev_gemv(int qtype, const void* w, size_t w_bytes, const float* x, float* y, int64_t n, int64_t k,
                  int64_t batch, void* stream);
 
