@@ -23,6 +23,7 @@ from __future__ import annotations
 
 import os
 import threading
+import weakref
 
 import numpy as np
 
@@ -108,28 +109,51 @@ def _raw_bytes(weight) -> np.ndarray:
 _GIB = 1 << 30
 
 # Page-locked memory that activations and results of resident-weight calls go
-# through (larger results, or x over 1 MiB, are copied without it). A call
-# takes one buffer and gives it back; at most two are kept between calls.
+# through (larger results, or x over 1 MiB, are copied without it).
 _PINNED_BYTES = 4 << 20
-_pinned_free: list = []
 
 
-def _take_pinned():
-    """A buffer no other call holds, or None where there is none to have."""
-    from . import device
-    try:
-        return _pinned_free.pop()
-    except IndexError:
-        pass
-    try:
-        return device.PinnedBuffer(_PINNED_BYTES)
-    except FrqDeviceError:
-        return None
+class _PinnedPool:
+    """Page-locked buffers between the calls of all backends: a call takes one
+    and gives it back, at most two are kept, and none once the last backend of
+    the process is gone."""
+
+    def __init__(self) -> None:
+        self._lock = threading.RLock()                    # a collection inside may end a backend
+        self._free: list = []
+        self._users = 0
+
+    def join(self, backend) -> None:
+        with self._lock:
+            self._users += 1
+        weakref.finalize(backend, self._leave).atexit = False
+
+    def _leave(self) -> None:
+        with self._lock:
+            self._users -= 1
+            drop = [] if self._users else self._free
+            if drop:
+                self._free = []
+        del drop                                          # freed outside the lock
+
+    def take(self):
+        """A buffer no other call holds, or None where there is none to have."""
+        from . import device
+        with self._lock:
+            if self._free:
+                return self._free.pop()
+        try:
+            return device.PinnedBuffer(_PINNED_BYTES)
+        except FrqDeviceError:
+            return None
+
+    def give(self, buf) -> None:
+        with self._lock:
+            if buf is not None and self._users and len(self._free) < 2:
+                self._free.append(buf)
 
 
-def _give_pinned(buf) -> None:
-    if buf is not None and len(_pinned_free) < 2:
-        _pinned_free.append(buf)
+_pinned = _PinnedPool()
 
 
 def _cache_capacity(setting) -> int:
@@ -187,6 +211,7 @@ class NativeBackend:
         self._neon = False
         self._scratch = None
         self._lock = threading.RLock()
+        _pinned.join(self)
         cap = _cache_capacity(os.environ.get("FLATRUN_AMD_WEIGHT_CACHE") if weight_cache is None else weight_cache)
         self._cache = WeightCache(cap) if cap > 0 else None
         self._stream_src = None
@@ -276,9 +301,9 @@ class NativeBackend:
             xb = (seq * k * 4 + 255) // 256 * 256
             with self._lock:
                 scratch = self._scratch_for(xb + (seq * n * 4 + 15) // 16 * 16)
-                pinned = _take_pinned()
+                pinned = _pinned.take()
                 device.gemv_host(qname, weight, x_c, out, n, k, seq, scratch, pinned, w_bytes=weight.nbytes)
-                _give_pinned(pinned)      # not after an error: a copy may still be pending, and freeing waits for it
+                _pinned.give(pinned)      # not after an error: a copy may still be pending, and freeing waits for it
         return out[0] if x_c.ndim == 1 else out
 
     def upload(self, weight) -> DeviceWeight:
