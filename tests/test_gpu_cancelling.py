@@ -123,9 +123,11 @@ def test_matrix_core_load_depths(frq, n, k, depth):
                                    ("Q8_0", 4864, 896), ("Q5_K", 128, 4096)])
 @pytest.mark.parametrize("seq", [2, 3, 4, 5, 33])
 def test_batched(frq, q, n, k, seq):
-    """The fp32 GEMM for two or more rows (per-row GEMVs for Q5_K, the
-    small-M matvec for a few rows of Q4_K, Q6_K and Q8_0), outliers in every
-    row, each row with another outlier set."""
+    """Every route of two or more rows: the small-M matvec for a few rows of
+    Q4_K, Q6_K and Q8_0 and per-row GEMVs for those of Q5_K, the pair GEMM
+    (Q5_K from four rows, 33 rows of the large Q4_K matrix) and the fp32 GEMM
+    (33 rows of the others); outliers in every row, each row with another
+    outlier set."""
     raw, cols = _input(q, n, k, seed=n + seq)
     xs = np.stack([outlier_x(k, cols, seed=100 + r, big=(2.0**(20 + r % 9), -(2.0**24), 3.0e4)) for r in range(seq)])
     y, _ = _run(q, raw, xs, n, k)

@@ -1,8 +1,10 @@
 """The 256 x 256 tile of the prefill GEMM (Q4_K products whose 256 x 128 tiles
 take two rounds or more), at ragged rows and columns, the smallest k and odd
 numbers of blocks: against the oracle, and bit for bit against the same rows
-of W in products that are too small for it (the order of sums is the same;
-8448 or more rows of W at 257 or more of x are not split over k)."""
+of W in products that the 256 x 128 tiles run (the order of sums is the same).
+These are pieces of 8448 rows of W or more, which are not split over k at 257 or
+more rows of x, and of 16384 at most, which one round of the smaller tiles covers
+up to 512 rows of x."""
 
 from __future__ import annotations
 
@@ -26,8 +28,10 @@ def test_big_tile(frq, m, ns, k):
     stride = sum(ns) + 3 if len(ns) > 1 else 0
     ys = run_group([("Q4_K", raw, n) for raw, n in zip(raws, ns)], xb, m, k, y_stride=stride)
     for raw, n, y in zip(raws, ns, ys):
-        cut = [0, n // 2, n] if n >= 2 * 8448 else [0, n]
-        for a, b in zip(cut, cut[1:]):
+        # (16385 rows have no such pair of pieces: the larger overlaps the smaller)
+        cuts = [(0, n)] if n <= 16384 else [(0, max(n // 2, 8448)), (n - max(n // 2, 8448), n)]
+        for a, b in cuts:
+            assert 8448 <= b - a <= 16384
             assert bits_equal(np.ascontiguousarray(y[:, a:b]), single("Q4_K", raw[a * row:b * row], xb, b - a, k))
         tail = n - 300
         check(np.ascontiguousarray(y[:, tail:]), raw[tail * row:], xb, 300, k)

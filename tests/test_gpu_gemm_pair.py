@@ -59,6 +59,36 @@ def test_edges(frq, q, n, k, rows):
     check(q, raw, xs[some], n, k, y[some], f"{q} {n}x{k} rows {rows}")
 
 
+@pytest.mark.parametrize("q,n,k,rows,plan", [
+    # the few-row kernel: one and two row tiles, ragged rows of W, an odd number
+    # of Q1_0 blocks, k unsplit (results stored directly), all of its LDS (eight
+    # units of Q4_K and Q5_K), more units than it has loads in flight
+    ("Q1_0", 8192, 4096, 16, ("few", 32, 8)), ("Q1_0", 8190, 4224, 16, ("few", 32, 6)),
+    ("Q1_0", 8200, 4224, 30, ("few", 32, 6)), ("Q1_0", 65551, 384, 4, ("few", 32, 1)),
+    ("Q5_K", 14301, 4096, 17, ("few", 32, 4)), ("Q5_K", 14336, 4096, 32, ("few", 32, 4)),
+    ("Q5_K", 65537, 512, 16, ("few", 32, 1)), ("Q5_K", 65601, 2048, 16, ("few", 32, 1)),
+    ("Q4_K", 66000, 1024, 20, ("few", 32, 1)), ("Q4_K", 65600, 2048, 16, ("few", 32, 1)),
+    ("Q4_K", 65601, 1280, 11, ("few", 32, 1)), ("Q5_K", 8192, 12544, 8, ("few", 32, 7)),
+    # the 128-row tile, one row or column past its end, k unsplit and split
+    ("Q4_K", 33000, 1024, 65, ("pair", 128, 1)), ("Q4_K", 20001, 768, 300, ("pair", 128, 1)),
+    ("Q4_K", 18945, 1280, 257, ("pair", 128, 1)), ("Q4_K", 18945, 3584, 200, ("pair", 128, 3)),
+    ("Q6_K", 30000, 1280, 129, ("pair", 128, 1)), ("Q6_K", 62765, 1024, 383, ("pair", 128, 1)),
+    # rows of x in two and three registers' worth of pieces, and too long for them
+    ("Q6_K", 3001, 8192, 33, ("pair", 64, 16)), ("Q6_K", 1500, 20480, 40, ("pair", 64, 40)),
+    ("Q5_K", 100, 24832, 33, ("pair", 64, 49)), ("Q5_K", 100, 20736, 70, ("pair", 64, 41)),
+    ("Q1_0", 300, 24704, 70, ("pair", 64, 49)),
+])
+def test_planned_edges(frq, q, n, k, rows, plan):
+    assert device.batch_plan(q, n, k, rows)[:3] == plan
+    raw = synth.make_blocks(q, n, k, seed=n + k)
+    xs = synth.make_x(k, seed=rows, batch=rows)
+    y = run(q, raw, xs, n, k)
+    assert np.isfinite(y).all()
+    some = np.unique(np.r_[:min(n, 260), max(0, n - 300):n, np.random.default_rng(n).choice(n, min(n, 400), replace=False)])
+    part = np.ascontiguousarray(raw.reshape(n, -1)[some]).reshape(-1)
+    check(q, part, xs, some.size, k, y[:, some], f"{q} {n}x{k} rows {rows}")
+
+
 @pytest.mark.parametrize("q,n,k,rows", [("Q5_K", 70, 4096, 9), ("Q1_0", 70, 4096, 40), ("Q4_K", 70, 2048, 66)])
 def test_rows_beyond_the_pairs(frq, q, n, k, rows):
     """Outliers from 2^14 to 2^40 above the rest, all rows tiny or huge, one inf

@@ -53,9 +53,9 @@ def test_gemv_shapes(frq, q, n, k):
 
 @pytest.mark.parametrize("q", QS)
 def test_gemv_batched(frq, q):
-    """Batched host entry: Q4_K, Q6_K and Q8_0 rows go through the fp32
-    GEMM (W read once), checked against the oracle; Q5_K and Q1_0 run one
-    GEMV per row, bit for bit the single-row results."""
+    """Batched host entry, three rows: Q4_K, Q6_K and Q8_0 take the small-M
+    matvec (W read once), checked against the oracle; Q5_K and Q1_0 run one
+    GEMV per row below four rows, bit for bit the single-row results."""
     be = synth.BLOCK[q][1]
     n, k = 45, 8 * be
     raw = synth.make_blocks(q, n, k, seed=3)
