@@ -40,17 +40,18 @@
 // Tiling: BM x BN of Y per workgroup; a wave owns 32 MT x 32 NT. W goes from
 // memory to registers to the matrix cores (lane = one row of W; both halves
 // of the wave read consecutive 16-byte parts), decoded once per workgroup
-// where WM = 1; x goes through LDS, 32 KB per barrier, double-buffered, as
-// every wave reads all of it. K is split over S workgroups where the tiles
+// where WM = 1; x goes through LDS, 32 KB per barrier, four buffers, as every
+// wave reads all of it. K is split over S workgroups where the tiles
 // do not fill the GPU; finish_kernel adds the partial planes in split order.
-// Measured (kernel us, gemm_f32 / here): 333 rows, Q4_K 18944 x 3584 261 / 125
-// (837 TFLOP/s of matrix work on rows padded to 384, about 1300 in a large
-// library product), Q6_K 3584 x 18944 351 / 173 (its scale per 16 elements:
-// eight times the vector work); whole calls, 97 rows of Q5_K 14336 x 4096 1391
-// (a GEMV per row) / 52, 16 rows of Q4_K 4096 x 14336 35.5 / 30.3 (few_kernel
-// 23.8). 128-row tiles
-// are bound by the matrix cores' issue and power, few rows by the chain of
-// decode and products per wave (2.9 us per 256 of k) and the three launches.
+// Measured (whole calls, us, W cold; gemm_f32 / here): 333 rows, Q4_K 18944 x 3584
+// 224 / 132 (800 TFLOP/s of matrix work on rows padded to 384 in the kernel, about
+// 1300 in a large library product), Q6_K 3584 x 18944 322 / 168 (its scale per 16
+// elements: eight times the vector work); 97 rows of Q5_K 14336 x 4096 1390 (a GEMV
+// per row) / 58; 16 rows of Q4_K 4096 x 14336 36 / 32 (few_kernel 25). 128-row
+// tiles are bound by the matrix cores' issue and power, few rows by the chain of
+// decode and products per wave (3.2 us per 256 of k) and the three launches. The
+// range of lo costs a vector instruction per two codes, or per sum with 128 rows:
+// 127 -> 132 us, 97 rows of Q5_K (with fp64 sums) 55 -> 58.
 // MFMA operand layouts (32x32x16, 8 values per lane): A lane l holds row l%32,
 // k = 8*(l/32) .. +7; B lane l column l%32, same k; D register r of lane l is
 // row 8*(r/4) + 4*(l/32) + r%4, column l%32. The order of k is free as long as
@@ -144,8 +145,10 @@ __device__ __forceinline__ void lds_copy(__amdgpu_buffer_rsrc_t r, uint32_t lane
 // The 2-byte aligned fields of Q6_K blocks are read by dword-aligned loads and
 // shifted when they are used: wide loads off dword boundaries run at a fraction
 // of the rate (4096 x 14336, 16 rows: 54 us against 39). A window starts at
-// the dword that holds the field's first byte and ends at the one that holds
-// its last, or inside the block.
+// the dword that holds the field's first byte and has one dword more than the
+// field: up to two bytes before the first block of W (on a base that is 2 past a
+// dword) or after its last one (on a dword) are read, in dwords that hold bytes of
+// W, and used for nothing.
 struct Window {
     gptr base;
     uint32_t off;           // of the dword that holds the byte at base + off
@@ -165,8 +168,8 @@ __device__ __forceinline__ uint32_t shifted(uint32_t lo, uint32_t hi, uint32_t s
 // One row's fields of one 256-element unit, as the lane (half h of its row)
 // needs them: Head<QT> those used all through the unit, Body<QT> the codes,
 // load<T> those of stage T (`unit` = the unit in the first of the
-// workgroup's rows, `row` the lane's row from there, `left` = blocks of Q8_0 /
-// Q1_0 from the unit on). frag<T, I>: the eight codes of slice
+// workgroup's rows, `row` the lane's row from there, `left` = blocks of Q1_0
+// from the unit on). frag<T, I>: the eight codes of slice
 // I of stage T; scale<T, I>: what the sum of the group that ends with that
 // slice is multiplied by. Stage / slice / element orders are those of
 // Order<QT> below.
@@ -599,13 +602,16 @@ __device__ __forceinline__ void interleave() {
     });
 }
 
-// WM x WN = 8 waves of 32 MT x 32 NT; LS stages of x per barrier (32 KB),
-// three buffers: period p + 2 is written while p is computed, so the first
-// fragments of p + 1 are read before the barrier. A wave's work is a sequence
-// of chains of matrix instructions, one tile and scale group each: the small
-// lo products before the hi ones (their sums round at their own size), into
-// one of two register sets, while the other one is scaled into its tile's
-// accumulator and the codes to come are made.
+// WM x WN = 8 waves of 32 MT x 32 NT; LS stages of x per barrier (32 KB), four
+// buffers: period p + 3 is written while p is computed, into the buffer that
+// p - 1 was read from; the barrier at the end of p - 1 completed the copies of
+// p + 1 (kCopies below), so its first fragments are read before the next one.
+// A wave's work is a sequence of chains of matrix instructions, one tile and
+// scale group each: the small lo products before the hi ones (their sums round
+// at their own size), into one of two register sets, while the other one is
+// scaled into its tile's accumulator and the codes to come are made. Where the
+// registers hold codes for lo and hi, the latter are made beside the products
+// (VALU 16 per chain); else (128 rows of Q4_K) the sums of lo are scaled.
 // DEPTH > 1: as many register sets of W, each loaded DEPTH units ahead (few
 // rows of x: the kernel waits for W); else one, whose stages are loaded again,
 // for the next unit, two stages ahead (128 rows: registers).
@@ -839,7 +845,9 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
                     if constexpr (kScaleT) {
                         constexpr int V = 2 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0);
                         interleave<4, V>();
-                        __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+                        // the scaling, and the chain before into its sums while the last lo product ends
+                        // (333 rows of Q4_K 18944 x 3584: 131.4 us, with the scaling alone 132.9)
+                        __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
                         interleave<5, V>();
                     } else {
                         interleave<8 + (kK4<QT> ? 1 : 0), 4 + (NT == 2 && PH == 0 ? 8 : 0) + (last ? 8 : 0)>();
@@ -1258,8 +1266,8 @@ __global__ void __launch_bounds__(256) finish_kernel(const float* __restrict__ p
 // 16 waves (four per SIMD) hide each other's chains of decode and products,
 // which bound the 32-row tile of gemm_pair_kernel at two waves per SIMD. Measured
 // (whole call, us, three launches with that tile / here): 16 rows of Q4_K
-// 4096 x 14336 30.3 / 23.8 (1.4 TB/s of W; bound by vector work, about five
-// instructions per weight), 18944 x 3584 30 / 25, Q1_0 8192 x 4096 21 / 17.
+// 4096 x 14336 31.9 / 24.6 (1.4 TB/s of W; bound by vector work, about five
+// instructions per weight), Q1_0 8192 x 1024 15.5 / 12.2, Q5_K 1024 x 1024 15.3 / 13.1.
 constexpr int kFewUnits = 8;
 constexpr int kFewAside = 256, kFewHead = kFewAside + 2048;   // LDS: factors and limits of the rows, a place for unused writes, x
 

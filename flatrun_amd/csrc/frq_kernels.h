@@ -229,7 +229,8 @@ hipError_t launch_gemm_f32(int qtype, const uint8_t* w, const float* x, float* y
 // Batched matvec with the fp32 contract, x as pairs of fp16 values
 // (frq_gemm_pair.hip): y[m, n] = x[m, k] . W[n, k]^T for raw Q4_K, Q5_K, Q6_K
 // or Q1_0 blocks, rows of y ldy >= n floats apart; x 16-byte aligned, w
-// 16-byte (Q4_K, Q5_K) / 2-byte aligned. At most kPairRows rows a launch.
+// 16-byte (Q4_K, Q5_K) / 2-byte aligned; of Q6_K, the whole dwords that hold its
+// first and last bytes are read. At most kPairRows rows a launch.
 // `scratch` (p.bytes, 256-byte aligned) holds the row factors and limits, the
 // sub-block sums, the pairs, the partial planes of a split k and marks for the
 // last kernel; launches sharing it must be ordered. With x_ready the first three are those of an earlier launch of the same x,

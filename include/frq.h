@@ -187,8 +187,8 @@ int frq_dev_dequant_f16(int qtype, const void* w, size_t w_bytes, int64_t n_elem
  * Q6_K: up to 10) the element-wise small-M matvec, one launch per two or
  * three rows (Q4_K with per-weight fp32 arithmetic as one row, a row's bits
  * the same in any batch this kernel takes; Q6_K and Q8_0 with the bits of a
- * batch-1 call); up to 3 rows that neither takes run one GEMV per row. Few output
- * tiles split k over workgroups whose fp32 partials a second kernel adds in
+ * batch-1 call); up to 3 rows that neither takes (4 of a small Q1_0 matrix) run
+ * one GEMV per row. Few output tiles split k over workgroups whose fp32 partials a second kernel adds in
  * a fixed order. Scratch of the stream: the pairs (4 bytes per element of up to
  * 1024 rows of x, padded to the tile) and the partials, rounded up to a power of
  * two of at most 1 GiB; buffers that it grew out of, less than 1 GiB together,
