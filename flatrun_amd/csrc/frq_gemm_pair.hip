@@ -1317,7 +1317,9 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
                                                    uint32_t* __restrict__ aux) {
     constexpr int kHalf = 8192 + (kK4<QT> ? 1024 : 0);   // pairs and sums of 16 rows x 128 k
     constexpr int kUnitBytes = (int)weight_row_bytes<QT>(kUnit);
-    constexpr int DEPTH = QT == kTypeQ5K ? 2 : 3;        // units of W in flight (registers)
+    // units of W in flight (registers; two tiles of Q5_K have at most four in all:
+    // 24 rows of 14336 x 4096 29.0 us, with two 29.9 and sums in fp32)
+    constexpr int DEPTH = QT == kTypeQ5K ? (MT == 2 ? 1 : 2) : 3;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave & 7, kh = wave >> 3, c = lane & 15, q = lane >> 4;
@@ -1430,9 +1432,8 @@ __global__ void __launch_bounds__(1024) few_kernel(const uint8_t* __restrict__ w
     }
     __syncthreads();
 
-    // sums in fp64 for Q5_K and Q1_0 (as in gemm_pair_kernel) where the registers
-    // allow: two tiles of Q5_K add at most four units
-    typedef typename std::conditional<(QT == kTypeQ5K && MT == 1) || QT == kTypeQ10, f64x4, f32x4>::type Sum;
+    // sums in fp64 for Q5_K and Q1_0, as in gemm_pair_kernel
+    typedef typename std::conditional<QT == kTypeQ5K || QT == kTypeQ10, f64x4, f32x4>::type Sum;
     Sum acc[MT][2] = {};
     float dmax = 0.0f;                                   // the largest |d| of the lane's rows of W
     const PairDecode dec(4 * kh + q);                    // this lane's sub-block

@@ -217,7 +217,7 @@ def test_many_rows_weight_by_weight(frq, q, n, k, rows, bad):
 
 
 @pytest.mark.parametrize("q,n,k,rows,plan", [
-    ("Q5_K", 8192, 4096, 12, ("few", 32, 8)), ("Q5_K", 4096, 11008, 40, ("pair", 64, 15)),
+    ("Q5_K", 8192, 4096, 12, ("few", 32, 8)), ("Q5_K", 11008, 3584, 24, ("few", 32, 5)), ("Q5_K", 4096, 11008, 40, ("pair", 64, 15)),
     ("Q5_K", 8192, 4096, 97, ("pair", 64, 4)), ("Q1_0", 8192, 4096, 97, ("pair", 64, 4)),
 ])
 def test_error_no_larger_than_one_gemv_per_row(frq, q, n, k, rows, plan):
