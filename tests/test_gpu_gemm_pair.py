@@ -257,3 +257,55 @@ def test_group_shares_the_pairs(frq):
     for q, n, r in zip(qs, ns, raws):
         assert bits_equal(y[:, off:off + n], run(q, r, xs, n, k)), q
         off += n
+
+
+def test_small_x_in_groups_and_graphs(frq):
+    """Matrices that share the pairs of a SwiGLU-made x, with outputs that hang on
+    its smallest values (k split and not): each has the bits it has alone, in a
+    group and in replays of a graph, and the bound holds."""
+    k, rows = 1024, 40
+    specs = [("Q5_K", 300), ("Q4_K", 33000), ("Q5_K", 65600)]
+    assert [device.batch_plan(q, n, k, rows)[:3] for q, n in specs] == [("pair", 64, 4), ("pair", 64, 1), ("pair", 64, 2)]
+    raws, at = [], None
+    for q, n in specs:
+        dense = synth.make_blocks(q, n, k, seed=n)
+        thin, at = zero_weights(q, dense, n, k, np.arange(n) % 2 == 0)
+        raw = dense.reshape(n, -1)
+        raw[::97] = thin.reshape(n, -1)[::97]
+        raws.append(raw.reshape(-1))
+    g, up = synth.make_x(k, seed=1, batch=rows) * 20, synth.make_x(k, seed=2, batch=rows)
+    xs = (g / (1 + np.exp(-g)) * up).astype(np.float32)
+    xs[:, at] *= np.float32(2.0 ** -45)
+    ws = [device.DeviceBuffer.from_host(r) for r in raws]
+    total = sum(n for _, n in specs)
+    xd, yd = device.DeviceBuffer.from_host(xs), device.DeviceBuffer(4 * rows * total)
+    s = device.Stream()
+    parts, off = [], 0
+    for (q, n), w, r in zip(specs, ws, raws):
+        parts.append((q, w, n, yd.ptr + 4 * off, r.nbytes))
+        off += n
+    try:
+        device.gemv_group(parts, xd, k, batch=rows, y_stride=total, stream=s)
+        s.synchronize()
+        y = yd.to_host(np.float32).reshape(rows, total)
+        with device.Graph.capture(s) as cap:
+            device.gemv_group(parts, xd, k, batch=rows, y_stride=total, stream=s)
+        try:
+            for _ in range(3):
+                device.gemv("Q4_K", ws[1], xd, yd, 33000, k, batch=7, stream=s, w_bytes=raws[1].nbytes)
+                cap.launch(s)
+                s.synchronize()
+                assert bits_equal(yd.to_host(np.float32).reshape(rows, total), y)
+        finally:
+            cap.destroy()
+    finally:
+        for b in ws + [xd, yd]:
+            b.free()
+        s.destroy()
+    off = 0
+    for (q, n), r in zip(specs, raws):
+        mine = np.ascontiguousarray(y[:, off:off + n])
+        assert bits_equal(mine, run(q, r, xs, n, k)), q
+        some = np.unique(np.r_[0:n:97, n - 40:n])
+        check(q, np.ascontiguousarray(r.reshape(n, -1)[some]).reshape(-1), xs, some.size, k, mine[:, some], q)
+        off += n
