@@ -321,9 +321,10 @@ constexpr int64_t kRowsBeforeGemm = 3;
 // 19.6 / 28.9 / 38.4 and 25). Four rows of a Q1_0 matrix that one row's
 // matrix-core kernel runs in some 3 us stay by rows too (rows 4 / 5: 2048 x 2048
 // 12.2 / 15.3 by rows, 15.3 by the pair GEMM; 4096 x 4096 14.8 / 18.2 and 16.1;
-// but 1024 x 1024 12.8 / 15.7 and 12.3, 896 x 4864 20.1 and 14.8).
+// but 1024 x 1024 12.8 / 15.7 and 12.3, 896 x 4864 20.1 and 14.8, 777 x 2560
+// 15.6 and 13.9).
 int64_t pair_rows_min(int qtype, const uint8_t* w, int64_t n, int64_t k) {
-    return qtype == FRQ_Q1_0 && k >= 2048 && k <= 4096 && n * k <= (1 << 24) && frq::gemv_q10_mx_ok(w, k) ? 5 : 4;
+    return qtype == FRQ_Q1_0 && k >= 2048 && frq::gemv_q10_mx_default(w, n, k) ? 5 : 4;
 }
 
 // Where gemm_f32 is the faster one of the two: its two launches against the

@@ -683,7 +683,10 @@ __global__ void __launch_bounds__(512) gemm_pair_kernel(
     // level in fp32, every 256 elements, or one sum in fp64 for Q5_K and Q1_0, whose
     // rows one GEMV each would give: 97 rows of Q5_K 14336 x 4096, error against 64
     // bits 1.12e-7 and 0.89e-7 (one GEMV per row 1.05e-7), 58 and 61 us.
-    constexpr bool kF64 = QT == kTypeQ5K || QT == kTypeQ10, kTwo = !kF64 && MT * NT <= 2;
+    // The 32-row tile of Q4_K, which may run through many units, as well: 16 rows of
+    // 8192 x 18944 1.31e-7 and 1.11e-7, 53.1 and 54.5 us.
+    constexpr bool kF64 = QT == kTypeQ5K || QT == kTypeQ10 || (QT == kTypeQ4K && MT * NT == 1);
+    constexpr bool kTwo = !kF64 && MT * NT <= 2;
     typedef typename std::conditional<kF64, double, float>::type Sum;
     Sum acc[MT][NT][16];
     f32x16 tot[kTwo ? MT : 1][NT], t[2];
@@ -1642,7 +1645,7 @@ void pair_run(const PairPlan& p, const uint8_t* w, const float* x, float* y, int
         pair_go<QT, 1, 8, 1, 1, 2>(p, w, x, y, ldy, s, scratch);
     else if (p.bm == 64)
         pair_go<QT, 1, 8, 2, 1, QT == kTypeQ10 ? 2 : 1>(p, w, x, y, ldy, s, scratch);
-    else if constexpr (QT == kTypeQ4K || QT == kTypeQ6K)
+    else if constexpr (QT == kTypeQ4K)
         pair_go<QT, 2, 4, 2, 2, 1>(p, w, x, y, ldy, s, scratch);
 }
 
@@ -1651,16 +1654,16 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // A call's estimated time (us): its launches + rounds of 256 workgroups (one per
 // CU), each a start and a workgroup's units of k, + the planes of a split k,
 // written and read (8 bytes of each output and split, in 3.1 MB). With few CUs
-// busy a unit takes up to 15 % less. The numbers fit 8900 measured calls: every tile of
-// each format at 1 to 64 splits, eleven matrices of 0.5 to 80 M weights, 2 to 512
-// rows, W cold in the caches. The plans chosen take 0.4 % more than the fastest
-// measured ones on average; one unit time for all formats, and few_kernel wherever
-// within 6 us of the tile, took 2.1 %. Some (us, both sides measured): 64- / 128-row
-// tile, Q6_K 18944 x 3584 at 200 rows 141 / 138, 3584 x 18944 at 333 172 / 174,
-// 14336 x 4096 at 128 61 / 68, Q4_K 18944 x 3584 at 200 119 / 113, at 333 149 / 140,
-// 4096 x 4096 at 333 54 / 56; few_kernel / 32-row tile, Q4_K 4096 x 14336 at 16
-// rows 25 / 32, 24 rows 29 / 32, Q5_K 1024 x 1024 at 12 13 / 15, Q1_0 8192 x 1024
-// at 8 12 / 15, 1024 x 4096 at 32 19 / 17.
+// busy a unit takes up to 15 % less. The numbers fit 90000 measured calls: every
+// tile of each format at 1 to 64 splits for 9900 random shapes of 3 to 512 rows (k
+// 512 to 24576, n 400 to 65536, W cold in the caches). The plans chosen take 0.7 %
+// (up to 32 rows) and 0.3 % more than the fastest measured ones on average; one
+// unit time for all formats, and few_kernel wherever within 6 us of the tile, took
+// 2.5 and 0.6 %. Some (us, both sides measured): 64- / 128-row tile, Q4_K 18944 x
+// 3584 at 200 rows 119 / 113, at 333 149 / 140, 4096 x 4096 at 333 54 / 56;
+// few_kernel / 32-row tile, Q4_K 4096 x 14336 at 16 rows 25 / 32, 24 rows 29 / 32,
+// Q5_K 1024 x 1024 at 12 13 / 15, Q1_0 8192 x 1024 at 8 12 / 15, 1024 x 4096 at 32
+// 19 / 17.
 struct PairCost {
     double launches, start, unit, plane;
     double us(int64_t workgroups, int64_t units, int64_t splits, double plane_us) const {
@@ -1673,13 +1676,13 @@ struct PairCost {
 PairCost pair_cost(int qtype, int bm) {
     const int f = qtype == kTypeQ4K ? 0 : qtype == kTypeQ5K ? 1 : qtype == kTypeQ10 ? 2 : 3;
     static constexpr double unit[5][4] = {
-        {2.1, 2.9, 1.7, 0.0}, {2.8, 3.6, 2.4, 0.0}, {3.2, 4.1, 3.0, 5.1}, {4.2, 5.3, 4.3, 5.3}, {8.2, 0.0, 0.0, 10.6}};
+        {2.35, 3.2, 1.4, 0.0}, {3.05, 3.5, 2.2, 0.0}, {3.7, 4.4, 2.75, 5.6}, {4.6, 5.6, 4.3, 5.7}, {8.4, 0.0, 0.0, 0.0}};
     switch (bm) {
-        case 16: return {5.3, 6.2, unit[0][f], 1.8};
-        case 17: return {9.2, 3.8, unit[1][f], 1.1};
-        case 32: return {8.7, 4.0, unit[2][f], 0.8};
-        case 64: return {12.8, 0.8, unit[3][f], 0.7};
-        default: return {12.8, 0.8, unit[4][f], 0.7};
+        case 16: return {5.5, 5.6, unit[0][f], 1.15};
+        case 17: return {8.6, 3.8, unit[1][f], 1.1};
+        case 32: return {8.5, 4.0, unit[2][f], 0.8};
+        case 64: return {12.0, 0.6, unit[3][f], 0.9};
+        default: return {12.0, 2.6, unit[4][f], 0.7};
     }
 }
 
@@ -1702,9 +1705,14 @@ bool plan_gemm_pair(int qtype, int64_t m, int64_t n, int64_t k, size_t cap, Pair
     const int64_t ntiles = (n + p->bn - 1) / p->bn;
     // The row tile and the split of k with the least estimated time.
     const double plane_us = (double)m * (double)n * 8.0 / 3.1e6;
-    // Q5_K and Q1_0, whose rows otherwise run one GEMV each, keep to the tiles
-    // with fp64 sums, which match a GEMV's error.
-    const bool wide = qtype == kTypeQ4K || qtype == kTypeQ6K;
+    // Only Q4_K has a 128-row tile. It adds all of a split's sums in one fp32 level:
+    // Q5_K and Q1_0, whose rows otherwise run one GEMV each, keep to the tiles with
+    // fp64 sums, which match a GEMV's error. For Q6_K it decoded W half as often but
+    // is bound by the scaling of its 16-element sums (us, error against 64 bits, 64- /
+    // 128-row tile: 18944 x 3584 at 200 rows 141 / 138; 62765 x 1024 at 383 191 and
+    // 0.98e-7 / 177 and 1.34e-7; 65000 x 1536 at 120 93 and 1.12e-7 / 90 and 2.06e-7;
+    // 14336 x 4096 at 128 61 / 68).
+    const bool wide = qtype == kTypeQ4K;
     const int bms[2] = {m <= 32 ? 32 : 64, m <= 32 ? 32 : m <= 64 || !wide ? 64 : 128};
     double best = 0.0;
     bool found = false;

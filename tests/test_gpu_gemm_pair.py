@@ -72,7 +72,7 @@ def test_edges(frq, q, n, k, rows):
     # the 128-row tile, one row or column past its end, k unsplit and split
     ("Q4_K", 33000, 1024, 65, ("pair", 128, 1)), ("Q4_K", 20001, 768, 300, ("pair", 128, 1)),
     ("Q4_K", 18945, 1280, 257, ("pair", 128, 1)), ("Q4_K", 18945, 3584, 200, ("pair", 128, 3)),
-    ("Q6_K", 30000, 1280, 129, ("pair", 128, 1)), ("Q6_K", 62765, 1024, 383, ("pair", 128, 1)),
+    ("Q4_K", 33001, 1792, 66, ("pair", 128, 1)), ("Q6_K", 62765, 1024, 383, ("pair", 64, 1)),
     # rows of x in two and three registers' worth of pieces, and too long for them
     ("Q6_K", 3001, 8192, 33, ("pair", 64, 16)), ("Q6_K", 1500, 20480, 40, ("pair", 64, 40)),
     ("Q5_K", 100, 24832, 33, ("pair", 64, 49)), ("Q5_K", 100, 20736, 70, ("pair", 64, 41)),
@@ -144,7 +144,7 @@ def zero_weights(q, raw, n, k, keep):
     ("Q5_K", 70, 4096, 9, ("pair", 32, 16)), ("Q6_K", 66000, 512, 11, ("pair", 32, 1)),
     ("Q4_K", 70, 2048, 66, ("pair", 64, 8)), ("Q6_K", 1500, 16384, 40, ("pair", 64, 32)),
     ("Q1_0", 65600, 512, 40, ("pair", 64, 1)), ("Q4_K", 33000, 1024, 66, ("pair", 128, 1)),
-    ("Q6_K", 33000, 1024, 66, ("pair", 128, 1)),
+    ("Q6_K", 33000, 1024, 66, ("pair", 64, 2)),
 ])
 def test_small_x_beside_large_on_zero_weights(frq, q, n, k, rows, plan):
     """x of a row 2^-15 to 2^-80 below its largest decide outputs whose other
@@ -265,7 +265,7 @@ def test_small_x_in_groups_and_graphs(frq):
     group and in replays of a graph, and the bound holds."""
     k, rows = 1024, 40
     specs = [("Q5_K", 300), ("Q4_K", 33000), ("Q5_K", 65600)]
-    assert [device.batch_plan(q, n, k, rows)[:3] for q, n in specs] == [("pair", 64, 4), ("pair", 64, 1), ("pair", 64, 2)]
+    assert [device.batch_plan(q, n, k, rows)[:3] for q, n in specs] == [("pair", 64, 4), ("pair", 64, 1), ("pair", 64, 1)]
     raws, at = [], None
     for q, n in specs:
         dense = synth.make_blocks(q, n, k, seed=n)
