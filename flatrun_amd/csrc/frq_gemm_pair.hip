@@ -18,9 +18,10 @@
 //     codes, scale and centre included.
 //   * the matrix cores sum 64 elements (Q6_K 16, one sub-block) in fp32, then
 //     acc += scale * sum in fp32 (the scale of a Q4_K / Q5_K block alone, since
-//     sc is in the code). With up to 64 rows a wave, Q5_K and Q1_0 keep acc in
-//     fp64, and the others add it to the result's accumulator every 256
-//     elements, so that the sums round less often at full size. Q4_K / Q5_K add -(dmin m - d R) sum(x) per 32-element sub-block
+//     sc is in the code). With up to 64 rows a wave, Q5_K, Q1_0 and 32 rows of
+//     Q4_K keep acc in fp64, and the others add it to the result's accumulator
+//     every 256 elements, so that the sums round less often at full size.
+//     Q4_K / Q5_K add -(dmin m - d R) sum(x) per 32-element sub-block
 //     on the matrix cores as well: three bf16 pieces of each factor, the six
 //     products down to 2^-24 of their product.
 //   With R the nearest integer, |d (sc q - R)| + |dmin m - d R| <= 3 |w|, so a
@@ -49,7 +50,7 @@
 // elements: eight times the vector work); 97 rows of Q5_K 14336 x 4096 1390 (a GEMV
 // per row) / 58; 16 rows of Q4_K 4096 x 14336 36 / 32 (few_kernel 25). 128-row
 // tiles are bound by the matrix cores' issue and power, few rows by the chain of
-// decode and products per wave (3.2 us per 256 of k) and the three launches. The
+// decode and products per wave (3.7 us per 256 of k) and the three launches. The
 // range of lo costs a vector instruction per two codes, or per sum with 128 rows:
 // 127 -> 132 us, 97 rows of Q5_K (with fp64 sums) 55 -> 58.
 // MFMA operand layouts (32x32x16, 8 values per lane): A lane l holds row l%32,
